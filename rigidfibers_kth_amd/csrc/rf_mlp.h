@@ -20,36 +20,35 @@ struct MlpLayout {
 };
 MlpLayout mlp_layout();
 
-// Activation and gradient buffers for a batch of up to `rows` rows.
+// Activation and gradient buffers for a batch of up to `rows` rows (the base
+// is 256-byte aligned; rows are padded to whole 16-byte vectors).
 struct MlpBuffers {
     int rows = 0;
-    float* Z = nullptr;        // [rows][kMlpIn] standardised input
+    float* Z = nullptr;        // [rows][128] standardised input, zero-padded
     float* H[3] = {nullptr};   // [rows][kMlpHidden]
-    float* Yhat = nullptr;     // [rows][kMlpOut]
-    float* D[4] = {nullptr};   // deltas: D[0..2] [rows][kMlpHidden], D[3] [rows][kMlpOut]
-    float* partial = nullptr;  // per-block partial losses
+    float* D[4] = {nullptr};   // deltas: D[0..2] [rows][kMlpHidden], D[3] [rows][16], zero-padded
+    float* partial = nullptr;  // per-workgroup partial losses
+    float* gpart = nullptr;    // [splits][parameters] partial gradients
 };
 int64_t mlp_buffer_floats(int rows);
 void mlp_buffer_bind(float* base, int rows, MlpBuffers* b);
-int64_t mlp_loss_blocks(int B);
 
 // X[i][kMlpIn] from the first 16 entries of each neighbour list (ldn >= 16).
 hipError_t mlp_features(int N, int ldn, const double* pos, const double* orient, const int* nbr,
                         const double* nbr_dist, float* X, hipStream_t s);
 // Y[i][3M]: coefficients of fiber i in its local frame.
 hipError_t mlp_targets(int N, int M, const double* orient, const double* x, float* Y, hipStream_t s);
-hipError_t mlp_forward(const float* w, int B, const float* X, MlpBuffers& buf, hipStream_t s);
-// buf.D[3] = d loss / d Yhat for the mean squared error on standardised
-// targets; buf.partial[blocks] = partial sums of squared errors.
-hipError_t mlp_loss(const float* w, int B, const float* Y, MlpBuffers& buf, hipStream_t s);
-hipError_t mlp_backward(const float* w, int B, MlpBuffers& buf, float* g, hipStream_t s);
+// Yhat [B][kMlpOut]: the network's standardised output.
+hipError_t mlp_forward(const float* w, int B, const float* X, float* Yhat, hipStream_t s);
+// Gradient of the mean squared error on standardised targets into g (blob
+// offsets, standardisation entries untouched); acc[0] += the sum of squared
+// errors.  With idx, batch row q is row idx[q] of X and Y.
+hipError_t mlp_gradient(const float* w, int B, const float* X, const float* Y, const int64_t* idx, MlpBuffers& buf,
+                        float* g, double* acc, hipStream_t s);
 // x (global, fiber-major 3M) from the de-standardised local prediction.
 hipError_t mlp_to_global(int N, int M, const double* orient, const float* w, const float* Yhat, double* x,
                          hipStream_t s);
 hipError_t mlp_adam(int n, float* w, const float* g, float* m, float* v, float lr, int step, hipStream_t s);
-hipError_t mlp_gather(int B, int W, const float* src, const int64_t* idx, float* dst, hipStream_t s);
-// acc[0] += the partial losses of the last mlp_loss.
-hipError_t mlp_accumulate_loss(int B, const MlpBuffers& buf, double* acc, hipStream_t s);
 
 // Host-side: Glorot-uniform weights (SplitMix64), standardisation from data.
 void mlp_init_weights(uint64_t seed, float* w);

@@ -117,110 +117,308 @@ __global__ void to_global_kernel(int N, int M, const double* __restrict__ orient
     }
 }
 
-// ---- dense layers ----------------------------------------------------------
-// C[m][n] (+)= sum_k A(m,k) B(k,n), A(m,k) = A[m*sam + k*sak], B(k,n) =
-// B[k*sbk + n*sbn]; 64x64 tiles per workgroup, K staged 16 at a time in LDS.
-// epi: 0 plain store, 1 add bias b[n] then tanh, 2 add bias, 3 accumulate.
-constexpr int kT = 64, kK = 16;
+// ---- the network -----------------------------------------------------------
+// One workgroup carries 16 rows of the batch through every layer: forward,
+// and for a gradient the loss and all deltas back to the first hidden layer,
+// the activations in LDS.  Every product is v_mfma_f32_16x16x4f32 (FP32
+// operands and accumulation): lane l supplies A[l%16][l/16] and B[l/16][l%16]
+// and holds D[4(l/16) + r][l%16].  The K index of a product is permuted, the
+// same way in both operands: step r of a group of 16 takes k = 4(l/16) + r, so
+// one 16-byte read of LDS feeds four steps.  The weights (200 KB) stream from
+// L2; a layer's loads are issued before its products.
+// What bounds it: seven dependent layers of L2 and LDS latency.  16 rows per
+// workgroup (the rows of one matrix instruction) give 256 workgroups at 4096
+// rows: 35 us for forward, loss and deltas, where one tiled product per layer
+// and pass took 640 us.
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));  // weight rows are only 4-byte aligned
+typedef float f2v __attribute__((ext_vector_type(2)));
 
-__global__ void __launch_bounds__(256) gemm_kernel(int Mr, int Nc, int Kd, const float* __restrict__ A, int64_t sam,
-                                                   int64_t sak, const float* __restrict__ B, int64_t sbk, int64_t sbn,
-                                                   float* __restrict__ C, int64_t ldc, const float* __restrict__ bias,
-                                                   int epi)
+constexpr int kRowTile = 16;   // rows per workgroup
+constexpr int kActStride = 132;  // LDS row stride: 16-byte aligned, rows four banks apart
+constexpr int kZStride = 128;  // standardised input, zero-padded
+constexpr int kDStride = 16;   // output deltas, zero-padded
+
+struct RowsArgs {
+    const float* w;
+    int W[4], b[4], in_mean, in_std, out_mean, out_std;
+    int B;
+    const float* X;
+    const float* Y;
+    const int64_t* idx;  // row of X and Y taken as batch row q (nullptr: q itself)
+    float* Yhat;
+    float* Z;            // gradient only, as everything below
+    float* H[3];
+    float* D[4];
+    float* partial;
+};
+
+__device__ __forceinline__ f4v mfma_f32(float a, float b, f4v c)
 {
-    __shared__ float As[kK][kT + 1];
-    __shared__ float Bs[kK][kT + 1];
-    const int m0 = blockIdx.y * kT, n0 = blockIdx.x * kT;
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < Kd; k0 += kK) {
-        for (int e = threadIdx.x; e < kK * kT; e += 256) {
-            const int kk = e / kT, mm = e % kT;
-            const int m = m0 + mm, k = k0 + kk;
-            As[kk][mm] = (m < Mr && k < Kd) ? A[(int64_t)m * sam + (int64_t)k * sak] : 0.f;
-            const int n = n0 + mm;
-            Bs[kk][mm] = (n < Nc && k < Kd) ? B[(int64_t)k * sbk + (int64_t)n * sbn] : 0.f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < kK; ++kk) {
-            float a[4], b[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                a[u] = As[kk][ty * 4 + u];
-                b[u] = Bs[kk][tx * 4 + u];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) acc[u][v] += a[u] * b[v];
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int m = m0 + ty * 4 + u, n = n0 + tx * 4 + v;
-            if (m >= Mr || n >= Nc) continue;
-            float val = acc[u][v];
-            float* c = C + (int64_t)m * ldc + n;
-            if (epi == 1) val = tanhf(val + bias[n]);
-            else if (epi == 2) val = val + bias[n];
-            else if (epi == 3) val = *c + val;
-            *c = val;
-        }
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// (x - mean)/std per feature
-__global__ void normalize_kernel(int B, int I, const float* __restrict__ X, const float* __restrict__ mean,
-                                 const float* __restrict__ sd, float* __restrict__ Z)
+// acc = act[16 rows][0, K) W^T for the output columns n0..n0+15 (n < O), W row-major [O][K].
+template <int K, int O>
+__device__ __forceinline__ f4v layer_tile(const float (&act)[kRowTile][kActStride], const float* __restrict__ W, int n0,
+                                          int lr, int lk)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)B * I) return;
-    const int f = (int)(t % I);
-    Z[t] = (X[t] - mean[f]) / sd[f];
+    constexpr int G = (K + 15) / 16;
+    const int n = n0 + lr;
+    f4v wv[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const int k = 16 * g + 4 * lk;
+        if (n < O && k + 3 < K) {
+            wv[g] = *reinterpret_cast<const f4u*>(W + n * K + k);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) wv[g][r] = (n < O && k + r < K) ? W[n * K + k + r] : 0.f;
+        }
+    }
+    f4v acc = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const f4v a = *reinterpret_cast<const f4v*>(&act[lr][16 * g + 4 * lk]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc = mfma_f32(a[r], wv[g][r], acc);
+    }
+    return acc;
 }
 
-// MSE loss on normalised targets: d = 2 (yhat - (y - mean)/sd) / (B*O);
-// per-block partial losses.
-__global__ void mse_kernel(int B, int O, const float* __restrict__ yhat, const float* __restrict__ Y,
-                           const float* __restrict__ mean, const float* __restrict__ sd, float* __restrict__ d,
-                           float* __restrict__ partial)
+// acc = delta[16 rows][0, O) W for the input columns n0..n0+15, W row-major [O][128].
+template <int O>
+__device__ __forceinline__ f4v back_tile(const float (&delta)[kRowTile][kActStride], const float* __restrict__ W, int n0,
+                                         int lr, int lk)
 {
-    __shared__ float sh[256];
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    float l = 0.f;
-    if (t < (int64_t)B * O) {
-        const int o = (int)(t % O);
-        const float diff = yhat[t] - (Y[t] - mean[o]) / sd[o];
-        d[t] = 2.f * diff / (float)((int64_t)B * O);
-        l = diff * diff;
+    constexpr int G = (O + 15) / 16;
+    f4v wv[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int o = 16 * g + 4 * lk + r;
+            wv[g][r] = (o < O) ? W[o * kMlpHidden + n0 + lr] : 0.f;
+        }
+    f4v acc = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const f4v a = *reinterpret_cast<const f4v*>(&delta[lr][16 * g + 4 * lk]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc = mfma_f32(a[r], wv[g][r], acc);
     }
-    sh[threadIdx.x] = l;
+    return acc;
+}
+
+template <bool GRAD>
+__global__ void __launch_bounds__(256) mlp_rows_kernel(const RowsArgs a)
+{
+    __shared__ __attribute__((aligned(16))) float act[2][kRowTile][kActStride];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = t >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
+    const int row0 = blockIdx.x * kRowTile;
+    for (int e = t; e < kRowTile * kZStride; e += 256) {  // standardised input
+        const int r = e / kZStride, c = e % kZStride;
+        const int row = row0 + r;
+        float z = 0.f;
+        if (row < a.B && c < kMlpIn) {
+            const int64_t src = a.idx ? a.idx[row] : row;
+            z = (a.X[src * kMlpIn + c] - a.w[a.in_mean + c]) / a.w[a.in_std + c];
+        }
+        act[0][r][c] = z;
+        if (GRAD && row < a.B) a.Z[(int64_t)row * kZStride + c] = z;
+    }
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
+    float h[3][2][4];  // this lane's activations (rows 4 lk + r, columns 32 wave + 16 u + lr)
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int n0 = 32 * wave + 16 * u;
+            const f4v acc = (l == 0) ? layer_tile<kMlpIn, kMlpHidden>(act[0], a.w + a.W[0], n0, lr, lk)
+                                     : layer_tile<kMlpHidden, kMlpHidden>(act[l & 1], a.w + a.W[l], n0, lr, lk);
+            const float bias = a.w[a.b[l] + n0 + lr];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float v = tanhf(acc[r] + bias);
+                h[l][u][r] = v;
+                act[(l + 1) & 1][4 * lk + r][n0 + lr] = v;
+                const int row = row0 + 4 * lk + r;
+                if (GRAD && row < a.B) a.H[l][(int64_t)row * kMlpHidden + n0 + lr] = v;
+            }
+        }
         __syncthreads();
     }
-    if (threadIdx.x == 0) partial[blockIdx.x] = sh[0];
+    // output layer (one tile): the third activation is in act[1]
+    if (wave == 0) {
+        const f4v acc = layer_tile<kMlpHidden, kMlpOut>(act[1], a.w + a.W[3], 0, lr, lk);
+        const float bias = (lr < kMlpOut) ? a.w[a.b[3] + lr] : 0.f;
+        float loss = 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = row0 + 4 * lk + r;
+            const float y = acc[r] + bias;
+            const bool live = row < a.B && lr < kMlpOut;
+            if (live && a.Yhat) a.Yhat[(int64_t)row * kMlpOut + lr] = y;
+            if constexpr (GRAD) {
+                // mean squared error on standardised targets
+                float d = 0.f, sq = 0.f;
+                if (live) {
+                    const int64_t src = a.idx ? a.idx[row] : row;
+                    const float diff = y - (a.Y[src * kMlpOut + lr] - a.w[a.out_mean + lr]) / a.w[a.out_std + lr];
+                    d = 2.f * diff / (float)((int64_t)a.B * kMlpOut);
+                    sq = diff * diff;
+                }
+                act[0][4 * lk + r][lr] = d;
+                loss += sq;
+                if (row < a.B) a.D[3][(int64_t)row * kDStride + lr] = d;
+            }
+        }
+        if constexpr (GRAD) {
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off, 64);
+            if (lane == 0) a.partial[blockIdx.x] = loss;
+        }
+    }
+    if constexpr (!GRAD) return;
+    __syncthreads();
+    // deltas of the hidden layers: (delta W) (1 - h^2)
+#pragma unroll
+    for (int l = 2; l >= 0; --l) {
+        const int in = l & 1;  // delta 3 in act[0], 2 in act[1], 1 in act[0]
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int n0 = 32 * wave + 16 * u;
+            const f4v acc = (l == 2) ? back_tile<kMlpOut>(act[in], a.w + a.W[3], n0, lr, lk)
+                                     : back_tile<kMlpHidden>(act[in], a.w + a.W[l + 1], n0, lr, lk);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float hv = h[l][u][r];
+                const float d = acc[r] * (1.f - hv * hv);
+                act[in ^ 1][4 * lk + r][n0 + lr] = d;
+                const int row = row0 + 4 * lk + r;
+                if (row < a.B) a.D[l][(int64_t)row * kMlpHidden + n0 + lr] = d;
+            }
+        }
+        __syncthreads();
+    }
 }
 
-// delta *= (1 - h^2)  (tanh derivative from the stored activation)
-__global__ void tanh_back_kernel(int64_t n, const float* __restrict__ h, float* __restrict__ delta)
+// dW_l[o][i] = sum_b delta_l[b][o] in_l[b][i] and db_l[o] = sum_b delta_l[b][o]
+// for all four layers in one launch: workgroup = (layer, 64 rows o, 32 columns
+// i) x one split of the batch, each wavefront a quarter of the split, the four
+// sums met in LDS.  A lane's 16-byte read of a delta row covers o = o0 + 4 lr
+// .. + 3 and feeds four 16 x 16 blocks, its 8-byte read of an input row two.
+// The split partials (blob order, from first_param) are added in a fixed order
+// by grad_reduce_kernel.  Bound by L2 reads of the deltas and activations; at
+// 4096 rows 13 us + 5 us for the sum, against 2.9 ms for four products over
+// the whole batch by four workgroups each and 2.9 ms for serial bias sums.
+constexpr int kGradTasks = 28;  // 8 + 8 + 8 (128 x 128 in 64 x 32) + 4 (15 x 128)
+constexpr int kMaxGradSplits = 32;
+
+struct GradArgs {
+    int B, splits;
+    const float* Z;
+    const float* H[3];
+    const float* D[4];
+    int W[4], b[4];  // offsets from first_param
+    float* out;      // [splits][stride]
+    int64_t stride;
+};
+
+__global__ void __launch_bounds__(256) mlp_grad_kernel(const GradArgs a)
 {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) delta[t] *= (1.f - h[t] * h[t]);
+    __shared__ float red[4][64 * 32];
+    __shared__ float redb[4][64];
+    const int task = blockIdx.x;
+    const int l = (task < 24) ? task / 8 : 3, tl = (l < 3) ? task % 8 : task - 24;
+    const int o0 = (l < 3) ? 64 * (tl / 4) : 0, i0 = 32 * (tl % 4);
+    const int O = (l < 3) ? kMlpHidden : kMlpOut, I = (l == 0) ? kMlpIn : kMlpHidden;
+    const int ldd = (l < 3) ? kMlpHidden : kDStride;
+    const float* delta = a.D[l];
+    const float* in = (l == 0) ? a.Z : a.H[l - 1];  // row stride 128 either way
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
+    const int per = ((a.B + a.splits - 1) / a.splits + 15) / 16 * 16;  // rows per split
+    const int b0 = blockIdx.y * per + wave * (per / 4);
+    const int b1 = min(a.B, b0 + per / 4);
+    const bool dl = l < 3 || lr < 4;  // 4 lr < kDStride
+    f4v acc[4][2];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) acc[m][u] = f4v{0.f, 0.f, 0.f, 0.f};
+    f4v bs = f4v{0.f, 0.f, 0.f, 0.f};
+    for (int b = b0; b < b1; b += 16) {  // per / 4 is a multiple of 4: guard each row
+        f4v dv[4];
+        f2v iv[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int row = b + 4 * q + lk;
+            const bool live = row < b1;
+            dv[q] = (live && dl) ? *reinterpret_cast<const f4v*>(delta + (int64_t)row * ldd + o0 + 4 * lr)
+                                 : f4v{0.f, 0.f, 0.f, 0.f};
+            iv[q] = live ? *reinterpret_cast<const f2v*>(in + (int64_t)row * 128 + i0 + 2 * lr) : f2v{0.f, 0.f};
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            bs += dv[q];
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) acc[m][u] = mfma_f32(dv[q][m], iv[q][u], acc[m][u]);
+        }
+    }
+    // block (m, u), value r of this lane: o = o0 + 4 (4 lk + r) + m, i = i0 + 2 lr + u
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) red[wave][(4 * (4 * lk + r) + m) * 32 + 2 * lr + u] = acc[m][u][r];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        float v = bs[m];
+        v += __shfl_xor(v, 16, 64);
+        v += __shfl_xor(v, 32, 64);
+        if (lk == 0) redb[wave][4 * lr + m] = v;
+    }
+    __syncthreads();
+    float* out = a.out + blockIdx.y * a.stride;
+    for (int e = t; e < 64 * 32; e += 256) {
+        const int o = o0 + e / 32, i = i0 + e % 32;
+        if (o < O && i < I) out[a.W[l] + (int64_t)o * I + i] = (red[0][e] + red[1][e]) + (red[2][e] + red[3][e]);
+    }
+    if (i0 == 0 && t < 64 && o0 + t < O)
+        out[a.b[l] + o0 + t] = (redb[0][t] + redb[1][t]) + (redb[2][t] + redb[3][t]);
 }
 
-// db[o] = sum_b delta[b][o]
-__global__ void bias_grad_kernel(int B, int O, const float* __restrict__ delta, float* __restrict__ db)
+// g[p] = sum of the split partials (no splits: g is complete), and in the last
+// workgroup acc[0] += the batch's partial losses.
+__global__ void __launch_bounds__(256) grad_reduce_kernel(int n, int splits, int64_t stride,
+                                                          const float* __restrict__ part, float* __restrict__ g,
+                                                          int losses, const float* __restrict__ partial,
+                                                          double* __restrict__ acc)
 {
-    const int o = blockIdx.x * blockDim.x + threadIdx.x;
-    if (o >= O) return;
+    if (blockIdx.x == gridDim.x - 1) {
+        __shared__ double sh[256];
+        double s = 0.0;
+        for (int i = threadIdx.x; i < losses; i += 256) s += partial[i];
+        sh[threadIdx.x] = s;
+        __syncthreads();
+        for (int st = 128; st > 0; st >>= 1) {
+            if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) acc[0] += sh[0];
+        return;
+    }
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= n) return;
     float s = 0.f;
-    for (int b = 0; b < B; ++b) s += delta[(int64_t)b * O + o];
-    db[o] = s;
+    for (int k = 0; k < splits; ++k) s += part[k * stride + p];
+    g[p] = s;
 }
 
 __global__ void adam_kernel(int n, float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
@@ -236,39 +434,7 @@ __global__ void adam_kernel(int n, float* __restrict__ w, const float* __restric
     w[t] -= lr * (mt / c1) / (sqrtf(vt / c2) + eps);
 }
 
-__global__ void gather_rows_kernel(int B, int W, const float* __restrict__ src, const int64_t* __restrict__ idx,
-                                   float* __restrict__ dst)
-{
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)B * W) return;
-    const int64_t b = t / W, c = t % W;
-    dst[t] = src[idx[b] * W + c];
-}
-
-// acc[0] += sum of partial[0..n)  (one block)
-__global__ void accumulate_kernel(int64_t n, const float* __restrict__ partial, double* __restrict__ acc)
-{
-    __shared__ double sh[256];
-    double t = 0.0;
-    for (int64_t i = threadIdx.x; i < n; i += 256) t += partial[i];
-    sh[threadIdx.x] = t;
-    __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-        if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) acc[0] += sh[0];
-}
-
 inline dim3 grid1(int64_t n, int bs = 256) { return dim3((unsigned)((n + bs - 1) / bs)); }
-
-hipError_t gemm(int Mr, int Nc, int Kd, const float* A, int64_t sam, int64_t sak, const float* B, int64_t sbk,
-                int64_t sbn, float* C, int64_t ldc, const float* bias, int epi, hipStream_t s)
-{
-    dim3 grid((Nc + kT - 1) / kT, (Mr + kT - 1) / kT);
-    hipLaunchKernelGGL(gemm_kernel, grid, dim3(256), 0, s, Mr, Nc, Kd, A, sam, sak, B, sbk, sbn, C, ldc, bias, epi);
-    return hipGetLastError();
-}
 
 }  // namespace
 
@@ -310,67 +476,79 @@ hipError_t mlp_targets(int N, int M, const double* orient, const double* x, floa
     return hipGetLastError();
 }
 
-// Forward pass of B rows of X; activations H[0..3] ([B][128] each) and the
-// normalised output Yhat [B][15] are kept for the backward pass.
-hipError_t mlp_forward(const float* w, int B, const float* X, MlpBuffers& buf, hipStream_t s)
+namespace {
+
+inline int64_t pad64(int64_t x) { return (x + 63) / 64 * 64; }
+inline int loss_blocks(int rows) { return (rows + kRowTile - 1) / kRowTile; }
+
+// Splits of the batch in mlp_grad_kernel: about 256 rows each, so that 28
+// tasks x splits fill the chip from a batch of 2048 on; a training batch of
+// 256 takes one split and writes the gradient directly.
+inline int grad_splits(int rows) { return std::max(1, std::min(kMaxGradSplits, (rows + 255) / 256)); }
+
+RowsArgs rows_args(const float* w, int B, const float* X, float* Yhat)
 {
     const MlpLayout L = mlp_layout();
-    hipLaunchKernelGGL(normalize_kernel, grid1((int64_t)B * kMlpIn), dim3(256), 0, s, B, kMlpIn, X, w + L.in_mean,
-                       w + L.in_std, buf.Z);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const int dims[5] = {kMlpIn, kMlpHidden, kMlpHidden, kMlpHidden, kMlpOut};
-    const float* in = buf.Z;
+    RowsArgs a{};
+    a.w = w;
     for (int l = 0; l < 4; ++l) {
-        float* out = (l < 3) ? buf.H[l] : buf.Yhat;
-        e = gemm(B, dims[l + 1], dims[l], in, dims[l], 1, w + L.W[l], 1, dims[l], out, dims[l + 1], w + L.b[l],
-                 (l < 3) ? 1 : 2, s);
-        if (e != hipSuccess) return e;
-        in = out;
+        a.W[l] = (int)L.W[l];
+        a.b[l] = (int)L.b[l];
     }
-    return hipSuccess;
+    a.in_mean = (int)L.in_mean;
+    a.in_std = (int)L.in_std;
+    a.out_mean = (int)L.out_mean;
+    a.out_std = (int)L.out_std;
+    a.B = B;
+    a.X = X;
+    a.Yhat = Yhat;
+    return a;
 }
 
-// Backward pass given dYhat in buf.D[3] ([B][15]); gradients into g (same
-// offsets as the weight blob; normalisation entries untouched).
-hipError_t mlp_backward(const float* w, int B, MlpBuffers& buf, float* g, hipStream_t s)
-{
-    const MlpLayout L = mlp_layout();
-    const int dims[5] = {kMlpIn, kMlpHidden, kMlpHidden, kMlpHidden, kMlpOut};
-    hipError_t e;
-    for (int l = 3; l >= 0; --l) {
-        const float* delta = buf.D[l];  // [B][dims[l+1]]
-        const float* in = (l == 0) ? buf.Z : buf.H[l - 1];
-        // dW[o][i] = sum_b delta[b][o] in[b][i]
-        e = gemm(dims[l + 1], dims[l], B, delta, 1, dims[l + 1], in, dims[l], 1, g + L.W[l], dims[l], nullptr, 0, s);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(bias_grad_kernel, grid1(dims[l + 1], 128), dim3(128), 0, s, B, dims[l + 1], delta,
-                           g + L.b[l]);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-        if (l > 0) {
-            // delta_prev[b][i] = sum_o delta[b][o] W[o][i], then * tanh'
-            float* dprev = buf.D[l - 1];
-            e = gemm(B, dims[l], dims[l + 1], delta, dims[l + 1], 1, w + L.W[l], dims[l], 1, dprev, dims[l], nullptr,
-                     0, s);
-            if (e != hipSuccess) return e;
-            hipLaunchKernelGGL(tanh_back_kernel, grid1((int64_t)B * dims[l]), dim3(256), 0, s, (int64_t)B * dims[l],
-                               buf.H[l - 1], dprev);
-            if ((e = hipGetLastError()) != hipSuccess) return e;
-        }
-    }
-    return hipSuccess;
-}
+}  // namespace
 
-hipError_t mlp_loss(const float* w, int B, const float* Y, MlpBuffers& buf, hipStream_t s)
+// Normalised output Yhat [B][15] of B rows of X.
+hipError_t mlp_forward(const float* w, int B, const float* X, float* Yhat, hipStream_t s)
 {
-    const MlpLayout L = mlp_layout();
-    const int64_t tot = (int64_t)B * kMlpOut;
-    hipLaunchKernelGGL(mse_kernel, grid1(tot), dim3(256), 0, s, B, kMlpOut, buf.Yhat, Y, w + L.out_mean, w + L.out_std,
-                       buf.D[3], buf.partial);
+    const RowsArgs a = rows_args(w, B, X, Yhat);
+    hipLaunchKernelGGL(mlp_rows_kernel<false>, dim3(loss_blocks(B)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
-int64_t mlp_loss_blocks(int B) { return ((int64_t)B * kMlpOut + 255) / 256; }
+// Gradient of the mean squared error of B rows of (X, Y) (rows idx[0..B) of
+// them when idx is given) into g (same offsets as the weight blob;
+// normalisation entries untouched); acc[0] += the sum of squared errors.
+hipError_t mlp_gradient(const float* w, int B, const float* X, const float* Y, const int64_t* idx, MlpBuffers& buf,
+                        float* g, double* acc, hipStream_t s)
+{
+    const MlpLayout L = mlp_layout();
+    RowsArgs a = rows_args(w, B, X, nullptr);
+    a.Y = Y;
+    a.idx = idx;
+    a.Z = buf.Z;
+    a.partial = buf.partial;
+    GradArgs ga{};
+    ga.B = B;
+    ga.splits = grad_splits(B);
+    ga.Z = buf.Z;
+    for (int l = 0; l < 3; ++l) ga.H[l] = a.H[l] = buf.H[l];
+    for (int l = 0; l < 4; ++l) {
+        ga.D[l] = a.D[l] = buf.D[l];
+        ga.W[l] = (int)(L.W[l] - L.first_param);
+        ga.b[l] = (int)(L.b[l] - L.first_param);
+    }
+    ga.out = (ga.splits > 1) ? buf.gpart : g + L.first_param;
+    ga.stride = pad64(L.num_params);
+    hipLaunchKernelGGL(mlp_rows_kernel<true>, dim3(loss_blocks(B)), dim3(256), 0, s, a);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(mlp_grad_kernel, dim3(kGradTasks, ga.splits), dim3(256), 0, s, ga);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    const int n = (ga.splits > 1) ? (int)L.num_params : 0;
+    hipLaunchKernelGGL(grad_reduce_kernel, dim3((n + 255) / 256 + 1), dim3(256), 0, s, n, ga.splits, ga.stride,
+                       buf.gpart, g + L.first_param, loss_blocks(B), buf.partial, acc);
+    return hipGetLastError();
+}
 
 hipError_t mlp_to_global(int N, int M, const double* orient, const float* w, const float* Yhat, double* x,
                          hipStream_t s)
@@ -389,21 +567,12 @@ hipError_t mlp_adam(int n, float* w, const float* g, float* m, float* v, float l
     return hipGetLastError();
 }
 
-hipError_t mlp_gather(int B, int W, const float* src, const int64_t* idx, float* dst, hipStream_t s)
-{
-    hipLaunchKernelGGL(gather_rows_kernel, grid1((int64_t)B * W), dim3(256), 0, s, B, W, src, idx, dst);
-    return hipGetLastError();
-}
-
-
-namespace {
-inline int64_t pad64(int64_t x) { return (x + 63) / 64 * 64; }
-}  // namespace
-
 int64_t mlp_buffer_floats(int rows)
 {
     const int64_t r = rows;
-    return pad64(r * kMlpIn) + 6 * pad64(r * kMlpHidden) + 2 * pad64(r * kMlpOut) + pad64(mlp_loss_blocks(rows));
+    const int splits = grad_splits(rows);
+    return pad64(r * kZStride) + 6 * pad64(r * kMlpHidden) + pad64(r * kDStride) + pad64(loss_blocks(rows)) +
+           (splits > 1 ? splits * pad64(mlp_layout().num_params) : 0);
 }
 
 void mlp_buffer_bind(float* base, int rows, MlpBuffers* b)
@@ -412,26 +581,20 @@ void mlp_buffer_bind(float* base, int rows, MlpBuffers* b)
     float* q = base;
     b->rows = rows;
     b->Z = q;
-    q += pad64(r * kMlpIn);
+    q += pad64(r * kZStride);
     for (int l = 0; l < 3; ++l) {
         b->H[l] = q;
         q += pad64(r * kMlpHidden);
     }
-    b->Yhat = q;
-    q += pad64(r * kMlpOut);
     for (int l = 0; l < 3; ++l) {
         b->D[l] = q;
         q += pad64(r * kMlpHidden);
     }
     b->D[3] = q;
-    q += pad64(r * kMlpOut);
+    q += pad64(r * kDStride);
     b->partial = q;
-}
-
-hipError_t mlp_accumulate_loss(int B, const MlpBuffers& buf, double* acc, hipStream_t s)
-{
-    hipLaunchKernelGGL(accumulate_kernel, dim3(1), dim3(256), 0, s, mlp_loss_blocks(B), buf.partial, acc);
-    return hipGetLastError();
+    q += pad64(loss_blocks(rows));
+    b->gpart = q;
 }
 
 // Glorot-uniform weights from SplitMix64 ((u >> 11) * 2^-53), zero biases.
@@ -487,7 +650,8 @@ hipError_t mlp_train(float* w, const float* dX, const float* dY, int64_t count, 
     const int64_t nb = count / batch;
     float* work = nullptr;
     const int64_t nbuf = mlp_buffer_floats(batch);
-    const int64_t need = 3 * L.total + nbuf + (int64_t)batch * (kMlpIn + kMlpOut);
+    const int64_t lt = pad64(L.total);
+    const int64_t need = 3 * lt + nbuf;
     hipError_t e = hipMalloc(&work, sizeof(float) * need);
     if (e != hipSuccess) return e;
     int64_t* didx = nullptr;
@@ -504,13 +668,11 @@ hipError_t mlp_train(float* w, const float* dX, const float* dY, int64_t count, 
         return z ^ (z >> 31);
     };
     float* g = work;
-    float* m = g + L.total;
-    float* v = m + L.total;
+    float* m = g + lt;
+    float* v = m + lt;
     MlpBuffers buf;
-    mlp_buffer_bind(v + L.total, batch, &buf);
-    float* bX = v + L.total + nbuf;
-    float* bY = bX + (int64_t)batch * kMlpIn;
-    if (e == hipSuccess) e = hipMemsetAsync(work, 0, sizeof(float) * 3 * L.total, s);
+    mlp_buffer_bind(v + lt, batch, &buf);
+    if (e == hipSuccess) e = hipMemsetAsync(work, 0, sizeof(float) * 3 * lt, s);
     int step = 0;
     for (int ep = 0; ep < epochs && e == hipSuccess; ++ep) {
         for (int64_t i = count - 1; i > 0; --i) std::swap(idx[i], idx[(int64_t)(next() % (uint64_t)(i + 1))]);
@@ -519,12 +681,7 @@ hipError_t mlp_train(float* w, const float* dX, const float* dY, int64_t count, 
         const float lr_e = lr * 0.5f * (1.f + std::cos(3.14159265358979f * (float)ep / (float)epochs));
         for (int64_t b = 0; b < nb && e == hipSuccess; ++b) {
             const int64_t* ib = didx + b * batch;
-            if ((e = mlp_gather(batch, kMlpIn, dX, ib, bX, s)) != hipSuccess) break;
-            if ((e = mlp_gather(batch, kMlpOut, dY, ib, bY, s)) != hipSuccess) break;
-            if ((e = mlp_forward(w, batch, bX, buf, s)) != hipSuccess) break;
-            if ((e = mlp_loss(w, batch, bY, buf, s)) != hipSuccess) break;
-            if ((e = mlp_accumulate_loss(batch, buf, dacc, s)) != hipSuccess) break;
-            if ((e = mlp_backward(w, batch, buf, g, s)) != hipSuccess) break;
+            if ((e = mlp_gradient(w, batch, dX, dY, ib, buf, g, dacc, s)) != hipSuccess) break;
             e = mlp_adam((int)L.num_params, w + L.first_param, g + L.first_param, m + L.first_param,
                          v + L.first_param, lr_e, ++step, s);
         }

@@ -685,7 +685,7 @@ int rf_sim::mlp_alloc()
     }
     if (d_mlp_w) return RF_OK;
     const MlpLayout L = mlp_layout();
-    const int64_t floats = L.total + (int64_t)N * (kMlpIn + kMlpOut) + mlp_buffer_floats(N);
+    const int64_t floats = L.total + (int64_t)N * (kMlpIn + 2 * kMlpOut);
     void* q = nullptr;
     if (hipMalloc(&q, sizeof(float) * floats) != hipSuccess) {
         rf::set_error("learned guess: cannot allocate network buffers");
@@ -695,8 +695,7 @@ int rf_sim::mlp_alloc()
     d_mlp_w = static_cast<float*>(q);
     d_mlp_X = d_mlp_w + L.total;
     d_mlp_Y = d_mlp_X + (int64_t)N * kMlpIn;
-    d_mlp_work = d_mlp_Y + (int64_t)N * kMlpOut;
-    mlp_buffer_bind(d_mlp_work, N, &mlp_buf);
+    d_mlp_Yhat = d_mlp_Y + (int64_t)N * kMlpOut;
     return RF_OK;
 }
 
@@ -711,8 +710,8 @@ int rf_sim::mlp_infer(double* x_out)
     }
     if ((rc = setup_neighbours())) return rc;
     HIP_TRY(mlp_features(N, knn, d_pos[lvl_three], d_orient[lvl_three], d_nbr, d_nbr_dist, d_mlp_X, stream));
-    HIP_TRY(mlp_forward(d_mlp_w, N, d_mlp_X, mlp_buf, stream));
-    HIP_TRY(mlp_to_global(N, M, d_orient[lvl_three], d_mlp_w, mlp_buf.Yhat, x_out, stream));
+    HIP_TRY(mlp_forward(d_mlp_w, N, d_mlp_X, d_mlp_Yhat, stream));
+    HIP_TRY(mlp_to_global(N, M, d_orient[lvl_three], d_mlp_w, d_mlp_Yhat, x_out, stream));
     return RF_OK;
 }
 
@@ -1745,28 +1744,26 @@ extern "C" int rf_mlp_forward_backward(rf_sim* s, const float* X, const float* Y
         return RF_EINVAL;
     }
     const MlpLayout L = mlp_layout();
-    const int64_t used = L.total + (int64_t)B * (kMlpIn + kMlpOut) + mlp_buffer_floats(B);
-    const int64_t floats = used + 4;  // + one 8-byte aligned double after `used`
+    // gradient blob, pairs, network buffers (each from a 256-byte boundary) and the loss sum
+    auto pad = [](int64_t v) { return (v + 63) / 64 * 64; };
+    const int64_t oX = pad(L.total), oY = oX + pad((int64_t)B * kMlpIn), oW = oY + pad((int64_t)B * kMlpOut);
+    const int64_t oA = oW + pad(mlp_buffer_floats(B));
     float* q = nullptr;
-    if (hipMalloc(&q, sizeof(float) * floats) != hipSuccess) {
+    if (hipMalloc(&q, sizeof(float) * (oA + 2)) != hipSuccess) {
         set_error("rf_mlp_forward_backward: cannot allocate");
         return RF_ENOMEM;
     }
     float* g = q;
-    float* dX = g + L.total;
-    float* dY = dX + (int64_t)B * kMlpIn;
-    float* work = dY + (int64_t)B * kMlpOut;
-    double* acc = reinterpret_cast<double*>(q + (used + 1) / 2 * 2);
+    float* dX = q + oX;
+    float* dY = q + oY;
+    double* acc = reinterpret_cast<double*>(q + oA);
     MlpBuffers buf;
-    mlp_buffer_bind(work, B, &buf);
+    mlp_buffer_bind(q + oW, B, &buf);
     hipError_t e = hipMemcpyAsync(dX, X, sizeof(float) * (size_t)B * kMlpIn, hipMemcpyHostToDevice, s->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(dY, Y, sizeof(float) * (size_t)B * kMlpOut, hipMemcpyHostToDevice, s->stream);
     if (e == hipSuccess) e = hipMemsetAsync(g, 0, sizeof(float) * L.total, s->stream);
     if (e == hipSuccess) e = hipMemsetAsync(acc, 0, sizeof(double), s->stream);
-    if (e == hipSuccess) e = mlp_forward(s->d_mlp_w, B, dX, buf, s->stream);
-    if (e == hipSuccess) e = mlp_loss(s->d_mlp_w, B, dY, buf, s->stream);
-    if (e == hipSuccess) e = mlp_accumulate_loss(B, buf, acc, s->stream);
-    if (e == hipSuccess) e = mlp_backward(s->d_mlp_w, B, buf, g, s->stream);
+    if (e == hipSuccess) e = mlp_gradient(s->d_mlp_w, B, dX, dY, nullptr, buf, g, acc, s->stream);
     double a = 0.0;
     if (e == hipSuccess) e = hipMemcpyAsync(grad, g, sizeof(float) * L.total, hipMemcpyDeviceToHost, s->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(&a, acc, sizeof(double), hipMemcpyDeviceToHost, s->stream);

@@ -100,8 +100,7 @@ struct rf_sim {
     float* d_mlp_w = nullptr;    // weight blob
     float* d_mlp_X = nullptr;    // [N][113] features
     float* d_mlp_Y = nullptr;    // [N][15] local-frame targets
-    float* d_mlp_work = nullptr; // activations for N rows
-    rf::MlpBuffers mlp_buf;
+    float* d_mlp_Yhat = nullptr; // [N][15] network output
     bool mlp_weights = false;    // a trained network is loaded
     bool r0_ready = false;       // d_r holds b - A x for the next GMRES start
     // LU workspace (allocated on first use)
