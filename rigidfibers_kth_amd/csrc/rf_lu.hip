@@ -971,6 +971,209 @@ __global__ void __launch_bounds__(256) lu_gemm_mfma_kernel(T* A, int64_t lda, Ge
         }
 }
 
+constexpr int kXcds = 8, kCusPerXcd = 32;
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+
+// 16 bytes per lane from src straight into LDS at dst (wavefront-uniform; lane
+// l's bytes land at dst + 16 l).  Kept out of the kernel templates: the host
+// pass cannot form the LDS address-space pointer.
+template <typename T>
+__device__ __forceinline__ void ring_load(const T* src, T* dst)
+{
+    __builtin_amdgcn_global_load_lds(src, (lds_ptr_t)dst, 16, 0, 0);
+}
+
+// Barrier without the memory fence of __syncthreads(): the stage data
+// arrives by the loads' own counter (waited for explicitly before it), and
+// the clobber keeps the compiler from moving LDS reads across it.
+__device__ __forceinline__ void stage_barrier() { asm volatile("s_barrier" ::: "memory"); }
+
+// s_waitcnt immediate for "at most v vector-memory operations in flight":
+// vmcnt in bits 3:0 and 15:14, expcnt in 6:4 (7: no wait), lgkmcnt in 11:8
+// (15: no wait).
+constexpr int vm_wait(int v) { return (v & 15) | ((v >> 4) << 14) | 0x0F70; }
+
+// Tile (tx, ty) of a TR x TC grid for this workgroup.  Workgroup ids go
+// round-robin over the 8 XCDs; each XCD takes an equal, contiguous share of
+// the tiles ordered by strips of `strip` tile rows and down each strip's columns,
+// so the tiles it runs together are a compact block and share a few L and U
+// panels in its L2.  (Whole square blocks dealt out in turn left XCDs up to 10 %
+// apart at n = 15000 and far more on small trailing matrices.)  False: no tile,
+// before any barrier.
+__device__ __forceinline__ bool xcd_tile(int TR, int TC, int strip, int& tx, int& ty)
+{
+    const int share = (TR * TC + kXcds - 1) / kXcds;
+    const int local = (int)blockIdx.x / kXcds;
+    const int idx = ((int)blockIdx.x % kXcds) * share + local;
+    if (local >= share || idx >= TR * TC) return false;
+    const int s = idx / (strip * TC), rem = idx - s * strip * TC;
+    const int h = min(strip, TR - s * strip);  // tile rows of this strip
+    ty = rem / h;
+    tx = s * strip + (rem - ty * h);
+    return true;
+}
+inline int xcd_grid(int TR, int TC) { return (TR * TC + kXcds - 1) / kXcds * kXcds; }
+
+// ---- FP64 trailing update with 128 x 128 tiles -----------------------------
+// C -= L21 U12 for whole super-panels: 4 wavefronts of 64 x 64 (16 blocks of
+// v_mfma_f64_16x16x4f64, the C tile in the accumulators from the start), K 16
+// at a time straight from the matrix into a two-stage LDS ring
+// (global_load_lds_dwordx4, no staging registers).  The FP64 matrix
+// instruction takes 64 cycles for 2048 flops, so LDS never bounds it: what
+// did was the traffic of 64 x 64 tiles (8 flops per byte read, in row-major
+// tile order): 49.9 ms for the super-panel updates of n = 15000.  128 x 128
+// tiles read 16, and the workgroups an XCD runs together (32 CUs x 2) take a
+// block of 8 x 8 tiles, so its L2 serves each L21 and U12 panel eight times.  Two
+// workgroups per CU: one loads or stores its C tile while the other
+// multiplies.  35.9 ms (59 TFLOP/s; the largest update keeps the matrix cores
+// 87 % busy at the clock the chip holds there); 38.6 ms with whole blocks dealt
+// to the XCDs, 40 ms with sign flips of L21 in the loop; three or four ring
+// stages of half the chunk, and more workgroup priorities, changed nothing.
+// LDS: A[k] rows of 128 doubles (one wavefront load, 1 KB) at a pitch of 1152
+// bytes, which puts the four k of a fragment read on both bank halves; B as
+// columns of 16 k (128 bytes, 8 columns a load), the pair of k's p of column c
+// at p ^ (c & 7), so 16 columns' reads spread over all banks.
+constexpr int kDT = 128, kDK = 16, kDPitch = 144;   // tile, K chunk, doubles between A rows
+constexpr int kDStage = kDK * kDPitch + kDT * kDK;  // doubles per ring stage
+constexpr int kDStrip = 8;                          // tile rows of an XCD's strip
+
+__global__ void __launch_bounds__(256, 2) lu_gemm_f64w_kernel(double* A, int64_t lda, GemmRange g)
+{
+    __shared__ __attribute__((aligned(1024))) double ring[2][kDStage];
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wr = (wave >> 1) * 64, wc = (wave & 1) * 64;
+    const int lr = lane & 15, lk = lane >> 4;
+    int tx, ty;
+    if (!xcd_tile((g.r1 - g.r0 + kDT - 1) / kDT, (g.c1 - g.c0 + kDT - 1) / kDT, kDStrip, tx, ty)) return;
+    const int rbase = g.r0 + tx * kDT, cbase = g.c0 + ty * kDT;
+    // Sources as a uniform base and a 32-bit lane offset; rows and columns past
+    // the range are clamped to its last pair / column (their products land only
+    // where nothing is stored).
+    const char* abase = reinterpret_cast<const char*>(A + (int64_t)(g.ka + wave * 4) * lda);
+    const char* bbase = reinterpret_cast<const char*>(A + (int64_t)cbase * lda + g.ka);
+    const unsigned aoff = 8u * (unsigned)min(rbase + 2 * lane, ((g.r1 + 1) & ~1) - 2);
+    unsigned boff[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int c = wave * 32 + q * 8 + (lane >> 3);
+        boff[q] = 8u * ((unsigned)min(c, g.c1 - 1 - cbase) * (unsigned)lda) + 16u * ((lane & 7) ^ (c & 7));
+    }
+    auto issue = [&](int st) {  // the next chunk
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            ring_load(reinterpret_cast<const double*>(abase + (int64_t)q * lda * 8 + aoff),
+                      &ring[st][(wave * 4 + q) * kDPitch]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            ring_load(reinterpret_cast<const double*>(bbase + boff[q]),
+                      &ring[st][kDK * kDPitch + (wave * 32 + q * 8) * kDK]);
+        abase += (int64_t)kDK * lda * 8;
+        bbase += kDK * 8;
+    };
+    issue(0);
+    // The accumulators hold -C: the FP64 matrix instruction shares the vector
+    // ALU, so the loop carries no sign flips of L21 (32 per chunk cost 10 %).
+    d4 acc[4][4];
+    const bool interior = rbase + kDT <= g.r1 && cbase + kDT <= g.c1;
+    double* cp = A + (int64_t)(cbase + wc + lk) * lda + rbase + wr + lr;  // element (0, 0, 0) of this lane
+    if (interior) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const double* cj = cp + (int64_t)(16 * j + 4 * r) * lda;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[i][j][r] = -cj[16 * i];
+            }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const bool in = rbase + wr + 16 * i + lr < g.r1 && cbase + wc + 16 * j + lk + 4 * r < g.c1;
+                    acc[i][j][r] = in ? -cp[(int64_t)(16 * j + 4 * r) * lda + 16 * i] : 0.0;
+                }
+    }
+    int bcol[4][4];  // this lane's B positions of a stage, by K step and column block
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int c = wc + 16 * j + lr, k = 4 * ks + lk;
+            bcol[ks][j] = kDK * kDPitch + c * kDK + 2 * ((k >> 1) ^ (c & 7)) + (k & 1);
+        }
+    auto multiply = [&](const double* stage) {
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            double a[4], b[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a[i] = stage[(4 * ks + lk) * kDPitch + wr + 16 * i + lr];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[j] = stage[bcol[ks][j]];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) mfma_16x16x4(b[j], a[i], acc[i][j]);
+        }
+    };
+    // this wavefront's loads of a chunk have landed and its LDS reads are
+    // done; after the barrier that holds for every wavefront's
+    auto turn = [&] {
+        __builtin_amdgcn_s_waitcnt(vm_wait(0) & ~0x0F00);
+        stage_barrier();
+    };
+    for (int kc = g.ka; kc < g.kb; kc += 2 * kDK) {  // an even number of chunks
+        turn();
+        issue(1);
+        multiply(&ring[0][0]);
+        turn();
+        if (kc + 2 * kDK < g.kb) issue(0);
+        multiply(&ring[1][0]);
+    }
+    if (interior) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                double* cj = cp + (int64_t)(16 * j + 4 * r) * lda;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) cj[16 * i] = -acc[i][j][r];
+            }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (rbase + wr + 16 * i + lr < g.r1 && cbase + wc + 16 * j + lk + 4 * r < g.c1)
+                    cp[(int64_t)(16 * j + 4 * r) * lda + 16 * i] = -acc[i][j][r];
+}
+
+// Below about 192 of these tiles the 64 x 64 kernel fills the chip better: a
+// tile takes 55 us alone on a CU, the smaller one 41 us with three to a CU.
+constexpr int kDMinTiles = 192;
+
+// Whether the kernel above takes the range: pairs of K chunks, 16-byte
+// aligned rows and K offsets (the last row pair may reach one row past an odd
+// r1: the columns are lda rows apart).
+inline bool f64w_fits(const GemmRange& g, int64_t lda)
+{
+    return (g.kb - g.ka) % (2 * kDK) == 0 && g.ka % 2 == 0 && g.r0 % 2 == 0 && lda % 2 == 0 && g.r1 - g.r0 >= 2 * kDT &&
+           g.c1 - g.c0 >= 2 * kDT && (int64_t)(g.r1 - g.r0) * (g.c1 - g.c0) >= (int64_t)kDMinTiles * kDT * kDT;
+}
+
+inline void launch_f64w(double* A, int64_t lda, const GemmRange& g, hipStream_t s)
+{
+    hipLaunchKernelGGL(lu_gemm_f64w_kernel,
+                       dim3(xcd_grid((g.r1 - g.r0 + kDT - 1) / kDT, (g.c1 - g.c0 + kDT - 1) / kDT)), dim3(256), 0, s, A,
+                       lda, g);
+}
+
 // fp16 matrix-core update of FP32 factors (preconditioner factors only):
 // C[:, j] = (C[:, j] s_j + (-L21) (U12[:, j] s_j)) / s_j with the operands
 // rounded to fp16 and FP32 accumulation (v_mfma_f32_16x16x32_f16).  |L21| <= 1
@@ -1308,30 +1511,9 @@ __global__ void __launch_bounds__(256, 3) lu_gemm_f16p_kernel(float* A, int64_t 
 // 256 x 128 tiles two workgroups share a CU and one's C traffic overlaps the
 // other's products: 12.1 ms, and 240 ms against 270 ms over a factorisation.
 constexpr int kWB = 256;  // tile rows
-constexpr int kXcds = 8, kCusPerXcd = 32;
 // below this trailing size the 128 x 128 tiles fill the chip better
 constexpr int kWideMin = 4096;
 __device__ __forceinline__ int wide_seg(int r, int s) { return (s ^ ((r >> 1) ^ (r >> 3))) & 3; }
-
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
-// 16 bytes per lane from src straight into LDS at dst (wavefront-uniform; lane
-// l's bytes land at dst + 16 l).  Kept out of the kernel templates: the host
-// pass cannot form the LDS address-space pointer.
-__device__ __forceinline__ void ring_load(const _Float16* src, _Float16* dst)
-{
-    __builtin_amdgcn_global_load_lds(src, (lds_ptr_t)dst, 16, 0, 0);
-}
-
-// Barrier without the memory fence of __syncthreads(): the stage data
-// arrives by the loads' own counter (waited for explicitly before it), and
-// the clobber keeps the compiler from moving LDS reads across it.
-__device__ __forceinline__ void stage_barrier() { asm volatile("s_barrier" ::: "memory"); }
-
-// s_waitcnt immediate for "at most v vector-memory operations in flight":
-// vmcnt in bits 3:0 and 15:14, expcnt in 6:4 (7: no wait), lgkmcnt in 11:8
-// (15: no wait).
-constexpr int vm_wait(int v) { return (v & 15) | ((v >> 4) << 14) | 0x0F70; }
 
 // Configuration: TN tile columns (each wavefront 128 x TN/2), STAGES ring
 // stages, WG workgroups per CU.  The one used, 256 x 128 with 3 stages (72 KB
@@ -1562,6 +1744,12 @@ hipError_t factor_impl(T* A, int64_t lda, int n, int nb, int* ipiv, int* info, i
                                        dim3(256), 0, s, A, lda, g, colscale);
             }
         } else if (use_mfma) {
+            if constexpr (sizeof(T) == 8) {
+                if (f64w_fits(g, lda)) {
+                    launch_f64w(A, lda, g, s);
+                    return;
+                }
+            }
             const int bn = gemm_bn<T>();
             // FP64 takes 64-row tiles everywhere (three workgroups per CU
             // instead of two: 85.7 against 91 ms for n = 15000); FP32 the
