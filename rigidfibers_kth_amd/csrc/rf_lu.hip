@@ -1891,15 +1891,21 @@ __global__ void mfma_probe_kernel(int mode, double* out64, float* out32)
     }
 }
 
-// ---- solves with the factors: permutation + one launch per block -----------
-// A solve with preconditioner factors runs once per GMRES iteration, so it
-// is built for few launches and no serial chains: once per
-// factorisation the pivots become one permutation and the 64x64 diagonal
-// blocks of L and U are inverted (one workgroup per block); each 64-row
-// block of the forward and backward sweeps is then one launch, in which
-// every workgroup forms y = inv(D) v_block (4 lanes per row) and updates 64
-// of the remaining rows (each wavefront takes 16 of the block's columns with
-// all 16 loads in flight; the 4 partial sums meet in LDS).
+// ---- solves with the factors ------------------------------------------------
+// Once per factorisation the pivots become one permutation and the 64 x 64
+// diagonal blocks of L and U are inverted (one workgroup per block).
+//   FP64 factors (one solve each): each 64-row block of the forward and
+// backward sweeps is one launch, in which every workgroup forms
+// y = inv(D) v_block (4 lanes per row) and updates 64 of the remaining rows
+// (each wavefront takes 16 of the block's columns with all 16 loads in
+// flight; the 4 partial sums meet in LDS).
+//   FP32 factors precondition: a solve runs once per GMRES iteration, and at
+// 4 to 7 us a launch the 938 launches of n = 30000 took 5.1 ms for 3.6 GB of
+// factors.  The inverses are therefore merged to 512 x 512 diagonal blocks, and
+// a block is two launches, y = inv(D) v_block over 16 workgroups (4.1 us) and
+// the rows beyond it in 128-row workgroups that stream its 512 columns (10.8 us
+// on average, 2.8 TB/s): 1.75 ms a solve, bound by the launch latency and
+// ramp of the updates.
 constexpr int kSB = 64;
 
 __global__ void permute_kernel(const double* __restrict__ x, const int* __restrict__ perm, int n,
@@ -1909,9 +1915,17 @@ __global__ void permute_kernel(const double* __restrict__ x, const int* __restri
     if (i < n) y[i] = x[perm[i]];
 }
 
-// inv[(2 b + u) 64^2 + 64 r + q] = (D_b^-1)[r][q], D_b the diagonal block b of
-// L (u = 0, unit lower) or U (u = 1).  Thread c computes column c of the
+// Element (r, q) of the inverse of diagonal block b of L (u = 0, unit lower) or
+// U (u = 1): FP64 inv[(2 b + u) 64^2 + 64 r + q]; FP32 the 64 x 64 diagonal
+// blocks of the merged ones (wide_inverse).  Thread c computes column c of the
 // inverse by substitution and touches only that column: no barriers.
+constexpr int kWI = 512;  // merged diagonal blocks
+__host__ __device__ inline float* wide_inverse(float* inv, int n, int upper, int block)
+{
+    const int blocks = (n + kWI - 1) / kWI;
+    return inv + ((size_t)upper * blocks + block) * kWI * kWI;  // column-major
+}
+
 template <typename T>
 __global__ void __launch_bounds__(kSB) block_inverse_kernel(const T* __restrict__ LU, int64_t lda, int n,
                                                             T* __restrict__ inv)
@@ -1947,8 +1961,185 @@ __global__ void __launch_bounds__(kSB) block_inverse_kernel(const T* __restrict_
         }
     }
     __syncthreads();
-    T* out = inv + ((size_t)b * 2 + upper) * kSB * kSB;
-    for (int r = 0; r < kSB; ++r) out[r * kSB + c] = X[r][c];
+    if constexpr (sizeof(T) == 4) {
+        T* out = wide_inverse(inv, n, upper, k0 / kWI) + (size_t)(k0 % kWI) * kWI + k0 % kWI;
+        for (int q = 0; q < kSB; ++q) out[(size_t)q * kWI + c] = X[c][q];
+    } else {
+        T* out = inv + ((size_t)b * 2 + upper) * kSB * kSB;
+        for (int r = 0; r < kSB; ++r) out[r * kSB + c] = X[r][c];
+    }
+}
+
+// Two inverses of size s, P of the first and Q of the second half, merged to
+// one of size 2 s:
+//   lower  [P 0; R Q], R = -Q (B P), B = L21;   upper  [P R; 0 Q], R = -P (B Q), B = U12.
+// Phase 0 forms the product in brackets into the block opposite to R (the
+// triangle the inverse leaves unused), phase 1 forms R.  64 x 64 tiles, 4
+// wavefronts of 32 x 32 on v_mfma_f32_16x16x4f32, K 16 at a time.  Inverse
+// entries of the other triangle read as zero (64-row granularity: earlier
+// merges left their products there), as do rows and columns past n.
+__global__ void __launch_bounds__(256) merge_inverse_kernel(const float* __restrict__ LU, int64_t lda, int n,
+                                                            float* inv, int s, int phase)
+{
+    __shared__ float As[16][64 + 4];
+    __shared__ float Bs[16][64 + 4];
+    const int upper = blockIdx.z, k0 = blockIdx.y * kWI;
+    const int bs = min(kWI, n - k0);
+    const int side = s / 64, tile = blockIdx.x % (side * side), pair = blockIdx.x / (side * side);
+    const int o = 2 * s * pair;            // first half at o, second at o + s
+    const int m = min(s, bs - o - s);      // size of the second half
+    if (m <= 0) return;
+    const int ti = (tile % side) * 64, tj = (tile / side) * 64;
+    float* W = wide_inverse(inv, n, upper, blockIdx.y);
+    const int rows = upper ? s : m, cols = upper ? m : s;
+    const int depth = (phase == 0) == (upper != 0) ? m : s;
+    // offsets in the block of A's rows / columns, B's rows / columns and the result
+    const int ar = upper ? o : o + s, ac = (phase == 0) == (upper != 0) ? o + s : o;
+    const int br = upper ? o + s : o, bc = (phase == 0) == (upper != 0) ? o + s : (phase == 0 ? o : (upper ? o : o + s));
+    const int cr = (phase == 0) ? (upper ? o + s : o) : ar, cc = (phase == 0) ? (upper ? o : o + s) : (upper ? o + s : o);
+    auto inv_at = [&](int r, int c) {
+        const bool in = upper ? r / 64 <= c / 64 : r / 64 >= c / 64;
+        return in ? W[(size_t)c * kWI + r] : 0.f;
+    };
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
+    const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32;
+    f4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = f4{0, 0, 0, 0};
+    for (int kc = 0; kc < depth; kc += 16) {
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int e = t + 256 * u;
+            {
+                const int i = e % 64, k = kc + e / 64;
+                const bool in = ti + i < rows && k < depth;
+                float v = 0.f;
+                if (in) v = (phase == 0) ? LU[(int64_t)(k0 + ac + k) * lda + k0 + ar + ti + i] : inv_at(ar + ti + i, ac + k);
+                As[e / 64][i] = v;
+            }
+            {
+                const int k = kc + e % 16, j = e / 16;
+                const bool in = tj + j < cols && k < depth;
+                float v = 0.f;
+                if (in) v = (phase == 0) ? inv_at(br + k, bc + tj + j) : W[(size_t)(bc + tj + j) * kWI + br + k];
+                Bs[e % 16][j] = v;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < 16; ks += 4) {
+            float a[2], b[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) a[i] = As[ks + lk][wr + 16 * i + lr];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) b[j] = Bs[ks + lk][wc + 16 * j + lr];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) mfma_16x16x4(a[i], b[j], acc[i][j]);
+        }
+    }
+    const float sign = (phase == 0) ? 1.f : -1.f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = ti + wr + 16 * i + 4 * lk + r, col = tj + wc + 16 * j + lr;
+                if (row < rows && col < cols) W[(size_t)(cc + col) * kWI + cr + row] = sign * acc[i][j][r];
+            }
+}
+
+// y = inv(D) v_block for a merged block: 32 rows per workgroup, a lane 4 rows
+// (16-byte loads) of every 32nd column of the block's triangle, all its loads
+// in flight; FP64 sums over the 8 lanes and 4 wavefronts of a row.
+template <int LOWER>
+__global__ void __launch_bounds__(256) wide_diag_kernel(int n, float* __restrict__ inv, const double* __restrict__ v,
+                                                        double* __restrict__ out, int block)
+{
+    __shared__ double vb[kWI];
+    __shared__ double part[4][32];
+    const int k0 = block * kWI, bs = min(kWI, n - k0);
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int r0 = blockIdx.x * 32, row = r0 + 4 * (lane & 7), cg = (lane >> 3) + 8 * wave;
+    const float* W = wide_inverse(inv, n, LOWER ? 0 : 1, block) + row;
+    const int lo = LOWER ? 0 : r0 / 64 * 64, hi = LOWER ? min(bs, r0 / 64 * 64 + 64) : bs;
+    f4 w[kWI / 32];
+#pragma unroll
+    for (int u = 0; u < kWI / 32; ++u) {
+        const int c = lo + cg + 32 * u;
+        w[u] = (c < hi) ? *reinterpret_cast<const f4*>(W + (size_t)c * kWI) : f4{0, 0, 0, 0};
+    }
+    for (int e = t; e < bs; e += 256) vb[e] = v[k0 + e];
+    __syncthreads();
+    double y[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int u = 0; u < kWI / 32; ++u) {
+        const int c = lo + cg + 32 * u;
+        const double x = (c < hi) ? vb[c] : 0.0;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y[r] += (double)w[u][r] * x;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+        for (int off = 8; off < 64; off <<= 1) y[r] += __shfl_xor(y[r], off, 64);
+        if (lane < 8) part[wave][4 * lane + r] = y[r];
+    }
+    __syncthreads();
+    if (t < 32 && r0 + t < bs) out[k0 + r0 + t] = (part[0][t] + part[1][t]) + (part[2][t] + part[3][t]);
+}
+
+// v -= LU[rows, block columns] y for the rows beyond the block (LOWER) or
+// before it: 128 rows per workgroup, 8 wavefronts of 64 columns, 8 bytes (2
+// rows) a lane and column with 16 loads in flight; FP64 sums.
+template <int LOWER>
+__global__ void __launch_bounds__(512) wide_update_kernel(const float* __restrict__ LU, int64_t lda, int n,
+                                                          const double* __restrict__ y, double* __restrict__ v,
+                                                          int block)
+{
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    constexpr int kCols = kWI / 8;
+    __shared__ double yb[kWI];
+    __shared__ double part[8][128];
+    const int k0 = block * kWI, bs = min(kWI, n - k0);
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int row = (LOWER ? k0 + bs : 0) + blockIdx.x * 128 + 2 * lane;
+    const int rend = LOWER ? n : k0;
+    const int c0 = wave * kCols;
+    yb[t] = (t < bs) ? y[k0 + t] : 0.0;
+    __syncthreads();
+    double s0 = 0.0, s1 = 0.0;
+    if (row < rend) {  // an odd last row reads its pair from the padding (lda is a multiple of 4)
+        const float* a = LU + (int64_t)(k0 + c0) * lda + row;
+#pragma unroll
+        for (int q = 0; q < kCols; q += 16) {
+            f2 w[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+                w[u] = (c0 + q + u < bs) ? *reinterpret_cast<const f2*>(a + (int64_t)(q + u) * lda) : f2{0.f, 0.f};
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                s0 += (double)w[u][0] * yb[c0 + q + u];
+                s1 += (double)w[u][1] * yb[c0 + q + u];
+            }
+        }
+    }
+    part[wave][2 * lane] = s0;
+    part[wave][2 * lane + 1] = s1;
+    __syncthreads();
+    const int i = (LOWER ? k0 + bs : 0) + blockIdx.x * 128 + t;
+    if (t < 128 && i < rend) {
+        double s = 0.0;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) s += part[w][t];
+        v[i] -= s;
+    }
 }
 
 // lower = 1: forward block (unit lower L), rows updated i >= k0+bs;
@@ -2027,8 +2218,9 @@ static size_t perm_bytes(int n) { return ((sizeof(int) * (size_t)n + 255) / 256)
 
 size_t lu_solve_aux_bytes(int n, int elem_bytes)
 {
-    const size_t blocks = ((size_t)n + kSB - 1) / kSB;
-    return perm_bytes(n) + blocks * 2 * kSB * kSB * (size_t)elem_bytes;
+    const size_t w = (elem_bytes == 4) ? kWI : kSB;  // diagonal blocks inverted as a whole
+    const size_t blocks = ((size_t)n + w - 1) / w;
+    return perm_bytes(n) + blocks * 2 * w * w * (size_t)elem_bytes;
 }
 
 hipError_t lu_prepare_solve(const void* LU, int elem_bytes, int64_t lda, int n, const int* ipiv, void* aux,
@@ -2053,29 +2245,56 @@ hipError_t lu_prepare_solve(const void* LU, int elem_bytes, int64_t lda, int n, 
     if (elem_bytes == 8)
         hipLaunchKernelGGL(block_inverse_kernel<double>, grid, dim3(kSB), 0, s, static_cast<const double*>(LU), lda,
                            n, static_cast<double*>(inv));
-    else
-        hipLaunchKernelGGL(block_inverse_kernel<float>, grid, dim3(kSB), 0, s, static_cast<const float*>(LU), lda, n,
-                           static_cast<float*>(inv));
+    else {
+        const float* f = static_cast<const float*>(LU);
+        hipLaunchKernelGGL(block_inverse_kernel<float>, grid, dim3(kSB), 0, s, f, lda, n, static_cast<float*>(inv));
+        for (int w = kSB; w < kWI; w *= 2) {
+            const int side = w / 64, pairs = kWI / (2 * w);
+            for (int phase = 0; phase < 2; ++phase)
+                hipLaunchKernelGGL(merge_inverse_kernel, dim3(side * side * pairs, (n + kWI - 1) / kWI, 2), dim3(256), 0,
+                                   s, f, lda, n, static_cast<float*>(inv), w, phase);
+        }
+    }
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t solve_blocks_impl(const T* LU, int64_t lda, int n, const void* aux, double* x, double* tmp, hipStream_t s)
+static hipError_t solve_f64(const double* LU, int64_t lda, int n, const int* perm, const double* inv, double* x,
+                            double* tmp, hipStream_t s)
 {
-    const int* perm = static_cast<const int*>(aux);
-    const T* inv = reinterpret_cast<const T*>(static_cast<const char*>(aux) + perm_bytes(n));
     const int nb = (n + kSB - 1) / kSB;
     hipLaunchKernelGGL(permute_kernel, dim3((n + 255) / 256), dim3(256), 0, s, x, perm, n, tmp);
     for (int b = 0; b < nb; ++b) {  // L z = P x: tmp -> x
         const int k0 = b * kSB, bs = std::min(kSB, n - k0);
         const int rows = n - k0 - bs;
-        hipLaunchKernelGGL((sweep_block_kernel<T, 1>), dim3(std::max(1, (rows + 63) / 64)), dim3(256), 0, s, LU,
+        hipLaunchKernelGGL((sweep_block_kernel<double, 1>), dim3(std::max(1, (rows + 63) / 64)), dim3(256), 0, s, LU,
                            lda, n, inv, tmp, x, k0, bs);
     }
     for (int b = nb - 1; b >= 0; --b) {  // U y = z: x -> tmp
         const int k0 = b * kSB, bs = std::min(kSB, n - k0);
-        hipLaunchKernelGGL((sweep_block_kernel<T, 0>), dim3(std::max(1, (k0 + 63) / 64)), dim3(256), 0, s, LU,
+        hipLaunchKernelGGL((sweep_block_kernel<double, 0>), dim3(std::max(1, (k0 + 63) / 64)), dim3(256), 0, s, LU,
                            lda, n, inv, x, tmp, k0, bs);
+    }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return launch_copy_vec(tmp, x, n, s);
+}
+
+static hipError_t solve_f32(const float* LU, int64_t lda, int n, const int* perm, float* inv, double* x, double* tmp,
+                            hipStream_t s)
+{
+    const int nb = (n + kWI - 1) / kWI;
+    hipLaunchKernelGGL(permute_kernel, dim3((n + 255) / 256), dim3(256), 0, s, x, perm, n, tmp);
+    for (int b = 0; b < nb; ++b) {  // L z = P x: tmp -> x
+        const int bs = std::min(kWI, n - b * kWI), rows = n - b * kWI - bs;
+        hipLaunchKernelGGL(wide_diag_kernel<1>, dim3((bs + 31) / 32), dim3(256), 0, s, n, inv, tmp, x, b);
+        if (rows > 0)
+            hipLaunchKernelGGL(wide_update_kernel<1>, dim3((rows + 127) / 128), dim3(512), 0, s, LU, lda, n, x, tmp, b);
+    }
+    for (int b = nb - 1; b >= 0; --b) {  // U y = z: x -> tmp
+        const int bs = std::min(kWI, n - b * kWI), rows = b * kWI;
+        hipLaunchKernelGGL(wide_diag_kernel<0>, dim3((bs + 31) / 32), dim3(256), 0, s, n, inv, x, tmp, b);
+        if (rows > 0)
+            hipLaunchKernelGGL(wide_update_kernel<0>, dim3((rows + 127) / 128), dim3(512), 0, s, LU, lda, n, tmp, x, b);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -2085,9 +2304,11 @@ hipError_t solve_blocks_impl(const T* LU, int64_t lda, int n, const void* aux, d
 hipError_t lu_solve_blocks(const void* LU, int elem_bytes, int64_t lda, int n, const void* aux, double* x,
                            double* tmp, hipStream_t s)
 {
+    const int* perm = static_cast<const int*>(aux);
+    char* inv = const_cast<char*>(static_cast<const char*>(aux)) + perm_bytes(n);
     if (elem_bytes == 8)
-        return solve_blocks_impl<double>(static_cast<const double*>(LU), lda, n, aux, x, tmp, s);
-    return solve_blocks_impl<float>(static_cast<const float*>(LU), lda, n, aux, x, tmp, s);
+        return solve_f64(static_cast<const double*>(LU), lda, n, perm, reinterpret_cast<const double*>(inv), x, tmp, s);
+    return solve_f32(static_cast<const float*>(LU), lda, n, perm, reinterpret_cast<float*>(inv), x, tmp, s);
 }
 
 }  // namespace rf

@@ -5,6 +5,7 @@ import pytest
 import scipy.linalg as sl
 
 import rigidfibers_kth_amd as rf
+from rigidfibers_kth_amd.layouts import layout
 from test_gpu_lu import _dominant_with_block_swaps, _random
 
 pytestmark = pytest.mark.gpu
@@ -33,3 +34,25 @@ def test_fp64_wide_update_on_a_matrix_that_pivots_everywhere():
     np.testing.assert_array_equal(ipiv, piv_ref)
     # growth and conditioning of a random matrix: n eps times the factors' size, with room for both
     assert np.abs(LU - lu_ref).max() <= 1e-10 * np.abs(lu_ref).max()
+
+
+@pytest.mark.parametrize("N,terms,mixed", [(10, 5, 0), (34, 5, 0), (35, 5, 1), (69, 5, 1), (103, 5, 0), (53, 7, 1),
+                                           (171, 3, 0), (177, 4, 1)])
+def test_fp32_factor_solve_at_block_edges(N, terms, mixed):
+    """(LU)^-1 r with FP32 factors against numpy, for systems below, at and
+    just past multiples of the 512-row diagonal blocks and the 64-row blocks
+    they are merged from; FP32 factors of a well-conditioned system."""
+    pos, ori = layout(N, 1e-2, 4000 + N)
+    p = rf.default_params(num_terms=terms, precond=rf.PRECOND_LU, lu_factor_fp32=1, precision=mixed, gmres_tol=1e-10,
+                          gmres_restart=30, gmres_max_iters=300)
+    with rf.Simulation(rf.Configuration(p, pos, ori)) as sim:
+        sim.assemble_system()
+        sim.solve_system()
+        assert sim.stats().last_backward_error <= 1e-10
+        A = sim.matrix()
+        r = np.random.default_rng(N).normal(size=sim.n)
+        z = sim.precond_apply(r)
+        again = sim.precond_apply(r)
+    ref = np.linalg.solve(A, r)
+    assert np.array_equal(z, again)
+    assert np.linalg.norm(z - ref) <= 1e-5 * np.linalg.norm(ref)
