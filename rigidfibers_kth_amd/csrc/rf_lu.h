@@ -25,9 +25,19 @@ namespace rf {
 // panel, reading the check through host_flag (two ints of coherent pinned
 // host memory: the flag and the copy's sequence word, which the host polls)
 // when it is not null.  info[0..1] are zero on entry.
+//
+// side (may be null): a second stream and two events.  The trailing columns
+// beyond the next super-panel are then updated on it while that super-panel
+// is factorised on s; s has waited for all of it when its own work is done,
+// and the side stream starts after what s holds at the call.
+struct LuSide {
+    hipStream_t stream = nullptr;
+    hipEvent_t main_done = nullptr, side_done = nullptr;
+};
 size_t lu_workspace_bytes(int n, int update_fp16);
 hipError_t lu_factor(void* A, int elem_bytes, int64_t lda, int n, int nb, int* ipiv, int* info, int use_mfma,
-                     int block_pivot, int update_fp16, void* ws, int* redone, int* host_flag, hipStream_t s);
+                     int block_pivot, int update_fp16, void* ws, int* redone, int* host_flag, hipStream_t s,
+                     const LuSide* side = nullptr);
 // x <- U^-1 L^-1 P x with FP64 vectors, one launch per 64-row block and
 // sweep (FP32 or FP64 factors).  aux holds
 // lu_solve_aux_bytes(n, elem_bytes): the row permutation and the inverses of

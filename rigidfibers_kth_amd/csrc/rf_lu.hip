@@ -1,19 +1,22 @@
 // rf_lu.hip -- dense LU with partial pivoting on gfx950 (the direct solver,
 // LAPACK dgesv at fortran/coeffs_and_vels.f90:62,158,333,514).
 //
-// Blocked right-looking factorisation, column-major, panel width NB, the
-// trailing update delayed to every second panel (super-panels of 2 NB):
-//   for each panel [k0, k1) (first bringing its columns up to date):
-//     either the block-pivoted panel (diagonal block in LDS, L21 = A21 U11^-1,
-//       checked against partial pivoting) or the column-by-column (Crout)
-//       panel with the pivot search over the whole column;
-//     apply the panel's row swaps to the other columns (laswp);
-//     U12 = L11^-1 A12 (unit lower triangular solve, the panel's rows first
-//       brought up to date);
-//   A22 -= L21 U12 once per super-panel on the matrix cores
-//     (v_mfma_f64_16x16x4f64 for FP64, v_mfma_f32_16x16x4f32 for FP32
-//     factors, or v_mfma_f32_16x16x32_f16 on fp16-rounded operands for FP32
-//     factors that only precondition).
+// Blocked factorisation, column-major, panel width NB (64), the trailing
+// update delayed to the end of each super-panel (512 columns in FP64, 1024 in
+// FP32):
+//   for each panel [k0, k1), its columns first brought up to date:
+//     either the block-pivoted panel (pivots inside the diagonal block,
+//       L21 = A21 U11^-1, checked against partial pivoting) or the
+//       column-by-column (Crout) panel with the pivot search over the whole
+//       column;
+//     the panel's row swaps and U12 = L11^-1 A12 on the super-panel's columns;
+//   the super-panel's swaps and U12 on the columns beyond, then
+//   A22 -= L21 U12 on the matrix cores (v_mfma_f64_16x16x4f64 for FP64,
+//     v_mfma_f32_16x16x4f32 for FP32 factors, or v_mfma_f32_16x16x32_f16 on
+//     fp16-rounded operands for FP32 factors that only precondition).
+// The panels are a chain of small launches, the updates fill the chip: with a
+// side stream the update of the columns beyond the next super-panel runs
+// beside that super-panel's chain.
 // Pivots: first index of the largest |a_ik| (LAPACK idamax), so the pivot
 // sequence is dgesv's whenever the arithmetic agrees.
 #include "rf_internal.h"
@@ -30,6 +33,10 @@ namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+
+// Wave priority of the panel chain's kernels: they run beside the side stream's
+// updates, which fill every CU (direct step at N=1000 59.5 -> 58.5 ms).
+constexpr int kChainPriority = 3;
 
 constexpr int kColThreads = 256;
 constexpr int kColMaxBlocks = 512;
@@ -441,100 +448,213 @@ __device__ __forceinline__ double wave_max(double v)
     return lane_value(v, 63);
 }
 
-// Diagonal block of width nb <= 64 by four wavefronts: lane r of wavefront w
-// holds row r of the columns [16 w, 16 w + 16) in registers (the column loop
-// fully unrolled).  For column j the wavefront that owns it finds the pivot
-// (the first largest |a_rj| over the rows not yet pivots, ties to the smaller
-// position in LAPACK's swapped order, as idamax), scales the column and
-// publishes the multipliers (0 for pivot rows) and the pivot lane in LDS;
-// after one barrier every wavefront subtracts l_r u_c from its columns c > j,
-// the pivot row's u_c coming from readlane.  Rows are not moved while the
-// block is factorised: each lane keeps the position its row holds in the
-// swapped order and every row is stored at its final position at the end.
-// Non-pivot rows take exactly the operations of a row-by-row elimination;
-// pivot rows take l = 0, which leaves them unchanged up to the sign of an
-// exact zero.  bak receives the original values, ipiv and info[1] as in
-// lu_diag_kernel.
-constexpr int kDiagCols = 16;  // columns per wavefront
-template <typename T>
-__global__ void __launch_bounds__(256) lu_diag64_kernel(T* A, int64_t lda, int k0, int nb, int* ipiv, int* info,
-                                                        T* __restrict__ bak, int64_t ldb)
+// Column c of the inverse of a 16 x 16 triangle (get(i, j): its entries; unit
+// diagonal for the lower one) into out[i] = X[i][c], by substitution.
+template <typename T, typename F>
+__device__ __forceinline__ void inverse16_column(bool upper, int c, F&& get, T* __restrict__ out)
 {
-    __shared__ T sl[2][64];
-    __shared__ int sp[2];
+    T x[16];
+    if (!upper) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            T v = (i == c) ? T(1) : T(0);
+#pragma unroll
+            for (int k = 0; k < i; ++k) v -= get(i, k) * x[k];
+            x[i] = v;
+        }
+    } else {
+#pragma unroll
+        for (int i = 15; i >= 0; --i) {
+            T v = (i == c) ? T(1) : T(0);
+#pragma unroll
+            for (int k = i + 1; k < 16; ++k) v -= get(i, k) * x[k];
+            x[i] = v / get(i, i);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) out[i] = x[i];
+}
+
+// Inverses of the 16 x 16 diagonal blocks of a 64-column panel's U11 (blocks 0
+// to 3) and L11 (4 to 7), column-major, 256 values each: the substitutions
+// with them are matrix-core products (lu_l21_kernel64, lu_rows_kernel).
+constexpr int kPanelInv = 8 * 256;
+
+// The same from the factored panel in the matrix (after a column-by-column panel).
+template <typename T>
+__global__ void __launch_bounds__(128) lu_inv16_kernel(const T* __restrict__ A, int64_t lda, int k0,
+                                                       T* __restrict__ inv)
+{
+    const int q = threadIdx.x / 16, c = threadIdx.x % 16, at = k0 + 16 * (q & 3);
+    inverse16_column<T>(
+        q < 4, c, [&](int i, int j) { return A[(int64_t)(at + j) * lda + at + i]; }, inv + q * 256 + c * 16);
+}
+
+// max(v, v of the lane selected by DPP control CTRL), unsigned.
+template <int CTRL, int ROWMASK>
+__device__ __forceinline__ unsigned dpp_umax(unsigned v)
+{
+    return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWMASK, 0xF, false));
+}
+__device__ __forceinline__ unsigned wave_umax(unsigned v)  // as wave_max
+{
+    v = dpp_umax<0x111, 0xF>(v);
+    v = dpp_umax<0x112, 0xF>(v);
+    v = dpp_umax<0x114, 0xF>(v);
+    v = dpp_umax<0x118, 0xF>(v);
+    v = dpp_umax<0x142, 0xA>(v);
+    v = dpp_umax<0x143, 0xC>(v);
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+// The top 32 bits of |v|: ordered as |v| up to ties.
+__device__ __forceinline__ unsigned magnitude_key(float v) { return (unsigned)__float_as_int(v) & 0x7FFFFFFFu; }
+__device__ __forceinline__ unsigned magnitude_key(double v)
+{
+    return (unsigned)((unsigned long long)__double_as_longlong(v) >> 32) & 0x7FFFFFFFu;
+}
+
+// Diagonal block of width nb <= 64 by eight wavefronts: lane r of wavefront w
+// holds row r of the columns [8 w, 8 w + 8) in registers.  In turn each
+// wavefront factorises its 8 columns without a barrier: for column j it finds
+// the pivot (the first largest |a_rj| over the rows not yet pivots, ties to
+// the smaller position in LAPACK's swapped order, as idamax), scales the
+// column and updates its remaining columns, the pivot row's entries coming
+// from readlane; multipliers (0 for pivot rows) and pivot lanes go to LDS, and
+// after one barrier per 8 columns the later wavefronts subtract the 8 rank-1
+// terms from theirs.  Rows are not moved while the block is factorised: each
+// lane keeps the position its row holds in the swapped order and every row is
+// stored at its final position at the end.  Non-pivot rows take exactly the
+// operations of a row-by-row elimination; pivot rows take l = 0, which leaves
+// them unchanged up to the sign of an exact zero.  bak receives the original
+// values, ipiv and info[1] as in lu_diag_kernel.
+// Bound by the dependent chain of a column and by instruction fetch (a launch
+// starts on a cold instruction cache), so both are kept short: the column loop
+// is not unrolled (column j sits in cur, the later ones move down one register
+// as they are updated); only the next column takes column j's update at once,
+// the others while the next pivot is searched; the maximum runs over the top
+// 32 bits (the full comparison only when several rows share them); every lane
+// divides its own entry while the maximum is found.  28 us in FP64 and 23 us in
+// FP32 per block (31 and 25 with the inverses below), 36 and 38 us with 64 unrolled
+// columns over four wavefronts and a barrier each.
+constexpr int kDiagCols = 8;  // columns per wavefront
+constexpr int kDiag64Threads = 64 * (64 / kDiagCols);
+template <typename T>
+__global__ void __launch_bounds__(kDiag64Threads) lu_diag64_kernel(T* A, int64_t lda, int k0, int nb, int* ipiv,
+                                                                   int* info, T* __restrict__ bak, int64_t ldb,
+                                                                   T* __restrict__ inv16)
+{
+    __builtin_amdgcn_s_setprio(kChainPriority);
+    __shared__ int row_at[64];         // lane of the row at each final position
+    __shared__ T S[64][64];            // finished columns: S[c][lane]
+    __shared__ T sl[kDiagCols][64];    // multipliers of the 8 columns in turn, 0 for pivot rows
+    __shared__ int sp[kDiagCols];      // their pivot lanes
+    __shared__ int spos[64];           // row positions after the last 8 columns, -1 - position for pivot rows
     const int r = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;  // wavefront-uniform
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c0 = w * kDiagCols;
     const bool live = r < nb;
     T a[kDiagCols];
 #pragma unroll
-    for (int c = 0; c < kDiagCols; ++c)
-        a[c] = (live && c0 + c < nb) ? A[(int64_t)(k0 + c0 + c) * lda + k0 + r] : T(0);
+    for (int c = 0; c < kDiagCols; ++c) a[c] = A[(int64_t)(k0 + min(c0 + c, nb - 1)) * lda + k0 + min(r, nb - 1)];
 #pragma unroll
-    for (int c = 0; c < kDiagCols; ++c)
-        if (live && c0 + c < nb) bak[(int64_t)(c0 + c) * ldb + r] = a[c];
-    int pos = r, my_ipiv = r;
+    for (int c = 0; c < kDiagCols; ++c) {
+        const bool in = live && c0 + c < nb;
+        if (in) bak[(int64_t)(c0 + c) * ldb + r] = a[c];
+        a[c] = in ? a[c] : T(0);
+    }
+    int pos = r;
     bool done = !live;
     bool zero = false;
-    // compile-time column indices keep a[] in registers
-    static_for<64>([&](auto jc) {
-        constexpr int j = decltype(jc)::value;
-        constexpr int owner = j / kDiagCols, jl = j % kDiagCols, par = j & 1;
-        if (j < nb) {  // uniform over the workgroup
-            if (w == owner) {
-                const double v = done ? -1.0 : fabs((double)a[jl]);
-                const double vmax = wave_max(v);
-                const unsigned long long cand = __ballot(v == vmax);
-                int p;
-                if (__popcll(cand) == 1) {
-                    p = __ffsll((unsigned long long)cand) - 1;
-                } else {  // exact ties (or no candidate left): the smallest position
-                    int k = (v == vmax) ? pos : 1 << 20;
+    const int turns = (nb + kDiagCols - 1) / kDiagCols;
+#pragma unroll 1
+    for (int s = 0; s < turns; ++s) {
+        const int cols = min(kDiagCols, nb - s * kDiagCols);
+        if (w == s) {
+            T cur = a[0], lprev = T(0);  // the later columns still lack lprev times row pprev
+            int pprev = 0, my_p = 0, my_pos = 0;  // lane jl: pivot lane of column jl and the position it came from
+#pragma unroll 1
+            for (int jl = 0; jl < cols; ++jl) {
+                const unsigned key = (!done && cur == cur) ? magnitude_key(cur) + 1u : 0u;
+                const unsigned kmax = wave_umax(key);
+                T rec = T(1) / (cur != T(0) ? cur : T(1));
+                T nxt = a[1] - lprev * lane_value(a[1], pprev);
+#pragma unroll
+                for (int c = 2; c < kDiagCols; ++c) a[c - 1] = a[c] - lprev * lane_value(a[c], pprev);
+                // keep this work here, beside the search, and off the path after it
+                asm volatile("" : "+v"(rec), "+v"(nxt));
+#pragma unroll
+                for (int c = 1; c < kDiagCols - 1; ++c) asm volatile("" : "+v"(a[c]));
+                const unsigned long long cand = __ballot(key == kmax);
+                int p = __ffsll((unsigned long long)cand) - 1;
+                if (__builtin_expect(kmax <= 1u || (cand & (cand - 1)) != 0, 0)) {
+                    // equal keys (or only zeros): the full values, then the smallest position
+                    const double v = (key == kmax && !done) ? fabs((double)cur) : -1.0;
+                    const double vmax = wave_max(v);
+                    if (!(vmax > 0.0)) zero = true;
+                    int k = (v == vmax && !done) ? pos : 1 << 20;
 #pragma unroll
                     for (int off = 32; off > 0; off >>= 1) k = min(k, __shfl_xor(k, off, 64));
-                    const unsigned long long at = __ballot(v == vmax && pos == k);
+                    const unsigned long long at = __ballot(v == vmax && pos == k && !done);
                     p = at ? __ffsll((unsigned long long)at) - 1 : 0;
                 }
                 p = __builtin_amdgcn_readfirstlane(p);
-                if (!(vmax > 0.0)) zero = true;
-                const T piv = lane_value(a[jl], p);
-                const T inv = (piv != T(0)) ? T(1) / piv : T(0);
+                const T inv = lane_value(rec, p);  // a zero pivot leaves its (all zero) column as it is
                 const bool pivot_row = done || r == p;
-                const T l = a[jl] * inv;
-                if (!pivot_row) a[jl] = l;
-                sl[par][r] = pivot_row ? T(0) : l;
-                if (r == 0) sp[par] = p;
+                const T l = cur * inv;
+                const T lz = pivot_row ? T(0) : l;
+                S[c0 + jl][r] = pivot_row ? cur : l;
+                sl[jl][r] = lz;
+                cur = nxt - lz * lane_value(nxt, p);
+                lprev = lz;
+                pprev = p;
+                const int j = c0 + jl, ppos = __builtin_amdgcn_readlane(pos, p);
+                my_p = (r == jl) ? p : my_p;
+                my_pos = (r == jl) ? ppos : my_pos;
+                pos = (r == p) ? j : (pos == j) ? ppos : pos;  // the row at position j moves to the pivot's position
+                done = pivot_row;
             }
-            __syncthreads();
-            const int p = __builtin_amdgcn_readfirstlane(sp[par]);
-            const T lr = sl[par][r];
-            const int ppos = __builtin_amdgcn_readlane(pos, p);
-            if (r == j) my_ipiv = ppos;
-            if (r != p && pos == j) pos = ppos;  // the row at position j moves to the pivot's position
-            if (r == p) {
-                pos = j;
-                done = true;
-            }
-            if (w == owner) {
-                static_for<kDiagCols>([&](auto cc) {
-                    constexpr int c = decltype(cc)::value;
-                    if constexpr (c > jl) a[c] -= lr * lane_value(a[c], p);
-                });
-            } else if (w > owner) {
-                static_for<kDiagCols>([&](auto cc) {
-                    constexpr int c = decltype(cc)::value;
-                    a[c] -= lr * lane_value(a[c], p);
-                });
+            spos[r] = done ? -1 - pos : pos;
+            if (r < cols) {
+                sp[r] = my_p;
+                ipiv[k0 + c0 + r] = k0 + my_pos;
             }
         }
-    });
+        __syncthreads();
+        const int st = spos[r];
+        done = st < 0;
+        pos = done ? -1 - st : st;
+        if (w > s) {  // w > s: all kDiagCols columns of turn s exist
+            T lr[kDiagCols];
+            int p[kDiagCols];
+#pragma unroll
+            for (int jl = 0; jl < kDiagCols; ++jl) {
+                lr[jl] = sl[jl][r];
+                p[jl] = __builtin_amdgcn_readfirstlane(sp[jl]);
+            }
+#pragma unroll
+            for (int jl = 0; jl < kDiagCols; ++jl)
+#pragma unroll
+                for (int c = 0; c < kDiagCols; ++c) a[c] -= lr[jl] * lane_value(a[c], p[jl]);
+        }
+        if (s + 1 < turns) __syncthreads();  // sl, sp and the row state have no readers left
+    }
     if (live) {
 #pragma unroll
         for (int c = 0; c < kDiagCols; ++c)
-            if (c0 + c < nb) A[(int64_t)(k0 + c0 + c) * lda + k0 + pos] = a[c];
-        if (w == 0) ipiv[k0 + r] = k0 + my_ipiv;
+            if (c0 + c < nb) A[(int64_t)(k0 + c0 + c) * lda + k0 + pos] = S[c0 + c][r];
     }
     if (r == 0 && zero) info[1] = 1;  // zero pivot: left to the column-by-column panel
+    if (!inv16) return;  // (nb = 64 otherwise)
+    if (w == 0) row_at[pos] = r;
+    __syncthreads();
+    if (r < 16) {  // wavefront w: block w of inv16
+        const int at = 16 * (w & 3);
+        int rl[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) rl[i] = row_at[at + i];
+        inverse16_column<T>(
+            w < 4, r, [&](int i, int j) { return S[at + j][rl[i]]; }, inv16 + w * 256 + r * 16);
+    }
 }
 
 // Broadcast of lane SRC of each group of 4 lanes (DPP quad_perm).
@@ -706,6 +826,322 @@ __global__ void __launch_bounds__(256) lu_u12_kernel(T* A, int64_t lda, int n, i
             colscale[col] = combine ? fminf(colscale[col], sc) : sc;
         }
     }
+}
+
+// ---- 64-column panels on the matrix cores -----------------------------------
+// v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32: lane (lr = l % 16, lk = l / 16)
+// supplies A[lr][lk] and B[lk][lr]; register r of the result is D[4 r + lk][lr]
+// in FP64 and D[4 lk + r][lr] in FP32 (rf_selftest_mfma_layout).  With
+// sub(r) that row, register r of a 16 x 16 result is exactly the B operand of
+// step r of a following product whose step r takes the inner indices sub(r):
+// a chain of block products needs no exchange between lanes.
+template <typename T>
+struct Mf;
+template <>
+struct Mf<double> {
+    using V = d4;
+    typedef double P __attribute__((ext_vector_type(2)));
+    static __device__ __forceinline__ int sub(int r, int lk) { return 4 * r + lk; }
+    static __device__ __forceinline__ d4 mul(double a, double b, d4 c)
+    {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    // four consecutive values (16-byte aligned)
+    static __device__ __forceinline__ d4 load4(const double* p)
+    {
+        const P u = *reinterpret_cast<const P*>(p), v = *reinterpret_cast<const P*>(p + 2);
+        return d4{u[0], u[1], v[0], v[1]};
+    }
+};
+template <>
+struct Mf<float> {
+    using V = f4;
+    static __device__ __forceinline__ int sub(int r, int lk) { return 4 * lk + r; }
+    static __device__ __forceinline__ f4 mul(float a, float b, f4 c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ f4 load4(const float* p) { return *reinterpret_cast<const f4*>(p); }
+};
+
+// L21 = A21 U11^-1 and its check, as lu_l21_kernel, for a 64-column panel: a
+// wavefront takes 16 rows, X_b = (A_b - sum_{q<b} X_q U_qb) inv(U_bb) over the
+// four 16-column blocks, everything transposed (D = X_b^T) so that rows lie
+// along the lanes.  All loads are issued first.
+// 10.8 us at n = 15000 in FP64 and 7.2 us at n = 30000 in FP32, against 21 and
+// 17.7 us for a quad-per-row substitution with its 64 dependent steps.
+template <typename T>
+__global__ void __launch_bounds__(256) lu_l21_kernel64(T* A, int64_t lda, int n, int k0, int* info,
+                                                       T* __restrict__ bak, int64_t ldb, const T* __restrict__ inv16)
+{
+    __builtin_amdgcn_s_setprio(kChainPriority);
+    using M = Mf<T>;
+    using V = typename M::V;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
+    const int row = k0 + 64 + blockIdx.x * 64 + wave * 16 + lr;
+    const bool live = row < n;
+    T* Ar = A + (int64_t)k0 * lda + min(row, n - 1);
+    V x[4], u[6], iv[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[b][r] = Ar[(int64_t)(16 * b + M::sub(r, lk)) * lda];
+#pragma unroll
+    for (int b = 1; b < 4; ++b)
+#pragma unroll
+        for (int q = 0; q < b; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                u[b * (b - 1) / 2 + q][r] = -A[(int64_t)(k0 + 16 * b + lr) * lda + k0 + 16 * q + M::sub(r, lk)];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) iv[b][r] = inv16[b * 256 + lr * 16 + M::sub(r, lk)];
+    if (live) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) bak[(int64_t)(16 * b + M::sub(r, lk)) * ldb + (row - k0)] = x[b][r];
+    }
+    bool big = false;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+#pragma unroll
+        for (int q = 0; q < b; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[b] = M::mul(u[b * (b - 1) / 2 + q][r], x[q][r], x[b]);
+        V y = V{0, 0, 0, 0};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y = M::mul(iv[b][r], x[b][r], y);
+        x[b] = y;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            big |= !(fabs((double)y[r]) <= 1.0);  // NaN included
+            if (live) Ar[(int64_t)(16 * b + M::sub(r, lk)) * lda] = y[r];
+        }
+    }
+    if (live && big) atomicOr(&info[1], 1);
+}
+
+// A panel's columns caught up with the earlier panels of its 256-column block:
+// C[k0:n, k0:k0+cols) -= L[k0:n, K0:k0) U[K0:k0, those columns), cols <= 64,
+// k0 - K0 a multiple of 64.  Operand fragments come straight from memory
+// (the U block is small, L is read once), one group of 16 K ahead of the
+// products: no LDS, no barriers, so a wavefront's time is its products' (64 or
+// 32 cycles each).  A wavefront takes 16 rows x 16 NCB columns; NCB = 4 where the
+// rows alone fill the chip, 1 below (four times the wavefronts, a quarter of
+// the chain).  The accumulators hold -C^T (D = (L U)^T: rows along the lanes).
+// 12 us + 3.5 us per 64 of K at n = 30000 in FP32 (22 us for fp16 tiles staged
+// through LDS over up to 960 of K), 5.8 us at n = 1500 in FP64 (26 us).
+template <typename T, int NCB>
+__global__ void __launch_bounds__(256) lu_cols_kernel(T* A, int64_t lda, int n, int K0, int k0, int cols)
+{
+    __builtin_amdgcn_s_setprio(kChainPriority);
+    using M = Mf<T>;
+    using V = typename M::V;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
+    const int rt = (NCB == 4) ? blockIdx.x * 4 + wave : blockIdx.x;   // 16-row tile
+    const int cb = (NCB == 4) ? 0 : wave;                             // first 16-column block
+    const int row = k0 + rt * 16 + lr;
+    if (k0 + rt * 16 >= n || 16 * cb >= cols) return;  // (uniform; no barriers below)
+    const int rowc = min(row, n - 1);
+    V acc[NCB];
+    const T* up[NCB];
+#pragma unroll
+    for (int j = 0; j < NCB; ++j) {
+        const int c0 = 16 * (cb + j);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[j][r] = -A[(int64_t)(k0 + min(c0 + M::sub(r, lk), cols - 1)) * lda + rowc];
+        up[j] = A + (int64_t)(k0 + min(c0 + lr, cols - 1)) * lda + K0 + 4 * lk;
+    }
+    const T* lp = A + (int64_t)(K0 + 4 * lk) * lda + rowc;
+    const int groups = (k0 - K0) / 16;
+    V lv, uv[NCB];
+    auto load = [&](V& l, V(&u)[NCB], int g) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) l[r] = lp[(int64_t)(16 * g + r) * lda];
+#pragma unroll
+        for (int j = 0; j < NCB; ++j) u[j] = M::load4(up[j] + 16 * g);
+    };
+    auto multiply = [&](const V& l, const V(&u)[NCB]) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < NCB; ++j) acc[j] = M::mul(u[j][r], l[r], acc[j]);
+    };
+    // three groups in flight
+    V lv1, uv1[NCB], lv2, uv2[NCB], lv3, uv3[NCB];
+    load(lv, uv, 0);
+    load(lv1, uv1, 1);
+    load(lv2, uv2, 2);
+    for (int g = 0; g < groups; g += 4) {  // groups is a multiple of 4
+        load(lv3, uv3, g + 3);
+        multiply(lv, uv);
+        load(lv, uv, min(g + 4, groups - 1));
+        multiply(lv1, uv1);
+        load(lv1, uv1, min(g + 5, groups - 1));
+        multiply(lv2, uv2);
+        load(lv2, uv2, min(g + 6, groups - 1));
+        multiply(lv3, uv3);
+    }
+    if (row >= n) return;
+#pragma unroll
+    for (int j = 0; j < NCB; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int c = 16 * (cb + j) + M::sub(r, lk);
+            if (c < cols) A[(int64_t)(k0 + c) * lda + row] = -acc[j][r];
+        }
+}
+
+// Row swaps ipiv[ka..kb) (kb - ka <= 64) applied to column c of A (one lane per
+// column), in order; most pivots are their own row.
+template <typename T>
+__device__ __forceinline__ void swap_rows(T* A, int64_t lda, int ka, int kb, const int* __restrict__ ipiv, int c,
+                                          bool live)
+{
+    const int lane = threadIdx.x & 63;
+    const int piv = (ka + lane < kb) ? ipiv[ka + lane] : ka + lane;
+    unsigned long long todo = __ballot(piv != ka + lane);
+    T* cc = A + (int64_t)c * lda;
+    while (todo) {
+        const int i = __ffsll(todo) - 1;
+        todo &= todo - 1;
+        const int p = __builtin_amdgcn_readlane(piv, i);
+        if (live) {
+            const T t = cc[ka + i];
+            cc[ka + i] = cc[p];
+            cc[p] = t;
+        }
+    }
+}
+
+// Rows of the panels [ka, kb) (64 columns each, inside the 256-column block
+// from K0) brought to their final U values in the columns [cbeg, cend): for
+// each panel in turn its row swaps (ipiv null: already applied), the catch-up
+// with the block's earlier rows, U12 -= L[panel, K0:panel) U[K0:panel), and
+// U12 = L11^-1 U12.  16 columns per workgroup, wavefront b the panel's rows
+// 16 b ..; the substitution over 16-row blocks multiplies with the inverted
+// diagonal blocks (inv16, one set per panel), a solved block going to the
+// other wavefronts through LDS.  With colscale the largest |u| of each column
+// gives the power of two that takes it into [2^11, 2^12) for the fp16 update
+// (combine: the smaller of this and the one already there).
+// One launch for up to four panels in place of a swap, a product and a
+// substitution each (5 + 27 + 13 us a panel, FP64 n = 15000): 15 us on a
+// super-panel's own columns at n = 1500, bound by the chain of loads, products
+// and LDS hand-overs of a panel.
+template <typename T>
+__global__ void __launch_bounds__(256) lu_rows_kernel(T* A, int64_t lda, const int* __restrict__ ipiv,
+                                                      const T* __restrict__ inv16, int K0, int ka, int kb, int cbeg,
+                                                      int cend, float* __restrict__ colscale, int combine)
+{
+    if (ipiv) __builtin_amdgcn_s_setprio(kChainPriority);
+    using M = Mf<T>;
+    using V = typename M::V;
+    __shared__ T xs[3][4][64];  // solved blocks 0..2 as B operands
+    __shared__ float smax[4][16];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lr = lane & 15, lk = lane >> 4;
+    const int col = cbeg + 16 * blockIdx.x + lr;
+    const bool live = col < cend;
+    const int colc = min(col, cend - 1);
+    T* Ac = A + (int64_t)colc * lda;
+    float cmax = 0.f;
+    for (int k0 = ka; k0 < kb; k0 += 64) {
+        if (ipiv) {
+            if (wave == 0) swap_rows(A, lda, k0, k0 + 64, ipiv, colc, live && lk == 0);
+            __syncthreads();  // the swaps are in place
+        }
+        const T* Lr = A + k0 + 16 * wave + lr;  // this wavefront's rows of L
+        V acc;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] = Ac[k0 + 16 * wave + M::sub(r, lk)];
+        V lb[3], iv;
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) lb[q][r] = (q < wave) ? -Lr[(int64_t)(k0 + 16 * q + M::sub(r, lk)) * lda] : T(0);
+        const T* ip = inv16 + (size_t)(k0 / 64) * kPanelInv + (4 + wave) * 256 + lr;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) iv[r] = ip[16 * M::sub(r, lk)];
+        const int groups = (k0 - K0) / 16;
+        if (groups > 0) {
+            auto load = [&](V& l, V& u, int g) {
+                u = M::load4(Ac + K0 + 16 * g + 4 * lk);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) l[r] = -Lr[(int64_t)(K0 + 16 * g + 4 * lk + r) * lda];
+            };
+            auto multiply = [&](const V& l, const V& u) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc = M::mul(l[r], u[r], acc);
+            };
+            V l0, u0, l1, u1, l2, u2, l3, u3;
+            load(l0, u0, 0);
+            load(l1, u1, 1);
+            load(l2, u2, 2);
+            for (int g = 0; g < groups; g += 4) {  // groups is a multiple of 4
+                load(l3, u3, g + 3);
+                multiply(l0, u0);
+                load(l0, u0, min(g + 4, groups - 1));
+                multiply(l1, u1);
+                load(l1, u1, min(g + 5, groups - 1));
+                multiply(l2, u2);
+                load(l2, u2, min(g + 6, groups - 1));
+                multiply(l3, u3);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (wave == q) {
+                V y = V{0, 0, 0, 0};
+#pragma unroll
+                for (int r = 0; r < 4; ++r) y = M::mul(iv[r], acc[r], y);
+                acc = y;
+                if (q < 3) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) xs[q][r][lane] = acc[r];
+                }
+            }
+            if (q == 3) break;
+            __syncthreads();
+            if (wave > q) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc = M::mul(lb[q][r], xs[q][r][lane], acc);
+            }
+        }
+        if (live) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                Ac[k0 + 16 * wave + M::sub(r, lk)] = acc[r];
+                cmax = fmaxf(cmax, fabsf((float)acc[r]));
+            }
+        }
+        __syncthreads();  // the panel's rows are stored, xs is free
+    }
+    if (colscale) {
+        cmax = fmaxf(cmax, __shfl_xor(cmax, 16, 64));
+        cmax = fmaxf(cmax, __shfl_xor(cmax, 32, 64));
+        if (lk == 0) smax[wave][lr] = cmax;
+        __syncthreads();
+        if (wave == 0 && lk == 0 && live) {
+            const float m = fmaxf(fmaxf(smax[0][lr], smax[1][lr]), fmaxf(smax[2][lr], smax[3][lr]));
+            const int e = (m > 0.f && m <= 3.0e38f) ? ilogbf(m) : 11;
+            const float sc = ldexpf(1.f, min(60, max(-60, 11 - e)));
+            colscale[col] = combine ? fminf(colscale[col], sc) : sc;
+        }
+    }
+}
+
+// Row swaps ipiv[ka..kb) applied to the columns [cbeg, cend): 64 columns per wavefront.
+template <typename T>
+__global__ void __launch_bounds__(64) lu_swap_kernel(T* A, int64_t lda, int ka, int kb, const int* __restrict__ ipiv,
+                                                     int cbeg, int cend)
+{
+    const int c = cbeg + blockIdx.x * 64 + threadIdx.x;
+    for (int k = ka; k < kb; k += 64) swap_rows(A, lda, k, min(kb, k + 64), ipiv, min(c, cend - 1), c < cend);
 }
 
 // Panel columns [k0, k0+nb), rows [k0, n), back from the copy the two
@@ -971,7 +1407,7 @@ __global__ void __launch_bounds__(256) lu_gemm_mfma_kernel(T* A, int64_t lda, Ge
         }
 }
 
-constexpr int kXcds = 8, kCusPerXcd = 32;
+constexpr int kXcds = 8;
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 // 16 bytes per lane from src straight into LDS at dst (wavefront-uniform; lane
@@ -1416,14 +1852,14 @@ __global__ void __launch_bounds__(256) pack_l_kernel(const float* __restrict__ A
 }
 
 // U: one thread per column and 8-K segment (two 16-byte reads, one write).
-__global__ void __launch_bounds__(256) pack_u_kernel(const float* __restrict__ A, int64_t lda, int n, int K0, int K1,
-                                                     int kwp, const float* __restrict__ colscale,
+__global__ void __launch_bounds__(256) pack_u_kernel(const float* __restrict__ A, int64_t lda, int c0, int c1, int K0,
+                                                     int K1, int kwp, const float* __restrict__ colscale,
                                                      _Float16* __restrict__ Up)
 {
     const int segs = kwp / 8;
     const int64_t gidx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int col = K1 + (int)(gidx / segs), seg = (int)(gidx % segs);
-    if (col >= n) return;
+    const int col = c0 + (int)(gidx / segs), seg = (int)(gidx % segs);
+    if (col >= c1) return;
     const int kw = K1 - K0, k0 = seg * 8;
     const float sc = colscale[col];
     const float* src = A + (int64_t)col * lda + K0 + k0;
@@ -1471,11 +1907,11 @@ struct HalfFromPacked {
     }
 };
 
-// The trailing update of a super-panel from the packed operands: rows and
-// columns [K1, n), kwp / 32 chunks of K.  Three workgroups per CU (168
+// The trailing update of a super-panel from the packed operands: rows [K1, n),
+// columns [c0, c1), kwp / 32 chunks of K.  Three workgroups per CU (168
 // VGPRs, accumulators in VGPRs): 1.6 % faster than two at n = 60000; four
 // spill the tile pointers and are 18 % slower.
-__global__ void __launch_bounds__(256, 3) lu_gemm_f16p_kernel(float* A, int64_t lda, int n, int K1, int kwp,
+__global__ void __launch_bounds__(256, 3) lu_gemm_f16p_kernel(float* A, int64_t lda, int n, int K1, int c0, int c1, int kwp,
                                                           const _Float16* __restrict__ Lp,
                                                           const _Float16* __restrict__ Up,
                                                           const float* __restrict__ colscale)
@@ -1486,11 +1922,11 @@ __global__ void __launch_bounds__(256, 3) lu_gemm_f16p_kernel(float* A, int64_t 
     st.Lp = Lp;
     st.Up = Up;
     st.ri = blockIdx.x * kHB;
-    st.cj = blockIdx.y * kHB;
+    st.cj = c0 - K1 + blockIdx.y * kHB;
     st.rn = n - K1;
-    st.cn = n - K1;
+    st.cn = c1 - K1;
     const bool vec = (K1 % 4 == 0) && (lda % 4 == 0);
-    f16_update_tile<kHB, kHB>(A, lda, K1 + st.ri, K1 + st.cj, n, n, vec, kwp / kHK, st, colscale, As, Bs);
+    f16_update_tile<kHB, kHB>(A, lda, K1 + st.ri, K1 + st.cj, n, c1, vec, kwp / kHK, st, colscale, As, Bs);
 }
 
 // The same update with wide tiles: 256 rows, and each wavefront a 128-row
@@ -1525,14 +1961,12 @@ struct WideCfg {
     static constexpr int kStageHalves = kWB * kHK + kBHalves;
     static constexpr int kJB = TN / 32;                      // 16-column blocks per wavefront
     static constexpr int kLoads = 4 + TN / 64;               // ring loads per wavefront and chunk
-    static constexpr int kBlockRows = (TN == 256) ? 4 : 8;   // tiles per XCD round: WG per CU of the XCD
-    static constexpr int kBlockCols = kCusPerXcd * WG / kBlockRows;
+    static constexpr int kStrip = (TN == 256) ? 4 : 8;       // tile rows of an XCD's strip: as many tiles across as down
 };
-using WideTwo = WideCfg<128, 3, 2>;
 
 template <int TN, int STAGES, int WG>
-__global__ void __launch_bounds__(256, WG) lu_gemm_f16w_kernel(float* A, int64_t lda, int n, int K1, int kwp,
-                                                           const _Float16* __restrict__ Lp,
+__global__ void __launch_bounds__(256, WG) lu_gemm_f16w_kernel(float* A, int64_t lda, int n, int K1, int c0, int c1,
+                                                           int kwp, const _Float16* __restrict__ Lp,
                                                            const _Float16* __restrict__ Up,
                                                            const float* __restrict__ colscale)
 {
@@ -1543,21 +1977,10 @@ __global__ void __launch_bounds__(256, WG) lu_gemm_f16w_kernel(float* A, int64_t
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wr = (wave >> 1) * 128, wc = (wave & 1) * (TN / 2);
     const int lr = lane & 15, lg = lane >> 4;
-    const int rn = n - K1;
-    // Tile of this workgroup: workgroup ids go round-robin over the 8 XCDs,
-    // and the workgroups one XCD runs together take a block of tiles, so its
-    // L2 serves each chunk of a few L and U panels to all of them (a
-    // row-major order would stream a different L panel per workgroup).  Ids
-    // past the last tile leave before the first barrier.
-    const int TR = (rn + kWB - 1) / kWB, TC = (rn + TN - 1) / TN;
-    const int nbi = (TR + C::kBlockRows - 1) / C::kBlockRows, nbj = (TC + C::kBlockCols - 1) / C::kBlockCols;
-    constexpr int per = C::kBlockRows * C::kBlockCols;
-    const int id = blockIdx.x, xcd = id % kXcds, local = id / kXcds;
-    const int blk = (local / per) * kXcds + xcd, slot = local % per;
-    const int tx = (blk % nbi) * C::kBlockRows + slot % C::kBlockRows;
-    const int ty = (blk / nbi) * C::kBlockCols + slot / C::kBlockRows;
-    if (blk >= nbi * nbj || tx >= TR || ty >= TC) return;
-    const int ri = tx * kWB, cj = ty * TN;  // packed row / column of the tile
+    const int rn = n - K1, cn = c1 - K1;
+    int tx, ty;
+    if (!xcd_tile((rn + kWB - 1) / kWB, (c1 - c0 + TN - 1) / TN, C::kStrip, tx, ty)) return;
+    const int ri = tx * kWB, cj = c0 - K1 + ty * TN;  // packed row / column of the tile
     const int rbase = K1 + ri, cbase = K1 + cj;
     const bool vec = (K1 % 4 == 0) && (lda % 4 == 0);
     const int nchunks = kwp / kHK;
@@ -1574,7 +1997,7 @@ __global__ void __launch_bounds__(256, WG) lu_gemm_f16w_kernel(float* A, int64_t
 #pragma unroll
     for (int q = 0; q < TN / 64; ++q) {
         const int r = wave * (TN / 4) + q * 16 + (lane >> 2);
-        bsrc[q] = Up + (size_t)min(cj + r, rn - 1) * kPackK + wide_seg(r, lane & 3) * 8;
+        bsrc[q] = Up + (size_t)min(cj + r, cn - 1) * kPackK + wide_seg(r, lane & 3) * 8;
     }
     auto issue = [&](int chunk, int st) {
         const int kc = chunk * kHK;
@@ -1598,7 +2021,7 @@ __global__ void __launch_bounds__(256, WG) lu_gemm_f16w_kernel(float* A, int64_t
         const int r = r0 + lr;
         return *reinterpret_cast<const h8*>(&ring[st][o * kWB * kHK + r * kHK + wide_seg(r, lg) * 8]);
     };
-    const bool interior = vec && rbase + kWB <= n && cbase + TN <= n;
+    const bool interior = vec && rbase + kWB <= n && cbase + TN <= c1;
     for (int ch = 0; ch < nchunks; ++ch) {
         __builtin_amdgcn_s_waitcnt(vm_wait((STAGES - 2) * C::kLoads));  // this wavefront's chunk ch has landed
         stage_barrier();  // ... and every wavefront's; stage (ch - 1) % STAGES has no readers left
@@ -1625,7 +2048,7 @@ __global__ void __launch_bounds__(256, WG) lu_gemm_f16w_kernel(float* A, int64_t
 #pragma unroll
     for (int j = 0; j < JB; ++j) {
         const int col = cbase + wc + 16 * j + lr;
-        inv[j] = (col < n) ? 1.f / colscale[col] : 0.f;
+        inv[j] = (col < c1) ? 1.f / colscale[col] : 0.f;
     }
     if (interior) {
         f4 c[JB][8];
@@ -1649,7 +2072,7 @@ __global__ void __launch_bounds__(256, WG) lu_gemm_f16w_kernel(float* A, int64_t
 #pragma unroll
     for (int j = 0; j < JB; ++j) {
         const int col = cbase + wc + 16 * j + lr;
-        if (col >= n) continue;
+        if (col >= c1) continue;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int row0 = rbase + wr + 16 * i + 4 * lg;
@@ -1661,23 +2084,19 @@ __global__ void __launch_bounds__(256, WG) lu_gemm_f16w_kernel(float* A, int64_t
     }
 }
 
-template <class Cfg, int TN, int STAGES, int WG>
-hipError_t launch_wide(float* A, int64_t lda, int n, int K1, int kwp, const _Float16* lpack, const _Float16* upack,
-                       const float* colscale, hipStream_t s)
+template <int TN, int STAGES, int WG>
+void launch_wide(float* A, int64_t lda, int n, int K1, int c0, int c1, int kwp, const _Float16* lpack,
+                 const _Float16* upack, const float* colscale, hipStream_t s)
 {
-    const int rem = n - K1;
-    const int TR = (rem + kWB - 1) / kWB, TC = (rem + TN - 1) / TN;
-    const int blocks = ((TR + Cfg::kBlockRows - 1) / Cfg::kBlockRows) * ((TC + Cfg::kBlockCols - 1) / Cfg::kBlockCols);
-    const int groups = (blocks + kXcds - 1) / kXcds * kXcds * Cfg::kBlockRows * Cfg::kBlockCols;
-    hipLaunchKernelGGL((lu_gemm_f16w_kernel<TN, STAGES, WG>), dim3(groups), dim3(256), 0, s, A, lda, n, K1, kwp, lpack,
-                       upack, colscale);
-    return hipGetLastError();
+    hipLaunchKernelGGL((lu_gemm_f16w_kernel<TN, STAGES, WG>),
+                       dim3(xcd_grid((n - K1 + kWB - 1) / kWB, (c1 - c0 + TN - 1) / TN)), dim3(256), 0, s, A, lda, n, K1,
+                       c0, c1, kwp, lpack, upack, colscale);
 }
 
 // Block-pivoted panel [k0, k1): diagonal block, then L21 below it; bak
 // receives the panel's original columns (rows [k0, n), leading dimension n).
 template <typename T>
-void block_panel(T* A, int64_t lda, int n, int k0, int k1, int* ipiv, int* info, T* bak, hipStream_t s)
+void block_panel(T* A, int64_t lda, int n, int k0, int k1, int* ipiv, int* info, T* bak, T* inv16, hipStream_t s)
 {
     const int nb = k1 - k0;
     const dim3 grid((n - k1 + 63) / 64);
@@ -1691,15 +2110,23 @@ void block_panel(T* A, int64_t lda, int n, int k0, int k1, int* ipiv, int* info,
             return;
         }
     }
-    // panels of at most 64 columns (all FP64 ones): four wavefronts
-    hipLaunchKernelGGL(lu_diag64_kernel<T>, dim3(1), dim3(256), 0, s, A, lda, k0, nb, ipiv, info, bak, (int64_t)n);
-    if (k1 < n)
+    // panels of at most 64 columns (all FP64 ones): eight wavefronts
+    hipLaunchKernelGGL(lu_diag64_kernel<T>, dim3(1), dim3(kDiag64Threads), 0, s, A, lda, k0, nb, ipiv, info, bak,
+                       (int64_t)n, inv16);
+    if (k1 >= n) return;
+    if (inv16)
+        hipLaunchKernelGGL(lu_l21_kernel64<T>, grid, dim3(256), 0, s, A, lda, n, k0, info, bak, (int64_t)n, inv16);
+    else
         hipLaunchKernelGGL((lu_l21_kernel<T, 64>), grid, dim3(256), 0, s, A, lda, n, k0, nb, info, bak, (int64_t)n);
 }
 
 constexpr size_t kWsScaleOffset = kColMaxBlocks * (sizeof(double) + sizeof(int)) + 64;
 size_t ws_backup_offset(int n) { return kWsScaleOffset + (sizeof(float) * (size_t)n + 255) / 256 * 256; }
-size_t ws_pack_offset(int n) { return ws_backup_offset(n) + (size_t)n * kMaxPanel * sizeof(float); }
+size_t ws_inv_offset(int n) { return ws_backup_offset(n) + (size_t)n * kMaxPanel * sizeof(float); }
+size_t ws_pack_offset(int n)
+{
+    return (ws_inv_offset(n) + ((size_t)n / 64 + 1) * kPanelInv * sizeof(double) + 255) / 256 * 256;
+}
 
 // Until *word == seq (a copy kernel stores it after its data at system
 // scope): spins up to a second, then waits for the stream and looks again.
@@ -1716,9 +2143,29 @@ static hipError_t wait_host_word(const unsigned* word, unsigned seq, hipStream_t
     return (__atomic_load_n(word, __ATOMIC_ACQUIRE) == seq) ? hipSuccess : hipErrorUnknown;
 }
 
+// 16-row tiles from which lu_cols_kernel gives a wavefront all 64 columns: a
+// wavefront for every SIMD
+constexpr int kColsWide = 1024;
+
+// Columns between the 64-column panels and the super-panels: inside such a
+// block the panels' columns and rows catch up one panel at a time, beyond it
+// with one update of K = 256.  Below 8192 rows the panels catch up over the
+// whole super-panel: those products are short and a launch saved counts more
+// (n = 1500: 2.19 against 2.24 ms of kernels); at n = 30000 they would read
+// 29 MB a panel and the rows' product over all columns takes 3 times as long.
+inline int mid_width(int n) { return n < 8192 ? (1 << 20) : 256; }
+// Trailing columns beyond the next super-panel from which they are updated on
+// the side stream while that super-panel is factorised: below, the update is
+// too short to hide anything.  With it the direct step at N=1000 went from 68.1
+// to 58.5 ms and the LU-preconditioned one at N=2000 (n = 30000) from 116 to 106
+// ms.  What is left of the overlap is lost where the chain's launches wait for a
+// tile of the update (55 us) to end: limiting the update's workgroups (448, 384,
+// 320 of 512) lost more than it gave.
+constexpr int kSideMin = 1024;
+
 template <typename T>
 hipError_t factor_impl(T* A, int64_t lda, int n, int nb, int* ipiv, int* info, int use_mfma, int block_pivot,
-                       int update_fp16, void* ws, int* redone, int* host_flag, hipStream_t s)
+                       int update_fp16, void* ws, int* redone, int* host_flag, hipStream_t s, const LuSide* side)
 {
     double* pval = static_cast<double*>(ws);
     int* pidx = reinterpret_cast<int*>(pval + kColMaxBlocks);
@@ -1729,7 +2176,7 @@ hipError_t factor_impl(T* A, int64_t lda, int n, int nb, int* ipiv, int* info, i
     _Float16* lpack = reinterpret_cast<_Float16*>(static_cast<char*>(ws) + ws_pack_offset(n));
     _Float16* upack = lpack + (size_t)n * kPackK;
     if (redone) *redone = 0;
-    auto gemm = [&](GemmRange g) {
+    auto gemm = [&](hipStream_t q, GemmRange g) {
         if (g.r1 <= g.r0 || g.c1 <= g.c0 || g.kb <= g.ka) return;
         const int rows = g.r1 - g.r0, cols = g.c1 - g.c0;
         if (f16) {
@@ -1738,87 +2185,199 @@ hipError_t factor_impl(T* A, int64_t lda, int n, int nb, int* ipiv, int* info, i
                 // take 64 x 64 tiles (same products per element)
                 if (rows <= 64 || cols <= 64)
                     hipLaunchKernelGGL((lu_gemm_f16_kernel<64, 64>), dim3((rows + 63) / 64, (cols + 63) / 64),
-                                       dim3(256), 0, s, A, lda, g, colscale);
+                                       dim3(256), 0, q, A, lda, g, colscale);
                 else
                     hipLaunchKernelGGL((lu_gemm_f16_kernel<kHB, kHB>), dim3((rows + kHB - 1) / kHB, (cols + kHB - 1) / kHB),
-                                       dim3(256), 0, s, A, lda, g, colscale);
+                                       dim3(256), 0, q, A, lda, g, colscale);
             }
         } else if (use_mfma) {
             if constexpr (sizeof(T) == 8) {
                 if (f64w_fits(g, lda)) {
-                    launch_f64w(A, lda, g, s);
+                    launch_f64w(A, lda, g, q);
                     return;
                 }
             }
             const int bn = gemm_bn<T>();
-            // FP64 takes 64-row tiles everywhere (three workgroups per CU
-            // instead of two: 85.7 against 91 ms for n = 15000); FP32 the
-            // narrow updates (a panel's columns or rows): twice the
-            // workgroups for the columns, no empty half for the rows
+            // FP64 takes 64-row tiles (three workgroups per CU instead of
+            // two: 85.7 against 91 ms for n = 15000); FP32 the narrow updates
+            // (a panel's columns or rows): twice the workgroups for the
+            // columns, no empty half for the rows
             if (sizeof(T) == 8 || rows <= kBMNarrow || cols <= bn)
                 hipLaunchKernelGGL((lu_gemm_mfma_kernel<T, kBMNarrow>),
-                                   dim3((rows + kBMNarrow - 1) / kBMNarrow, (cols + bn - 1) / bn), dim3(256), 0, s, A,
+                                   dim3((rows + kBMNarrow - 1) / kBMNarrow, (cols + bn - 1) / bn), dim3(256), 0, q, A,
                                    lda, g);
             else
                 hipLaunchKernelGGL((lu_gemm_mfma_kernel<T, kBM>), dim3((rows + kBM - 1) / kBM, (cols + bn - 1) / bn),
-                                   dim3(256), 0, s, A, lda, g);
+                                   dim3(256), 0, q, A, lda, g);
         } else {
             hipLaunchKernelGGL(lu_gemm_valu_kernel<T>, dim3((rows + kTile - 1) / kTile, (cols + kTile - 1) / kTile),
-                               dim3(256), 0, s, A, lda, g);
+                               dim3(256), 0, q, A, lda, g);
         }
     };
-    // Super-panels of two panels: inside one, each panel's columns and rows
-    // catch up with the earlier panel (narrow updates), and the trailing
-    // matrix takes one update with K = 2 nb per super-panel, which halves its
-    // read-modify-write traffic.
+    // [k0, k1): the block-pivoted panel and its check, or (when that fails, or
+    // without block pivoting) the column-by-column one
+    auto panel = [&](int k0, int k1, T* inv16) -> hipError_t {
+        bool columns = !block_pivot;
+        if (block_pivot) {
+            block_panel<T>(A, lda, n, k0, k1, ipiv, info, bak, inv16, s);
+            // the check decides before anything else reads the panel
+            int flag = 0;
+            hipError_t e;
+            if (host_flag) {  // own copy kernel: the runtime's device-to-host copy stalls the queue
+                // it ends with a sequence word in host_flag[1]: spin on that
+                // rather than sleep in a stream synchronisation
+                unsigned* seq_word = reinterpret_cast<unsigned*>(host_flag + 1);
+                const unsigned seq = __atomic_load_n(seq_word, __ATOMIC_ACQUIRE) + 1u;
+                e = launch_to_host(info + 1, host_flag, sizeof(int), s, seq_word, seq);
+                if (e == hipSuccess) e = wait_host_word(seq_word, seq, s);
+                flag = __atomic_load_n(host_flag, __ATOMIC_ACQUIRE);
+            } else {
+                e = hipMemcpyAsync(&flag, info + 1, sizeof(int), hipMemcpyDeviceToHost, s);
+                if (e == hipSuccess) e = hipStreamSynchronize(s);
+            }
+            if (e != hipSuccess) return e;
+            if (flag) {
+                hipLaunchKernelGGL(lu_restore_kernel<T>, dim3((n - k0 + 255) / 256, k1 - k0), dim3(256), 0, s, A,
+                                   lda, n, k0, k1 - k0, bak, (int64_t)n);
+                e = hipMemsetAsync(info + 1, 0, sizeof(int), s);
+                if (e != hipSuccess) return e;
+                columns = true;
+                if (redone) *redone += 1;
+            }
+        }
+        for (int j = k0; j < k1 && columns; ++j) {
+            const int rows = n - j;
+            const int blocks = std::max(1, std::min(kColMaxBlocks, (rows + kColThreads - 1) / kColThreads));
+            hipLaunchKernelGGL(lu_crout_kernel<T>, dim3(blocks), dim3(kColThreads), 0, s, A, lda, n, k0, k1, j,
+                               ipiv, info, pval, pidx, counter);
+        }
+        if (k1 < n && columns) {
+            hipLaunchKernelGGL(lu_scale_kernel<T>, dim3((n - k1 + 255) / 256), dim3(256), 0, s, A, lda, n, k1 - 1);
+            if (inv16) hipLaunchKernelGGL(lu_inv16_kernel<T>, dim3(1), dim3(128), 0, s, A, lda, k0, inv16);
+        }
+        return hipGetLastError();
+    };
+    // the trailing columns [c0, c1) (rows [K1, n)) after the super-panel
+    // [K0, K1), whose L the fp16 update finds packed (pack_l)
+    auto pack_l = [&](hipStream_t q, int K0, int K1) {
+        if constexpr (sizeof(T) == 4) {
+            const int rem = n - K1, kwp = (K1 - K0 + kHK - 1) / kHK * kHK;
+            if (f16)
+                hipLaunchKernelGGL(pack_l_kernel, dim3((rem + 63) / 64, (kwp + 63) / 64), dim3(256), 0, q, A, lda, n, K0,
+                                   K1, kwp, lpack);
+        }
+    };
+    auto update = [&](hipStream_t q, int K0, int K1, int c0, int c1) {
+        if (!f16) {
+            gemm(q, {K1, n, c0, c1, K0, K1});
+            return;
+        }
+        if constexpr (sizeof(T) == 4) {  // from packed fp16 operands
+            const int rem = n - K1, kwp = (K1 - K0 + kHK - 1) / kHK * kHK;
+            const int64_t units = (int64_t)(c1 - c0) * (kwp / 8);
+            hipLaunchKernelGGL(pack_u_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, q, A, lda, c0, c1, K0,
+                               K1, kwp, colscale, upack);
+            if (rem >= kWideMin)  // 256 x 128 tiles, two workgroups per CU, in XCD-local blocks
+                launch_wide<128, 3, 2>(A, lda, n, K1, c0, c1, kwp, lpack, upack, colscale, q);
+            else
+                hipLaunchKernelGGL(lu_gemm_f16p_kernel, dim3((rem + kHB - 1) / kHB, (c1 - c0 + kHB - 1) / kHB), dim3(256),
+                                   0, q, A, lda, n, K1, c0, c1, kwp, lpack, upack, colscale);
+        }
+    };
     const int sb = std::max(1, super_width<T>() / nb) * nb;
+    hipError_t e;
+    if (nb == 64 && use_mfma) {
+        T* inv = reinterpret_cast<T*>(static_cast<char*>(ws) + ws_inv_offset(n));
+        const int mid = std::min(sb, mid_width(n));
+        auto swaps = [&](hipStream_t q, int ka, int kb, int c0, int c1) {
+            if (c1 > c0)
+                hipLaunchKernelGGL(lu_swap_kernel<T>, dim3((c1 - c0 + 63) / 64), dim3(64), 0, q, A, lda, ka, kb, ipiv, c0,
+                                   c1);
+        };
+        auto rows = [&](hipStream_t q, int B0, int ka, int kb, int c0, int c1, bool swap, float* scale, int combine) {
+            if (c1 > c0)
+                hipLaunchKernelGGL(lu_rows_kernel<T>, dim3((c1 - c0 + 15) / 16), dim3(256), 0, q, A, lda,
+                                   swap ? ipiv : nullptr, inv, B0, ka, kb, c0, c1, scale, combine);
+        };
+        // the super-panel's own columns, on the main stream
+        auto factor = [&](int K0, int K1) -> hipError_t {
+            for (int B0 = K0; B0 < K1; B0 += mid) {
+                const int B1 = std::min(K1, B0 + mid);
+                for (int k0 = B0; k0 < B1; k0 += 64) {
+                    const int k1 = std::min(B1, k0 + 64), tiles = (n - k0 + 15) / 16;
+                    if (k0 > B0) {
+                        if (tiles >= kColsWide)
+                            hipLaunchKernelGGL((lu_cols_kernel<T, 4>), dim3((tiles + 3) / 4), dim3(256), 0, s, A, lda, n,
+                                               B0, k0, k1 - k0);
+                        else
+                            hipLaunchKernelGGL((lu_cols_kernel<T, 1>), dim3(tiles), dim3(256), 0, s, A, lda, n, B0, k0,
+                                               k1 - k0);
+                    }
+                    T* pinv = (k1 < n) ? inv + (size_t)(k0 / 64) * kPanelInv : nullptr;
+                    if ((e = panel(k0, k1, pinv)) != hipSuccess) return e;
+                    swaps(s, k0, k1, K0, k0);  // the rows of L that the next launches read
+                    rows(s, B0, k0, k1, k1, B1, true, nullptr, 0);
+                }
+                rows(s, B0, B0, B1, B1, K1, true, colscale, 0);
+                gemm(s, {B1, n, B1, K1, B0, B1});
+            }
+            return hipGetLastError();
+        };
+        // [K0, K1)'s swaps, rows and update on trailing columns
+        auto trailing = [&](hipStream_t q, int K0, int K1, int c0, int c1) {
+            swaps(q, K0, K1, c0, c1);
+            for (int B0 = K0; B0 < K1; B0 += mid) {
+                const int B1 = std::min(K1, B0 + mid);
+                rows(q, B0, B0, B1, c0, c1, false, colscale, B0 > K0);
+                gemm(q, {B1, K1, c0, c1, B0, B1});
+            }
+            update(q, K0, K1, c0, c1);
+        };
+        // While a super-panel is factorised (a chain of small launches on the
+        // main stream), the side stream brings the columns beyond it up to
+        // date with the previous one; the main stream takes the next
+        // super-panel's own columns out of that update first.
+        bool pending = false;  // side work the main stream has not waited for
+        if ((e = factor(0, std::min(n, sb))) != hipSuccess) return e;
+        for (int K0 = 0; K0 < n; K0 += sb) {
+            const int K1 = std::min(n, K0 + sb), K2 = std::min(n, K1 + sb);
+            if (pending) {
+                if ((e = hipStreamWaitEvent(s, side->side_done, 0)) != hipSuccess) return e;
+                pending = false;
+            }
+            if (K1 < n) pack_l(s, K0, K1);
+            if (side && n - K2 >= kSideMin) {
+                if ((e = hipEventRecord(side->main_done, s)) != hipSuccess) return e;
+                if ((e = hipStreamWaitEvent(side->stream, side->main_done, 0)) != hipSuccess) return e;
+                swaps(side->stream, K0, K1, 0, K0);
+                trailing(side->stream, K0, K1, K2, n);
+                if ((e = hipEventRecord(side->side_done, side->stream)) != hipSuccess) return e;
+                pending = true;
+                trailing(s, K0, K1, K1, K2);
+            } else {
+                swaps(s, K0, K1, 0, K0);
+                if (K1 < n) trailing(s, K0, K1, K1, n);
+            }
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+            if (K1 < n && (e = factor(K1, K2)) != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
+    // Other panel widths.  Inside a super-panel each panel's columns and rows
+    // catch up with the earlier panels (narrow updates), and the trailing
+    // matrix takes one update per super-panel.
     for (int K0 = 0; K0 < n; K0 += sb) {
         const int K1 = std::min(n, K0 + sb);
         for (int k0 = K0; k0 < K1; k0 += nb) {
             const int k1 = std::min(K1, k0 + nb);
-            gemm({k0, n, k0, k1, K0, k0});  // the panel's columns
-            bool columns = !block_pivot;
-            if (block_pivot) {
-                block_panel<T>(A, lda, n, k0, k1, ipiv, info, bak, s);
-                // the check decides before anything else reads the panel
-                int flag = 0;
-                hipError_t e;
-                if (host_flag) {  // own copy kernel: the runtime's device-to-host copy stalls the queue
-                    // it ends with a sequence word in host_flag[1]: spin on that
-                    // rather than sleep in a stream synchronisation
-                    unsigned* seq_word = reinterpret_cast<unsigned*>(host_flag + 1);
-                    const unsigned seq = __atomic_load_n(seq_word, __ATOMIC_ACQUIRE) + 1u;
-                    e = launch_to_host(info + 1, host_flag, sizeof(int), s, seq_word, seq);
-                    if (e == hipSuccess) e = wait_host_word(seq_word, seq, s);
-                    flag = __atomic_load_n(host_flag, __ATOMIC_ACQUIRE);
-                } else {
-                    e = hipMemcpyAsync(&flag, info + 1, sizeof(int), hipMemcpyDeviceToHost, s);
-                    if (e == hipSuccess) e = hipStreamSynchronize(s);
-                }
-                if (e != hipSuccess) return e;
-                if (flag) {
-                    hipLaunchKernelGGL(lu_restore_kernel<T>, dim3((n - k0 + 255) / 256, k1 - k0), dim3(256), 0, s, A,
-                                       lda, n, k0, k1 - k0, bak, (int64_t)n);
-                    e = hipMemsetAsync(info + 1, 0, sizeof(int), s);
-                    if (e != hipSuccess) return e;
-                    columns = true;
-                    if (redone) *redone += 1;
-                }
-            }
-            for (int j = k0; j < k1 && columns; ++j) {
-                const int rows = n - j;
-                const int blocks = std::max(1, std::min(kColMaxBlocks, (rows + kColThreads - 1) / kColThreads));
-                hipLaunchKernelGGL(lu_crout_kernel<T>, dim3(blocks), dim3(kColThreads), 0, s, A, lda, n, k0, k1, j,
-                                   ipiv, info, pval, pidx, counter);
-            }
-            if (k1 < n && columns)
-                hipLaunchKernelGGL(lu_scale_kernel<T>, dim3((n - k1 + 255) / 256), dim3(256), 0, s, A, lda, n, k1 - 1);
+            gemm(s, {k0, n, k0, k1, K0, k0});  // the panel's columns
+            if ((e = panel(k0, k1, nullptr)) != hipSuccess) return e;
             const int outside = n - (k1 - k0);
             if (outside > 0)
                 hipLaunchKernelGGL(lu_laswp_kernel<T>, dim3((outside + 255) / 256), dim3(256), 0, s, A, lda, n, k0,
                                    k1, ipiv);
             if (k1 < n) {
-                gemm({k0, k1, k1, n, K0, k0});  // the panel's rows right of it
+                gemm(s, {k0, k1, k1, n, K0, k0});  // the panel's rows right of it
                 const dim3 ugrid((n - k1 + 63) / 64);
                 const int combine = (k0 > K0) ? 1 : 0;
                 bool wide = false;
@@ -1833,31 +2392,13 @@ hipError_t factor_impl(T* A, int64_t lda, int n, int nb, int* ipiv, int* info, i
                     hipLaunchKernelGGL((lu_u12_kernel<T, 64>), ugrid, dim3(256), 0, s, A, lda, n, k0, k1 - k0, colscale,
                                        combine);
             }
-            hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
+            if ((e = hipGetLastError()) != hipSuccess) return e;
         }
-        if (f16 && K1 < n) {  // the trailing matrix from packed fp16 operands
-            if constexpr (sizeof(T) == 4) {
-                const int rem = n - K1, kwp = (K1 - K0 + kHK - 1) / kHK * kHK;
-                hipLaunchKernelGGL(pack_l_kernel, dim3((rem + 63) / 64, (kwp + 63) / 64), dim3(256), 0, s, A, lda, n,
-                                   K0, K1, kwp, lpack);
-                const int64_t units = (int64_t)rem * (kwp / 8);
-                hipLaunchKernelGGL(pack_u_kernel, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s, A, lda, n,
-                                   K0, K1, kwp, colscale, upack);
-                if (rem >= kWideMin) {  // 256 x 128 tiles, two workgroups per CU, in XCD-local blocks
-                    const hipError_t e = launch_wide<WideTwo, 128, 3, 2>(A, lda, n, K1, kwp, lpack, upack, colscale, s);
-                    if (e != hipSuccess) return e;
-                } else {
-                    const int tiles = (rem + kHB - 1) / kHB;
-                    hipLaunchKernelGGL(lu_gemm_f16p_kernel, dim3(tiles, tiles), dim3(256), 0, s, A, lda, n, K1, kwp,
-                                       lpack, upack, colscale);
-                }
-            }
-        } else {
-            gemm({K1, n, K1, n, K0, K1});  // the trailing matrix
+        if (K1 < n) {
+            pack_l(s, K0, K1);
+            update(s, K0, K1, K1, n);
         }
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
+        if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     return hipSuccess;
 }
@@ -2204,14 +2745,18 @@ size_t lu_workspace_bytes(int n, int update_fp16)
 }
 
 hipError_t lu_factor(void* A, int elem_bytes, int64_t lda, int n, int nb, int* ipiv, int* info, int use_mfma,
-                     int block_pivot, int update_fp16, void* ws, int* redone, int* host_flag, hipStream_t s)
+                     int block_pivot, int update_fp16, void* ws, int* redone, int* host_flag, hipStream_t s,
+                     const LuSide* side)
 {
     if (nb < 1 || nb > (elem_bytes == 4 ? kMaxPanel : 64) || !ws || lda % 4 != 0) return hipErrorInvalidValue;
-    if (elem_bytes == 8)
-        return factor_impl<double>(static_cast<double*>(A), lda, n, nb, ipiv, info, use_mfma, block_pivot, 0, ws,
-                                   redone, host_flag, s);
-    return factor_impl<float>(static_cast<float*>(A), lda, n, nb, ipiv, info, use_mfma, block_pivot, update_fp16, ws,
-                              redone, host_flag, s);
+    const hipError_t e =
+        (elem_bytes == 8) ? factor_impl<double>(static_cast<double*>(A), lda, n, nb, ipiv, info, use_mfma, block_pivot,
+                                                0, ws, redone, host_flag, s, side)
+                          : factor_impl<float>(static_cast<float*>(A), lda, n, nb, ipiv, info, use_mfma, block_pivot,
+                                               update_fp16, ws, redone, host_flag, s, side);
+    // after an error s may not have waited for the side stream
+    if (e != hipSuccess && side) (void)hipStreamSynchronize(side->stream);
+    return e;
 }
 
 static size_t perm_bytes(int n) { return ((sizeof(int) * (size_t)n + 255) / 256) * 256; }

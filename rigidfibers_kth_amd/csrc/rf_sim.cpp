@@ -107,6 +107,10 @@ struct PhaseTimer {
 
 rf_sim::~rf_sim()
 {
+    if (lu_side.stream) {
+        (void)hipStreamSynchronize(lu_side.stream);
+        (void)hipStreamDestroy(lu_side.stream);
+    }
     for (void* q : allocs) (void)hipFree(q);
     if (h_dots) (void)hipHostFree(h_dots);
     if (h_y) (void)hipHostFree(h_y);
@@ -541,6 +545,11 @@ int rf_sim::factorize(bool* done, bool precond_only)
         d_info = d_ipiv + n;
         d_lu_ws = static_cast<char*>(q) + piv_bytes;
         HIP_TRY(hipMemsetAsync(d_lu_ws, 0, lu_workspace_bytes(n, ws_fp16), stream));
+        HIP_TRY(hipStreamCreateWithFlags(&lu_side.stream, hipStreamNonBlocking));
+        for (hipEvent_t* ev : {&lu_side.main_done, &lu_side.side_done}) {
+            HIP_TRY(hipEventCreateWithFlags(ev, hipEventDisableTiming));
+            events.push_back(*ev);
+        }
     }
     // panel width 64 (one wavefront factorises the diagonal block); FP32
     // factors accept up to 128
@@ -563,7 +572,7 @@ int rf_sim::factorize(bool* done, bool precond_only)
     lu_have = false;
     int redone = 0;
     HIP_TRY(lu_factor(d_LU, es, lda, n, nb, d_ipiv, d_info, p.lu_valu_update ? 0 : 1, p.lu_column_panel ? 0 : 1,
-                      fp16 ? 1 : 0, d_lu_ws, &redone, reinterpret_cast<int*>(h_dots), stream));
+                      fp16 ? 1 : 0, d_lu_ws, &redone, reinterpret_cast<int*>(h_dots), stream, &lu_side));
     stats.lu_panel_fallbacks += redone;
     HIP_TRY(hipMemcpyAsync(h_dots, d_info, 2 * sizeof(int), hipMemcpyDeviceToHost, stream));
     if (p.profile) {
@@ -1913,10 +1922,22 @@ extern "C" int rf_selftest_lu(int32_t n, int32_t elem_bytes, int32_t nb, int32_t
     if (e == hipSuccess) e = hipMemset(dW, 0, lu_workspace_bytes(n, update_fp16));
     int* d_ipiv = static_cast<int*>(dP);
     int redone = 0;
+    // as a handle's: a stream of its own and a side stream
+    hipStream_t main_stream = nullptr;
+    LuSide side;
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&main_stream, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&side.stream, hipStreamNonBlocking);
+    for (hipEvent_t* ev : {&side.main_done, &side.side_done})
+        if (e == hipSuccess) e = hipEventCreateWithFlags(ev, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipDeviceSynchronize();  // the copies above are on the null stream
     if (e == hipSuccess)
         e = lu_factor(dA, elem_bytes, lda, n, nb, d_ipiv, d_ipiv + n, valu ? 0 : 1, column_panel ? 0 : 1,
-                      update_fp16, dW, &redone, nullptr, nullptr);
+                      update_fp16, dW, &redone, nullptr, main_stream, &side);
     if (e == hipSuccess) e = hipDeviceSynchronize();
+    for (hipEvent_t ev : {side.main_done, side.side_done})
+        if (ev) (void)hipEventDestroy(ev);
+    for (hipStream_t q : {side.stream, main_stream})
+        if (q) (void)hipStreamDestroy(q);
     std::vector<int> piv((size_t)n + 2);
     if (e == hipSuccess) e = hipMemcpy(piv.data(), dP, sizeof(int) * ((size_t)n + 2), hipMemcpyDeviceToHost);
     if (e == hipSuccess) e = hipMemcpy(host.data(), dA, host.size(), hipMemcpyDeviceToHost);

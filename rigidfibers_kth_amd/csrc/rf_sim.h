@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "rf_internal.h"
+#include "rf_lu.h"
 #include "rf_mlp.h"
 
 struct rf_sim {
@@ -108,6 +109,7 @@ struct rf_sim {
     int* d_ipiv = nullptr;
     int* d_info = nullptr;
     void* d_lu_ws = nullptr;   // pivot-search partials and counter
+    rf::LuSide lu_side;        // stream and events of the overlapped trailing updates
     void* d_lu_aux = nullptr;  // FP32 factors: permutation and diagonal-block inverses
     double* d_lu_tmp = nullptr;
     bool lu_factored = false;  // d_LU holds the factors of the current matrix

@@ -56,3 +56,34 @@ def test_fp32_factor_solve_at_block_edges(N, terms, mixed):
     ref = np.linalg.solve(A, r)
     assert np.array_equal(z, again)
     assert np.linalg.norm(z - ref) <= 1e-5 * np.linalg.norm(ref)
+
+
+# With more than 1024 columns beyond the next super-panel (512 columns in FP64,
+# 1024 in FP32) their update runs on the side stream beside the factorisation
+# of that super-panel: 2048 + 512, FP32 from 3072 + 1024 on, with whole and ragged ends, panels
+# redone column by column in between, and the fp16 update's tiles.
+@pytest.mark.parametrize("n,es,fp16", [(2049, 8, 0), (3100, 8, 0), (3073, 4, 0), (4300, 4, 0), (4611, 4, 1),
+                                       (6200, 4, 1)])
+def test_overlapped_updates_give_partial_pivoting(n, es, fp16):
+    A = _dominant_with_block_swaps(n, 64, n + 1)
+    if es == 4:
+        A = A.astype(np.float32).astype(np.float64)
+    lu_ref, piv_ref = sl.lu_factor(A)
+    LU, ipiv, info, fb = rf.selftest_lu(A, es, 0, update_fp16=fp16)
+    again, _, _, _ = rf.selftest_lu(A, es, 0, update_fp16=fp16)
+    assert info == 0 and fb == 0
+    np.testing.assert_array_equal(ipiv, piv_ref)
+    np.testing.assert_array_equal(LU, again)
+    # FP64 and FP32 rounding of sums over n of a diagonally dominant matrix; fp16 operands
+    tol = 1e-12 if es == 8 else (2e-3 if fp16 else 1e-5)
+    assert np.abs(LU - lu_ref).max() <= tol * np.abs(lu_ref).max()
+
+
+def test_overlapped_updates_with_redone_panels():
+    n = 3200
+    A = _random(n, 29)
+    lu_ref, piv_ref = sl.lu_factor(A)
+    LU, ipiv, info, fb = rf.selftest_lu(A, 8, 0)
+    assert info == 0 and fb == (n - 1) // 64
+    np.testing.assert_array_equal(ipiv, piv_ref)
+    assert np.abs(LU - lu_ref).max() <= 1e-10 * np.abs(lu_ref).max()
