@@ -39,13 +39,15 @@ __device__ __forceinline__ int sym6(int a, int b)
 // recurrences of the near field (c < 10) are FP64; RB is the arithmetic type
 // of the 26-step backward recurrences of the far field (double, or float in
 // mixed precision, whose error is then ~FP32 rounding of the moments).
+// BRANCH: the recurrences by c (kByDistance), or those the caller knows to apply.
+enum MomentBranch { kByDistance, kForward, kBackward };
 template <int M>
 struct Moments {
     double r0x, r0y, r0z, px, py, pz;
     double I[M + 3], J[M + 3], S[M + 3];
 };
 
-template <int M, typename RB>
+template <int M, typename RB, MomentBranch BRANCH = kByDistance>
 __device__ __forceinline__ void analytic_moments(double X0, double X1, double X2, const double* xj, const double* tj,
                                                  Moments<M>& mo)
 {
@@ -79,7 +81,7 @@ __device__ __forceinline__ void analytic_moments(double X0, double X1, double X2
         S[0] = ((2.0 + b) * iue3 - (-2.0 + b) * iub3) * i6d + ((2.0 / 3.0) * id) * J[0];
         S[1] = (-(b + 2.0 * c) * iue3 + (2.0 * c - b) * iub3) * i6d - (b * id * (1.0 / 3.0)) * J[0];
     }
-    if (c < 10.0) {
+    if (BRANCH == kForward || (BRANCH == kByDistance && c < 10.0)) {
         // forward recurrences (Int_analytical.f90:123-136,172-176,197-200)
 #pragma unroll
         for (int n = 2; n < NM; ++n) {

@@ -25,7 +25,24 @@ struct Tables {
     double wv[kMaxQuad] = {0};  // weights
     // wp[k*LQ + p] = w_p * P_k(s_p), k = 0..M (P_0 = 1)
     double wp[(kMaxTerms + 1) * kMaxQuad] = {0};
+    // Far pairs of the analytic operator (rf_operator.hip): for each distance
+    // class the outer nodes and their weights W[k][node] (which reproduce the
+    // composite rule's sums w_p P_k on the interpolant through the nodes), and
+    // the inner Gauss nodes with w_q P_l(s_q); offsets into far[].
+    struct FarClass {
+        int n = 0, q = 0;  // outer and inner nodes
+        int node = 0, W = 0, sq = 0, wP = 0;
+        double dist2 = 0.0;  // from this centre distance squared on
+    };
+    static constexpr int kFarClasses = 3;
+    FarClass fc[kFarClasses];
+    double point_c = 0.0;  // least |R|^2 of a single point for the inner nodes of class 0
+    int far_total = 0;
+    double far[704] = {0};
 };
+
+// Inner Gauss nodes of the far classes by M, and their centre distances.
+constexpr int far_inner_nodes(int M, int c) { return c == 0 ? 11 : M <= 5 ? 10 - c : 10; }
 
 void build_tables(int M, int noqi, double eps, Tables* t);
 
@@ -63,13 +80,15 @@ enum { kOpAx = 0, kOpResidual = 1, kOpRhs = 2, kOpVelocity = 3 };
 struct OperatorPlan {
     int N = 0, M = 0, LQ = 0, analytic = 1;
     int T = 1, threads = 64, splits = 1, src_per_split = 1, src_stride = 4;
+    int far = 0;  // analytic: far pairs by quadrature (needs the far source vectors and tables)
 };
-OperatorPlan plan_operator(int N, int M, int LQ, int analytic, int num_cus);
+// far = 0: every analytic pair through the moments (less scratch)
+OperatorPlan plan_operator(int N, int M, int LQ, int analytic, int num_cus, int far = 1);
 // doubles of device scratch one launch needs (source vectors + split partials)
 size_t operator_scratch_doubles(const OperatorPlan& p);
 hipError_t launch_operator(const OperatorPlan& p, const Tables& t, int mode, const double* pos, const double* orient,
-                           const double* force, const double* x, const double* wp, const double* pv, double* scratch,
-                           double* y, hipStream_t s);
+                           const double* force, const double* x, const double* wp, const double* pv, const double* far,
+                           double* scratch, double* y, hipStream_t s);
 // The output map of `mode` alone, from the split partials the last
 // launch_operator left in `scratch`: every mode's kernel forms all IF_k
 // (k = 0..M), so the velocity sums (mode kOpVelocity) of an evaluation whose

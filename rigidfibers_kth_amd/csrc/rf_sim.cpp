@@ -26,6 +26,114 @@ void set_error(const std::string& msg) { g_error = msg; }
 
 int assemble_targets_per_block(int LQ, int M, bool analytic);
 
+namespace {
+
+// P_0..P_M at x
+void legendre_values(int M, double x, double* P)
+{
+    P[0] = 1.0;
+    if (M >= 1) P[1] = x;
+    for (int k = 1; k < M; ++k) P[k + 1] = ((2.0 * k + 1.0) * x * P[k] - k * P[k - 1]) / (k + 1.0);
+}
+
+// n-point Gauss-Legendre rule: Newton's iteration on P_n from the Chebyshev guess
+constexpr int kMaxGauss = 16;
+struct GaussRule {
+    double x[kMaxGauss], w[kMaxGauss];
+};
+GaussRule gauss_rule(int n)
+{
+    GaussRule r{};
+    for (int i = 0; i < n; ++i) {
+        long double x = std::cos(3.14159265358979323846L * (n - i - 0.25L) / (n + 0.5L)), d = 1.0L;
+        for (int it = 0; it < 8; ++it) {
+            long double p0 = 1.0L, p1 = x;
+            for (int k = 1; k < n; ++k) {
+                const long double p2 = ((2 * k + 1) * x * p1 - k * p0) / (k + 1);
+                p0 = p1;
+                p1 = p2;
+            }
+            d = n * (x * p1 - p0) / (x * x - 1.0L);
+            x -= p1 / d;
+        }
+        r.x[i] = (double)x;
+        r.w[i] = (double)(2.0L / ((1.0L - x * x) * d * d));
+    }
+    return r;
+}
+
+// Distance classes of the far pairs (see Tables): from centre distance dist on,
+// n outer nodes and far_inner_nodes(M, c) inner nodes reproduce the composite
+// outer rule and the exact inner integrals to about 1e-13 of the largest entry
+// (worst orientations; measured for M = 5 and 8: 2e-13 at 4.2, 1e-13 at 5.5 and
+// 8).  The reference's own far recurrences, started at n = 27, are off by 4e-11
+// at M = 5 and 6e-9 at M = 8 where they set in (|R|^2 = 10); for M > 5 the first
+// class starts where they are as good as the quadrature.
+void build_far_tables(Tables* t)
+{
+    static const std::vector<GaussRule> rules = [] {
+        std::vector<GaussRule> r(kMaxGauss);
+        for (int n = 1; n < kMaxGauss; ++n) r[n] = gauss_rule(n);
+        return r;
+    }();
+    const double dist[2][Tables::kFarClasses] = {{4.2, 5.5, 8.0}, {5.2, 6.0, 8.0}};
+    const int outer[Tables::kFarClasses] = {14, 12, 10};
+    const int M = t->M;
+    int off = 0;
+    for (int c = 0; c < Tables::kFarClasses; ++c) {
+        Tables::FarClass& f = t->fc[c];
+        f.dist2 = dist[M <= 5 ? 0 : 1][c] * dist[M <= 5 ? 0 : 1][c];
+        f.n = std::min(outer[c], t->LQ);
+        f.q = far_inner_nodes(M, c);
+        f.node = off;
+        f.W = f.node + f.n;
+        f.sq = f.W + (M + 1) * f.n;
+        f.wP = f.sq + f.q;
+        off = f.wP + (M + 1) * f.q;
+        double P[kMaxTerms + 1];
+        if (f.n == t->LQ) {  // no fewer nodes than points: the points themselves
+            for (int p = 0; p < f.n; ++p) t->far[f.node + p] = t->pv[p];
+            for (int k = 0; k <= M; ++k)
+                for (int p = 0; p < f.n; ++p) t->far[f.W + k * f.n + p] = t->wp[k * t->LQ + p];
+        } else {
+            // W[k][a] = sum_p w_p P_k(s_p) L_a(s_p), L_a the Lagrange
+            // polynomials of the Gauss nodes in barycentric form
+            const GaussRule& g = rules[f.n];
+            double bw[kMaxGauss];
+            for (int a = 0; a < f.n; ++a) {
+                t->far[f.node + a] = g.x[a];
+                bw[a] = ((a & 1) ? -1.0 : 1.0) * std::sqrt((1.0 - g.x[a] * g.x[a]) * g.w[a]);
+                for (int k = 0; k <= M; ++k) t->far[f.W + k * f.n + a] = 0.0;
+            }
+            for (int p = 0; p < t->LQ; ++p) {
+                double la[kMaxGauss], sum = 0.0;
+                int hit = -1;
+                for (int a = 0; a < f.n; ++a) {
+                    const double dx = t->pv[p] - g.x[a];
+                    if (std::fabs(dx) < 1e-14) hit = a;
+                    la[a] = bw[a] / dx;
+                    sum += la[a];
+                }
+                for (int a = 0; a < f.n; ++a) {
+                    const double L = hit >= 0 ? (a == hit ? 1.0 : 0.0) : la[a] / sum;
+                    for (int k = 0; k <= M; ++k) t->far[f.W + k * f.n + a] += t->wp[k * t->LQ + p] * L;
+                }
+            }
+        }
+        const GaussRule& g = rules[f.q];
+        for (int q = 0; q < f.q; ++q) {
+            t->far[f.sq + q] = g.x[q];
+            legendre_values(M, g.x[q], P);
+            for (int l = 0; l <= M; ++l) t->far[f.wP + l * f.q + q] = g.w[q] * P[l];
+        }
+    }
+    // 11 inner nodes at a single point: 2e-14 from |R|^2 = 10 on for M <= 5, 7e-14 from 17 on for M = 8
+    t->point_c = (M <= 5) ? 10.0 : 17.0;
+    t->far_total = off;
+}
+
+}  // namespace
+
 // fortran/quadrature.f90:6-96, fortran/matrix_assembly.f90:8-57,294-305,370
 void build_tables(int M, int noqi, double eps, Tables* t)
 {
@@ -66,6 +174,7 @@ void build_tables(int M, int noqi, double eps, Tables* t)
             t->wp[(k + 1) * t->LQ + p] = t->wv[p] * Pk;
         }
     }
+    build_far_tables(t);
 }
 
 }  // namespace rf
@@ -146,6 +255,7 @@ int rf_sim::alloc_all()
     ALLOC(d_force, N3);
     ALLOC(d_wp, (size_t)(kMaxTerms + 1) * kMaxQuad);
     ALLOC(d_pv, (size_t)kMaxQuad);
+    ALLOC(d_far, sizeof(tab.far) / sizeof(double));
     const size_t es = mixed ? sizeof(float) : sizeof(double);
     {
         void* q = nullptr;
@@ -908,7 +1018,7 @@ int rf_sim::apply_operator(int mode, const double* x, double* y)
         if ((rc = timed_pair(&ea, &eb))) return rc;
         HIP_TRY(hipEventRecord(ea, stream));
     }
-    HIP_TRY(launch_operator(planOp, tab, mode, d_pos[lvl_three], d_orient[lvl_three], d_force, x, d_wp, d_pv, d_op, y,
+    HIP_TRY(launch_operator(planOp, tab, mode, d_pos[lvl_three], d_orient[lvl_three], d_force, x, d_wp, d_pv, d_far, d_op, y,
                             stream));
     if (p.profile) {
         HIP_TRY(hipEventRecord(eb, stream));
@@ -1396,6 +1506,8 @@ extern "C" int rf_create(const rf_params* params, int32_t num_fibers, const doub
         e = hipMemcpyAsync(s->d_wp, s->tab.wp, sizeof(s->tab.wp), hipMemcpyHostToDevice, s->stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(s->d_pv, s->tab.pv, sizeof(s->tab.pv), hipMemcpyHostToDevice, s->stream);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(s->d_far, s->tab.far, sizeof(s->tab.far), hipMemcpyHostToDevice, s->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
     if (e != hipSuccess) {
         delete s;

@@ -45,6 +45,7 @@ struct rf_sim {
     double* d_force = nullptr;
     double* d_wp = nullptr;
     double* d_pv = nullptr;
+    double* d_far = nullptr;  // Tables::far
     void* d_A = nullptr;  // n x n, lda, double or float
     void* d_W = nullptr;  // 6N x 3(M+1)N, ldw
     double* d_b = nullptr;
