@@ -45,20 +45,11 @@ __device__ __forceinline__ void unpack(const V& v, double (&o)[N])
 // Workgroup: 64*RPL consecutive rows x one column split.  Wavefront w of the
 // workgroup takes columns c0+w, c0+w+4, ...; each lane loads 16 bytes (RPL
 // rows) per column, so one wavefront load is a 1 KiB contiguous segment.
-// With xs.nrm2 the vector is x / sqrt(*xs.nrm2), formed exactly as
-// scale_copy_kernel forms it, and the workgroups of the first row block
-// store it to xs.out (each column once): the next Arnoldi vector and its
-// product in one pass.
-struct XScale {
-    const double* nrm2;
-    double* out;
-};
-
 template <typename T>
 __global__ void __launch_bounds__(kGemvThreads) gemv_parts_kernel(int cols, int64_t ld, const T* __restrict__ A,
                                                                   const double* __restrict__ x,
                                                                   double* __restrict__ parts, int64_t pstride,
-                                                                  int cols_per_split, XScale xs)
+                                                                  int cols_per_split)
 {
     using V = typename Vec16<T>::type;
     constexpr int RPL = Vec16<T>::n;
@@ -72,9 +63,6 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_parts_kernel(int cols, int6
     double acc[RPL];
 #pragma unroll
     for (int r = 0; r < RPL; ++r) acc[r] = 0.0;
-    const bool scaled = xs.nrm2 != nullptr;
-    const double inv = scaled ? 1.0 / sqrt(*xs.nrm2) : 1.0;
-    const bool store_x = scaled && xs.out != nullptr && blockIdx.x == 0 && lane == 0;
     const T* Ab = A + row0;
     int c = c0 + wave;
     for (; c + 4 * (kGemvUnroll - 1) < c1; c += 4 * kGemvUnroll) {
@@ -83,11 +71,7 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_parts_kernel(int cols, int6
 #pragma unroll
         for (int u = 0; u < kGemvUnroll; ++u) {
             v[u] = __builtin_nontemporal_load(reinterpret_cast<const V*>(Ab + (int64_t)(c + 4 * u) * ld));
-            xv[u] = scaled ? x[c + 4 * u] * inv : x[c + 4 * u];
-        }
-        if (store_x) {
-#pragma unroll
-            for (int u = 0; u < kGemvUnroll; ++u) xs.out[c + 4 * u] = xv[u];
+            xv[u] = x[c + 4 * u];
         }
 #pragma unroll
         for (int u = 0; u < kGemvUnroll; ++u) {
@@ -99,8 +83,7 @@ __global__ void __launch_bounds__(kGemvThreads) gemv_parts_kernel(int cols, int6
     }
     for (; c < c1; c += 4) {
         const V v = __builtin_nontemporal_load(reinterpret_cast<const V*>(Ab + (int64_t)c * ld));
-        const double xv = scaled ? x[c] * inv : x[c];
-        if (store_x) xs.out[c] = xv;
+        const double xv = x[c];
         double e[RPL];
         unpack(v, e);
 #pragma unroll
@@ -202,98 +185,336 @@ __global__ void __launch_bounds__(kDotThreads) multidot_kernel(const double* __r
     }
 }
 
-// w -= V[:, :k] h
-__global__ void orth_update_kernel(const double* __restrict__ V, int64_t ldv, int k, const double* __restrict__ h,
-                                   double* __restrict__ w, int n)
+// ---------------------------------------------------------------------------
+// One Arnoldi step after the product (or the norm of a residual) in one launch:
+//     w = sum of the product's column splits (or b minus it, or w as it is),
+//     h1 = V^T w, w -= V h1, h2 = V^T w, w -= V h2, |w|^2, v_next = w / |w|,
+// h1, h2 and |w|^2 to the host.  As separate kernels (split sums, dots, update
+// with dots, update with norm, scaling) the step is up to five launches whose
+// time is latency: 26 us of an iteration at n = 1500, 31 at n = 4995, 36 at
+// n = 15000 and 72 at n = 60000; in one launch it is 8.7, 11.6, 13.3 and 28 us,
+// bound by the three exchanges and, from a few rows a thread on, by the loads
+// of V (n = 15000 with 16 workgroups and two rows a thread: 23 us).
+//
+// Up to 32 workgroups split the rows, each thread its own; the sums cross the
+// workgroups three times.  A workgroup publishes its partial sums as they are,
+// with agent-scope stores into slots that hold kEmpty until then, and reads
+// those of all others in the same fixed order (so every workgroup computes the
+// same bits): no counter, and no release fence, which would write a whole L2
+// back.  A launch uses one of two sets of slots and empties its own slots of
+// the other set for the next launch on the stream.
+// The workgroups wait for each other, so all of them must be resident at once.
+// Two fit a CU (128 registers), 512 the chip: the launches of 32 streams to
+// n = 8192 (16 workgroups) and of 16 above, where a process has four hardware
+// queues by default; any other kernel that holds a place ends
+// by itself.  The wait is bounded all the same: after kSpinLimit polls a
+// workgroup goes on with NaN and the host's words stay empty, which the host
+// reports.  Those words are published like the slots, each by itself (the
+// host empties them before the launch): a sequence word after them needs a
+// system-scope fence that the whole step would wait for.
+constexpr int kArnThreads = 512;
+constexpr int kArnWaves = kArnThreads / 64;
+constexpr int kArnMaxK = 64;             // basis vectors at most
+constexpr int kArnBlocks = 32;           // workgroups at most (a power of two)
+constexpr int kSpinLimit = 1 << 22;      // a few seconds
+constexpr unsigned long long kEmpty = kArnoldiEmpty, kNaN = 0x7FF8000000000000ull;
+
+struct ArnArgs {
+    const double* parts;  // [splits][pstride]: w is their sum; null: w as it is
+    int splits;
+    int64_t pstride;
+    const double* b;      // not null: w = b - the sum
+    double* w;
+    double* V;
+    int64_t ldv;
+    int k, n;
+    double* v_next;       // w / |w|, or null
+    unsigned long long* slots;  // [2][3][slot_rows][gridDim.x]
+    int set, slot_rows;
+    double* nrm_out;      // |w|^2 on the device
+    unsigned long long* host;  // h1 at 0, h2 at ld_host, |w|^2 at 2 ld_host
+    int ld_host;
+};
+
+// v of the lane across offset OFF (for 4: the lane mirrored within its eight,
+// which differs in bit 2 too), by DPP.
+template <int OFF>
+__device__ __forceinline__ double dpp_across(double v)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double s = w[i];
-    for (int j = 0; j < k; ++j) s -= V[(int64_t)j * ldv + i] * h[j];
-    w[i] = s;
+    constexpr int ctrl = OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : OFF == 4 ? 0x141 : 0x128;
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), ctrl, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), ctrl, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+// OFF = 32, 16: a in the lanes below and b in those above, each summed over
+// the pair of lanes, by the half (row) swap that exchanges both at once.
+template <int OFF>
+__device__ __forceinline__ double swap_sum(double a, double b)
+{
+    auto swap = [](unsigned x, unsigned y) {
+        if constexpr (OFF == 32)
+            return __builtin_amdgcn_permlane32_swap(x, y, false, false);
+        else
+            return __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    };
+    const auto lo = swap((unsigned)__double2loint(a), (unsigned)__double2loint(b));
+    const auto hi = swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b));
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+// a[0..CH) (CH = 16 or 32) summed over the wavefront; lane l ends with the sum
+// of index arn_index<CH>(l) in a[0].  Each step halves the values a lane
+// keeps; it stays in the vector unit (through LDS the 32 exchanges of two
+// words by eight wavefronts took about 1 us a reduction).
+template <int CH>
+__device__ __forceinline__ int arn_index(int lane)
+{
+    int j = 0;
+#pragma unroll
+    for (int bit = 5, half = CH / 2; half >= 1; --bit, half /= 2) j += ((lane >> bit) & 1) * half;
+    return j;
+}
+template <int CH, int HALF = CH / 2, int OFF = 32>
+__device__ __forceinline__ void wave_sums(double (&a)[CH], int lane)
+{
+    if constexpr (OFF >= 16) {
+#pragma unroll
+        for (int u = 0; u < HALF; ++u) a[u] = swap_sum<OFF>(a[u], a[u + HALF]);
+        wave_sums<CH, HALF / 2, OFF / 2>(a, lane);
+    } else if constexpr (HALF >= 1) {
+        const bool hi = (lane & OFF) != 0;
+#pragma unroll
+        for (int u = 0; u < HALF; ++u) {
+            const double send = hi ? a[u] : a[u + HALF];
+            const double keep = hi ? a[u + HALF] : a[u];
+            a[u] = keep + dpp_across<OFF>(send);
+        }
+        wave_sums<CH, HALF / 2, OFF / 2>(a, lane);
+    } else if constexpr (OFF >= 1) {
+        a[0] += dpp_across<OFF>(a[0]);
+        wave_sums<CH, 0, OFF / 2>(a, lane);
+    }
 }
 
-// Fused w -= V[:, :k] h and the dots that follow it: out[j] = V[:, j]^T w for
-// j < nd (nd = k or 0) and out[nd] = w^T w, with w updated in the same pass.
-// Rows, partial sums and the last workgroup's fixed-order reduction follow
-// orth_update_kernel then multidot_kernel exactly (same grid-stride rows per
-// thread, same wave and block sums, same partial layout), so the results are
-// bit-identical to the two-kernel sequence with one launch less.  k <= MAXK.
-// With hc.dst the last workgroup then does what to_host_kernel does: copies
-// hc.words words from hc.src (out included) to host memory and stores the
-// sequence word after them at system scope.
-template <int MAXK>
-__global__ void __launch_bounds__(kDotThreads) orth_dots_kernel(const double* __restrict__ V, int64_t ldv, int k,
-                                                                const double* __restrict__ h,
-                                                                double* __restrict__ w, int n, int nd,
-                                                                double* __restrict__ parts,
-                                                                unsigned int* counter, double* __restrict__ out,
-                                                                HostCopy hc)
+struct ArnShared {
+    double sh[kArnWaves][32];
+    double h[2][kArnMaxK];
+    double nrm;
+    int late;  // a wait ran out
+};
+
+// The workgroup's sums of a[0..count) into slots [row0 + j][block].
+template <int CH>
+__device__ __forceinline__ void arn_publish(double (&a)[CH], int count, unsigned long long* slots, ArnShared& S)
 {
-    __shared__ double hs[MAXK];
-    __shared__ double sh[MAXK + 1][kDotThreads / 64];
-    __shared__ bool last;
-    if (threadIdx.x < MAXK) hs[threadIdx.x] = (threadIdx.x < k) ? h[threadIdx.x] : 0.0;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    wave_sums<CH>(a, lane);
+    if ((lane & (64 / CH - 1)) == 0) S.sh[wave][arn_index<CH>(lane)] = a[0];
     __syncthreads();
-    double acc[MAXK + 1];
-#pragma unroll
-    for (int j = 0; j <= MAXK; ++j) acc[j] = 0.0;
-    const int nbx = gridDim.x;
-    for (int i = blockIdx.x * kDotThreads + threadIdx.x; i < n; i += nbx * kDotThreads) {
-        double v[MAXK];
-#pragma unroll
-        for (int j = 0; j < MAXK; ++j) v[j] = (j < k) ? V[(int64_t)j * ldv + i] : 0.0;
-        double x = w[i];
-#pragma unroll
-        for (int j = 0; j < MAXK; ++j)
-            if (j < k) x -= v[j] * hs[j];
-        w[i] = x;
-#pragma unroll
-        for (int j = 0; j < MAXK; ++j)
-            if (j < nd) acc[j] += v[j] * x;
-        acc[MAXK] += x * x;
-    }
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-    for (int j = 0; j <= MAXK; ++j) {
-        if (j < nd || j == MAXK) {
-            const double t = wave_sum(acc[j]);
-            if (lane == 0) sh[j][wv] = t;
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x <= nd) {  // slot nd carries the norm
-        const int src = (threadIdx.x == nd) ? MAXK : threadIdx.x;
+    if ((int)threadIdx.x < count) {
         double t = 0.0;
-        for (int q = 0; q < (int)(blockDim.x >> 6); ++q) t += sh[src][q];
-        parts[(int64_t)threadIdx.x * nbx + blockIdx.x] = t;
-    }
-    __threadfence();
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned int prev = atomicAdd(counter, 1u);
-        last = (prev == (unsigned int)nbx - 1);
+#pragma unroll
+        for (int q = 0; q < kArnWaves; ++q) t += S.sh[q][threadIdx.x];
+        unsigned long long bits = __double_as_longlong(t);
+        if (bits == kEmpty) bits = kNaN;
+        __hip_atomic_store(&slots[(size_t)threadIdx.x * gridDim.x + blockIdx.x], bits, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
-    if (last) {
-        __threadfence();
-        for (int jj = threadIdx.x; jj <= nd; jj += kDotThreads) {
-            double t = 0.0;
-            for (int b = 0; b < nbx; ++b)
-                t += __hip_atomic_load(&parts[(int64_t)jj * nbx + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            out[jj] = t;
+}
+
+// out[j] = the sum over all workgroups of slot row j, j < count.
+__device__ __forceinline__ void arn_gather(int count, unsigned long long* slots, double* out, ArnShared& S)
+{
+    const int nb = gridDim.x;  // a power of two up to 32: a row's slots share a wavefront
+    for (int e = threadIdx.x; e < count * nb; e += kArnThreads) {
+        unsigned long long bits = kEmpty;
+        for (int spin = 0; spin < kSpinLimit && bits == kEmpty; ++spin)
+            bits = __hip_atomic_load(&slots[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (bits == kEmpty) S.late = 1;
+        double v = __longlong_as_double(bits);
+        if (nb > 1) v += dpp_across<1>(v);
+        if (nb > 2) v += dpp_across<2>(v);
+        if (nb > 4) v += dpp_across<4>(v);
+        if (nb > 8) v += dpp_across<8>(v);
+        if (nb > 16) v = swap_sum<16>(v, v);
+        if (e % nb == 0) out[e / nb] = v;
+    }
+    __syncthreads();
+}
+
+// ONE: one row a thread and k <= 32: w and the thread's row of V stay in
+// registers, V is read once.
+template <bool ONE>
+__global__ void __launch_bounds__(kArnThreads, 4) arnoldi_kernel(const ArnArgs a)
+{
+    constexpr int CH = ONE ? 32 : 16;  // basis vectors held at a time
+    __shared__ ArnShared S;
+    const int tid = threadIdx.x, nb = gridDim.x, k = a.k, n = a.n;
+    const int step = nb * kArnThreads;
+    const int first = blockIdx.x * kArnThreads + tid;
+    const size_t set = (size_t)3 * a.slot_rows * nb;
+    unsigned long long* slots = a.slots + (size_t)a.set * set;
+    unsigned long long* other = a.slots + (size_t)(1 - a.set) * set;
+    for (int e = tid; e < 3 * a.slot_rows; e += kArnThreads)
+        __hip_atomic_store(&other[(size_t)e * nb + blockIdx.x], kEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) S.late = 0;
+    auto phase = [&](int ph, int row) { return slots + ((size_t)ph * a.slot_rows + row) * nb; };
+    // w of rows i and i2 (the same row: once)
+    auto product2 = [&](int i, int i2, double& w1, double& w2) {
+        w1 = w2 = 0.0;
+        if (!a.parts) return;
+        for (int q = 0; q < a.splits; q += 16) {
+            double p1[16], p2[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                const double* row = a.parts + (int64_t)min(q + u, a.splits - 1) * a.pstride;
+                p1[u] = row[i];
+                if constexpr (!ONE) p2[u] = row[i2];
+            }
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                w1 += (q + u < a.splits) ? p1[u] : 0.0;
+                if constexpr (!ONE) w2 += (q + u < a.splits) ? p2[u] : 0.0;
+            }
         }
-        if (threadIdx.x == 0) atomicExch(counter, 0u);
-        if (hc.dst) {
-            __threadfence();
-            __syncthreads();
-            for (int i = threadIdx.x; i < hc.words; i += kDotThreads)
-                hc.dst[i] = __hip_atomic_load(&hc.src[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __threadfence_system();
-            __syncthreads();
-            if (threadIdx.x == 0) __hip_atomic_store(hc.seq_word, hc.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (a.b) {
+            w1 = a.b[i] - w1;
+            w2 = a.b[i2] - w2;
+        }
+    };
+    // columns c0.. of V at row i; past the last vector, the last one again
+    auto load = [&](int i, int c0, double (&v)[CH]) {
+#pragma unroll
+        for (int g = 0; g < CH; g += 8) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[g + u] = 0.0;
+            if (c0 + g < k) {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[g + u] = a.V[(int64_t)min(c0 + g + u, k - 1) * a.ldv + i];
+            }
+        }
+    };
+    auto subtract = [&](double w, const double (&v)[CH], const double* h) {
+#pragma unroll
+        for (int g = 0; g < CH; ++g) w -= v[g] * h[g];
+        return w;
+    };
+    if (tid < kArnMaxK) S.h[0][tid] = S.h[1][tid] = 0.0;  // zero past k
+    double w = 0.0, v[CH], acc[CH];
+    auto clear = [&] {
+#pragma unroll
+        for (int j = 0; j < CH; ++j) acc[j] = 0.0;
+    };
+    if constexpr (ONE) {
+        const int i = min(first, n - 1);
+        if (k > 0) load(i, 0, v);
+        double same;
+        if (a.parts)
+            product2(i, i, w, same);
+        else
+            w = a.w[i];
+        if (first >= n) w = 0.0;
+        if (k == 0 && a.parts && first < n) a.w[i] = w;
+        for (int ph = 0; ph < 2 && k > 0; ++ph) {
+#pragma unroll
+            for (int j = 0; j < CH; ++j) acc[j] = v[j] * w;
+            arn_publish(acc, k, phase(ph, 0), S);
+            arn_gather(k, phase(ph, 0), S.h[ph], S);
+            w = (first < n) ? subtract(w, v, S.h[ph]) : 0.0;
+        }
+        clear();
+        acc[0] = w * w;
+    } else {
+        // two rows at a time: i and i + step (past the end, row i again with w = 0)
+        double v2[CH], w2 = 0.0;
+        auto rows = [&](auto body) {
+            for (int i = first; i < n; i += 2 * step) body(i, i + step < n ? i + step : i, i + step < n);
+        };
+        auto load2 = [&](int i, int i2, bool two) {
+            w = a.w[i];
+            w2 = two ? a.w[i2] : 0.0;
+        };
+        auto store2 = [&](int i, int i2, bool two) {
+            a.w[i] = w;
+            if (two) a.w[i2] = w2;
+        };
+        rows([&](int i, int i2, bool two) {
+            product2(i, i2, w, w2);
+            if (a.parts) store2(i, i2, two);
+        });
+        for (int ph = 0; ph < 2 && k > 0; ++ph) {
+            for (int c0 = 0; c0 < k; c0 += CH) {
+                clear();
+                rows([&](int i, int i2, bool two) {
+                    load(i, c0, v);
+                    load(i2, c0, v2);
+                    load2(i, i2, two);
+                    if (ph == 1 && k <= CH) {  // the update with its dots
+                        w = subtract(w, v, S.h[0]);
+                        w2 = two ? subtract(w2, v2, S.h[0]) : 0.0;
+                        store2(i, i2, two);
+                    }
+#pragma unroll
+                    for (int j = 0; j < CH; ++j) acc[j] += v[j] * w + v2[j] * w2;
+                });
+                arn_publish(acc, min(CH, k - c0), phase(ph, c0), S);
+            }
+            arn_gather(k, phase(ph, 0), S.h[ph], S);
+            if (ph == 0 && k <= CH) continue;
+            clear();
+            rows([&](int i, int i2, bool two) {
+                load2(i, i2, two);
+                for (int c0 = 0; c0 < k; c0 += CH) {
+                    load(i, c0, v);
+                    load(i2, c0, v2);
+                    w = subtract(w, v, S.h[ph] + c0);
+                    w2 = subtract(w2, v2, S.h[ph] + c0);
+                }
+                if (!two) w2 = 0.0;
+                store2(i, i2, two);
+                acc[0] += w * w + w2 * w2;
+            });
+        }
+        if (k == 0) {
+            clear();
+            rows([&](int i, int i2, bool two) {
+                load2(i, i2, two);
+                acc[0] += w * w + w2 * w2;
+            });
         }
     }
+    arn_publish(acc, 1, phase(2, 0), S);
+    arn_gather(1, phase(2, 0), &S.nrm, S);
+    const double nrm = S.nrm;
+    if (blockIdx.x == 0) {
+        if (tid == 0) *a.nrm_out = nrm;
+        auto send = [&](int at, double v) {
+            unsigned long long bits = __double_as_longlong(v);
+            if (bits == kEmpty) bits = kNaN;
+            __hip_atomic_store(&a.host[at], bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        };
+        if (!S.late) {
+            if (tid < k) {
+                send(tid, S.h[0][tid]);
+                send(a.ld_host + tid, S.h[1][tid]);
+            }
+            if (tid == 0) send(2 * a.ld_host, nrm);
+        }
+    }
+    if (a.v_next) {
+        const double inv = 1.0 / sqrt(nrm);
+        if constexpr (ONE) {
+            if (first < n) a.v_next[first] = w * inv;
+        } else {
+            for (int i = first; i < n; i += step) a.v_next[i] = a.w[i] * inv;
+        }
+    }
+}
+
+__global__ void fill_slots_kernel(unsigned long long* slots, int count)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < count) slots[i] = kEmpty;
 }
 
 // v = w / sqrt(nrm2[idx])
@@ -402,19 +623,22 @@ GemvPlan plan_gemv(int rows, int cols, int64_t ld, int elem_bytes, int num_cus)
     return p;
 }
 
+int64_t gemv_parts_stride(const GemvPlan& p)
+{
+    return (int64_t)p.row_blocks * 64 * (16 / p.elem_bytes);
+}
+
 size_t gemv_parts_elems(const GemvPlan& p)
 {
-    const int rows_per_block = 64 * (16 / p.elem_bytes);
-    return (size_t)p.splits * (size_t)p.row_blocks * rows_per_block;
+    return (size_t)p.splits * (size_t)gemv_parts_stride(p);
 }
 
 hipError_t launch_gemv(const GemvPlan& p, const void* A, const double* x, double* parts, double* y, const double* b,
-                       int mode, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1, const double* x_nrm2, double* x_out)
+                       int mode, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1)
 {
-    const XScale xs{x_nrm2, x_out};
     const int rows_per_block = 64 * (16 / p.elem_bytes);
     if (p.ld % rows_per_block != 0) return hipErrorInvalidValue;  // loads assume whole row blocks
-    const int64_t pstride = (int64_t)p.row_blocks * rows_per_block;
+    const int64_t pstride = gemv_parts_stride(p);
     const int cps = (p.cols + p.splits - 1) / p.splits;
     dim3 grid(p.row_blocks, p.splits);
     if (ev0) {
@@ -423,16 +647,17 @@ hipError_t launch_gemv(const GemvPlan& p, const void* A, const double* x, double
     }
     if (p.elem_bytes == 8)
         hipLaunchKernelGGL(gemv_parts_kernel<double>, grid, dim3(kGemvThreads), 0, s, p.cols, p.ld,
-                           static_cast<const double*>(A), x, parts, pstride, cps, xs);
+                           static_cast<const double*>(A), x, parts, pstride, cps);
     else
         hipLaunchKernelGGL(gemv_parts_kernel<float>, grid, dim3(kGemvThreads), 0, s, p.cols, p.ld,
-                           static_cast<const float*>(A), x, parts, pstride, cps, xs);
+                           static_cast<const float*>(A), x, parts, pstride, cps);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (ev1) {
         e = hipEventRecord(ev1, s);
         if (e != hipSuccess) return e;
     }
+    if (!y) return hipSuccess;  // the partial sums are what the caller wants
     hipLaunchKernelGGL(reduce_splits_kernel, dim3((p.rows * kSplitLanes + 255) / 256), dim3(256), 0, s, parts,
                        p.splits, pstride, p.rows, b, mode, y);
     return hipGetLastError();
@@ -458,26 +683,54 @@ hipError_t launch_multidot(const double* V, int64_t ldv, int k, const double* w,
     return hipGetLastError();
 }
 
-hipError_t launch_orth_dots(const double* V, int64_t ldv, int k, const double* h, double* w, int n, int with_dots,
-                            double* parts, unsigned int* counter, double* out, hipStream_t s, const HostCopy& hc)
+// workgroups of an n-row step: one row a thread as far as 32 go
+static int arnoldi_blocks(int n)
 {
-    const int nd = with_dots ? k : 0;
-    const dim3 grid(multidot_blocks(n)), block(kDotThreads);
-    if (hc.dst && (hc.words < 0 || hc.words > 16384 || !hc.src || !hc.seq_word)) return hipErrorInvalidValue;
-    if (k <= 16) {
-        hipLaunchKernelGGL(orth_dots_kernel<16>, grid, block, 0, s, V, ldv, k, h, w, n, nd, parts, counter, out, hc);
-        return hipGetLastError();
-    }
-    if (k <= 32) {
-        hipLaunchKernelGGL(orth_dots_kernel<32>, grid, block, 0, s, V, ldv, k, h, w, n, nd, parts, counter, out, hc);
-        return hipGetLastError();
-    }
-    hipLaunchKernelGGL(orth_update_kernel, dim3((n + 255) / 256), dim3(256), 0, s, V, ldv, k, h, w, n);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    e = launch_multidot(with_dots ? V : nullptr, ldv, nd, w, n, parts, counter, out, s);
-    if (e != hipSuccess || !hc.dst) return e;
-    return launch_to_host(hc.src, hc.dst, sizeof(unsigned) * (size_t)hc.words, s, hc.seq_word, hc.seq);
+    int nb = 1;
+    while (nb < kArnBlocks && nb * kArnThreads < n) nb *= 2;
+    return nb;
+}
+
+size_t arnoldi_slots(int max_k)
+{
+    return (size_t)2 * 3 * std::max(1, max_k) * kArnBlocks;
+}
+
+hipError_t launch_arnoldi_init(unsigned long long* slots, int max_k, hipStream_t s)
+{
+    const int count = (int)arnoldi_slots(max_k);
+    hipLaunchKernelGGL(fill_slots_kernel, dim3((count + 255) / 256), dim3(256), 0, s, slots, count);
+    return hipGetLastError();
+}
+
+hipError_t launch_arnoldi(const ArnoldiStep& st, hipStream_t s)
+{
+    if (st.n < 1 || st.k < 0 || st.k > st.max_k || st.max_k > kArnMaxK || !st.w || !st.slots || !st.host ||
+        !st.nrm_out)
+        return hipErrorInvalidValue;
+    ArnArgs a;
+    a.parts = st.product ? st.parts : nullptr;
+    a.splits = st.product ? st.product->splits : 0;
+    a.pstride = st.product ? gemv_parts_stride(*st.product) : 0;
+    a.b = st.b;
+    a.w = st.w;
+    a.V = st.V;
+    a.ldv = st.ldv;
+    a.k = st.k;
+    a.n = st.n;
+    a.v_next = st.v_next;
+    a.slots = st.slots;
+    a.set = st.set & 1;
+    a.slot_rows = std::max(1, st.max_k);
+    a.nrm_out = st.nrm_out;
+    a.host = st.host;
+    a.ld_host = st.ld_host;
+    const int nb = arnoldi_blocks(st.n);
+    if (st.n <= nb * kArnThreads && st.k <= 32)
+        hipLaunchKernelGGL(arnoldi_kernel<true>, dim3(nb), dim3(kArnThreads), 0, s, a);
+    else
+        hipLaunchKernelGGL(arnoldi_kernel<false>, dim3(nb), dim3(kArnThreads), 0, s, a);
+    return hipGetLastError();
 }
 
 hipError_t launch_scale_copy(const double* w, const double* nrm2, int idx, int n, double* v, hipStream_t s)

@@ -292,6 +292,16 @@ int rf_sim::alloc_all()
     ALLOC(d_dparts, (size_t)kMaxDotBlocks * (m + 2) + 64);
     ALLOC(d_dots, (size_t)(3 * (m + 2) + 8));
     ALLOC(d_counter, 1);
+    {
+        void* q = nullptr;
+        if (hipMalloc(&q, sizeof(unsigned long long) * arnoldi_slots(m)) != hipSuccess) {
+            rf::set_error("device allocation failed");
+            return RF_ENOMEM;
+        }
+        allocs.push_back(q);
+        d_slots = static_cast<unsigned long long*>(q);
+        HIP_TRY(launch_arnoldi_init(d_slots, m, stream));
+    }
     ALLOC(d_op, operator_scratch_doubles(planOp));
     ALLOC(d_res64, (size_t)lda);
     ALLOC(d_dx, (size_t)lda);
@@ -379,14 +389,14 @@ void rf_sim::resolve_timed()
     ev_pending.swap(running);
 }
 
-int rf_sim::gemv_A(const double* x, double* y, const double* b, int mode, const double* x_nrm2, double* x_out)
+int rf_sim::gemv_A(const double* x, double* y, const double* b, int mode)
 {
     hipEvent_t a = nullptr, e = nullptr;
     if (p.profile) {
         int rc = timed_pair(&a, &e);
         if (rc) return rc;
     }
-    HIP_TRY(launch_gemv(planA, d_A, x, d_gparts, y, b, mode, stream, a, e, x_nrm2, x_out));
+    HIP_TRY(launch_gemv(planA, d_A, x, d_gparts, y, b, mode, stream, a, e));
     if (p.profile) timed_push(a, e, kGemvA);
     return RF_OK;
 }
@@ -394,22 +404,12 @@ int rf_sim::gemv_A(const double* x, double* y, const double* b, int mode, const 
 // The copy into h_dots whose sequence number is host_seq has landed: its
 // sequence word is written after its data at system scope.  Normally it has
 // by the time the stream reports completion; otherwise wait for the stream
-// and look again, and report a stale copy as an error.  poll: the stream
-// holds more work after the copy, so watch the sequence word itself (up to
-// a second) before waiting for the whole stream.
-int rf_sim::await_host_copy(bool poll)
+// and look again, and report a stale copy as an error.
+int rf_sim::await_host_copy()
 {
     const unsigned* w = host_seq_word();
     for (int spin = 0; spin < 1024; ++spin)
         if (__atomic_load_n(w, __ATOMIC_ACQUIRE) == host_seq) return RF_OK;
-    if (poll) {
-        const auto t0 = std::chrono::steady_clock::now();
-        for (;;) {
-            for (int spin = 0; spin < 4096; ++spin)
-                if (__atomic_load_n(w, __ATOMIC_ACQUIRE) == host_seq) return RF_OK;
-            if (std::chrono::steady_clock::now() - t0 > std::chrono::seconds(1)) break;
-        }
-    }
     HIP_TRY(hipStreamSynchronize(stream));
     if (__atomic_load_n(w, __ATOMIC_ACQUIRE) == host_seq) return RF_OK;
     rf::set_error("the dot block copied to host memory is stale (sequence word " +
@@ -426,13 +426,72 @@ int rf_sim::fetch_dots(int count)
     return await_host_copy();
 }
 
-// ||v||^2 into h_dots[0]
+// ||v||^2, in d_dots[0] too
 int rf_sim::norm2(const double* v, double* out)
 {
-    HIP_TRY(launch_multidot(nullptr, 0, 0, v, n, d_dparts, d_counter, d_dots, stream));
-    int rc = fetch_dots(1);
-    if (rc) return rc;
-    *out = h_dots[0];
+    int rc = arnoldi(const_cast<double*>(v), false, nullptr, nullptr, 0, nullptr);
+    if (rc || (rc = await_arnoldi(0))) return rc;
+    *out = h_dots[2 * (restart + 2)];
+    return RF_OK;
+}
+
+int rf_sim::arnoldi(double* w, bool product, const double* b, double* V, int k, double* v_next)
+{
+    ArnoldiStep st;
+    st.product = product ? &planA : nullptr;
+    st.parts = d_gparts;
+    st.b = b;
+    st.w = w;
+    st.V = V;
+    st.ldv = lda;
+    st.k = k;
+    st.n = n;
+    st.max_k = restart;
+    st.v_next = v_next;
+    st.slots = d_slots;
+    st.set = arn_set;
+    st.nrm_out = d_dots;
+    st.host = reinterpret_cast<unsigned long long*>(h_dots);
+    st.ld_host = restart + 2;
+    for (int j = 0; j < k; ++j)
+        for (int i : {j, st.ld_host + j}) __atomic_store_n(&st.host[i], kArnoldiEmpty, __ATOMIC_RELAXED);
+    __atomic_store_n(&st.host[2 * st.ld_host], kArnoldiEmpty, __ATOMIC_RELEASE);
+    HIP_TRY(launch_arnoldi(st, stream));
+    arn_set ^= 1;
+    return RF_OK;
+}
+
+// The scalars of the last arnoldi(.., k, ..) have landed in h_dots.  The
+// stream may hold more work after the step: watch the words (up to a second)
+// before waiting for the whole stream.
+int rf_sim::await_arnoldi(int k)
+{
+    const unsigned long long* h = reinterpret_cast<const unsigned long long*>(h_dots);
+    const int ld = restart + 2;
+    auto landed = [&] {
+        if (__atomic_load_n(&h[2 * ld], __ATOMIC_ACQUIRE) == kArnoldiEmpty) return false;
+        for (int j = 0; j < k; ++j)
+            for (int i : {j, ld + j})
+                if (__atomic_load_n(&h[i], __ATOMIC_ACQUIRE) == kArnoldiEmpty) return false;
+        return true;
+    };
+    const auto t0 = std::chrono::steady_clock::now();
+    for (;;) {
+        for (int spin = 0; spin < 4096; ++spin)
+            if (landed()) return RF_OK;
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::seconds(1)) break;
+    }
+    HIP_TRY(hipStreamSynchronize(stream));
+    if (landed()) return RF_OK;
+    rf::set_error("an Arnoldi step ended without its result");
+    return RF_EHIP;
+}
+
+int rf_sim::residual_norm(const double* x, double* r, double* v, double* rr)
+{
+    int rc = gemv_A(x, nullptr, nullptr, 0);
+    if (rc || (rc = arnoldi(r, true, d_b, nullptr, 0, v)) || (rc = await_arnoldi(0))) return rc;
+    *rr = h_dots[2 * (restart + 2)];
     return RF_OK;
 }
 
@@ -515,31 +574,27 @@ int rf_sim::solve_gmres(int* iters_out, double* be_out, int* status_out, int max
         return RF_OK;
     }
     // r0 = b - A x (the learned guess leaves it in d_r)
-    if (r0_ready)
-        r0_ready = false;
-    else if ((rc = gemv_A(d_x, d_r, d_b, 1)))
-        return rc;
     double beta2;
-    if ((rc = norm2(d_r, &beta2))) return rc;
+    if (r0_ready) {
+        r0_ready = false;
+        if ((rc = norm2(d_r, &beta2))) return rc;
+        HIP_TRY(launch_scale_copy(d_r, d_dots, 0, n, d_V, stream));
+    } else if ((rc = residual_norm(d_x, d_r, d_V, &beta2))) {
+        return rc;
+    }
     double beta = std::sqrt(beta2);
     stats.last_initial_residual = beta / bn;
     if (beta == 0.0) {
         *be_out = 0.0;
         return RF_OK;
     }
-    // norm2 left ||r0||^2 in d_dots[0]
-    HIP_TRY(launch_scale_copy(d_r, d_dots, 0, n, d_V, stream));
     int iterOut = 0;
-    const int64_t ldv = lda;
-    double* D1 = d_dots;
-    double* D2 = d_dots + (m + 2);
-    double* D3 = d_dots + 2 * (m + 2);
-    // w = A v_j, or A M^-1 v_j with the right preconditioner
+    // w = A v_j, or A M^-1 v_j with the right preconditioner (its splits in d_gparts)
     auto matvec = [&](int j) -> int {
         const double* vj = d_V + (size_t)j * lda;
-        if (!prec_ready) return gemv_A(vj, d_w, nullptr, 0);
+        if (!prec_ready) return gemv_A(vj, nullptr, nullptr, 0);
         const int r = precond_apply(vj, d_z);
-        return r ? r : gemv_A(d_z, d_w, nullptr, 0);
+        return r ? r : gemv_A(d_z, nullptr, nullptr, 0);
     };
     for (;;) {
         std::fill(H.begin(), H.end(), 0.0);
@@ -547,37 +602,21 @@ int rf_sim::solve_gmres(int* iters_out, double* be_out, int* status_out, int max
         g[0] = beta;
         double bea = 0.0;
         bool have_xc = false;
-        bool w_ready = false;  // d_w already holds the product for v_jH
+        bool w_ready = false;  // d_gparts already holds the product for v_jH
         for (int jH = 0; jH < m; ++jH) {
             const int k = jH + 1;
             if (!w_ready && (rc = matvec(jH))) return rc;
             w_ready = false;
-            HIP_TRY(launch_multidot(d_V, ldv, k, d_w, n, d_dparts, d_counter, D1, stream));
-            HIP_TRY(launch_orth_dots(d_V, ldv, k, D1, d_w, n, 1, d_dparts, d_counter, D2, stream));
-            // The second pass ends by copying the Hessenberg column to the
-            // host.  The next basis vector is then on the device, so its
-            // product is queued before the host waits (it is discarded if
-            // this iteration ends the solve); without a preconditioner the
-            // product forms v_k = w / |w| itself and stores it.
-            HostCopy hc;
-            hc.src = reinterpret_cast<const unsigned*>(d_dots);
-            hc.dst = reinterpret_cast<unsigned*>(h_dots);
-            hc.words = (int)(sizeof(double) / sizeof(unsigned)) * 3 * (m + 2);
-            hc.seq_word = host_seq_word();
-            hc.seq = ++host_seq;
-            HIP_TRY(launch_orth_dots(d_V, ldv, k, D2, d_w, n, 0, d_dparts, d_counter, D3, stream, hc));
-            const bool next = k < m && total_before(iterOut, m, k) < maxit;
-            if (next && !prec_ready) {
-                if ((rc = gemv_A(d_w, d_w, nullptr, 0, D3, d_V + (size_t)k * ldv))) return rc;
+            // The step sends the Hessenberg column to the host.  The next
+            // basis vector is then on the device, so its product is queued
+            // before the host waits (it is discarded if this iteration ends
+            // the solve).
+            if ((rc = arnoldi(d_w, true, nullptr, d_V, k, k < m ? d_V + (size_t)k * lda : nullptr))) return rc;
+            if (k < m && total_before(iterOut, m, k) < maxit) {
+                if ((rc = matvec(k))) return rc;
                 w_ready = true;
-            } else if (k < m) {
-                HIP_TRY(launch_scale_copy(d_w, D3, 0, n, d_V + (size_t)k * ldv, stream));
-                if (next) {
-                    if ((rc = matvec(k))) return rc;
-                    w_ready = true;
-                }
             }
-            if ((rc = await_host_copy(true))) return rc;
+            if ((rc = await_arnoldi(k))) return rc;
             for (int j = 0; j < k; ++j) H[j + (size_t)jH * ldh] = h_dots[j] + h_dots[(m + 2) + j];
             const double dnormw = std::sqrt(h_dots[2 * (m + 2)]);
             H[k + (size_t)jH * ldh] = dnormw;
@@ -594,9 +633,8 @@ int rf_sim::solve_gmres(int* iters_out, double* be_out, int* status_out, int max
                 std::copy(y.begin(), y.begin() + k, h_y);
                 if ((rc = update_iterate(k))) return rc;
                 have_xc = true;
-                if ((rc = gemv_A(d_xc, d_r, d_b, 1))) return rc;
                 double rr;
-                if ((rc = norm2(d_r, &rr))) return rc;
+                if ((rc = residual_norm(d_xc, d_r, nullptr, &rr))) return rc;
                 const double be = std::sqrt(rr) / bn;
                 if (be <= tol || total >= maxit) {
                     HIP_TRY(launch_copy_vec(d_xc, d_x, n, stream));
@@ -614,15 +652,13 @@ int rf_sim::solve_gmres(int* iters_out, double* be_out, int* status_out, int max
             if ((rc = update_iterate(m))) return rc;
         }
         HIP_TRY(launch_copy_vec(d_xc, d_x, n, stream));
-        if ((rc = gemv_A(d_x, d_r, d_b, 1))) return rc;
-        if ((rc = norm2(d_r, &beta2))) return rc;
+        if ((rc = residual_norm(d_x, d_r, d_V, &beta2))) return rc;
         beta = std::sqrt(beta2);
         if (beta == 0.0) {
             *iters_out = iterOut * m;
             *be_out = 0.0;
             return RF_OK;
         }
-        HIP_TRY(launch_scale_copy(d_r, d_dots, 0, n, d_V, stream));
     }
 }
 
@@ -741,9 +777,8 @@ int rf_sim::solve_lu(double* be_out)
     if (es == 8) {
         HIP_TRY(launch_copy_vec(d_b, d_x, n, stream));
         if ((rc = lu_apply(d_x))) return rc;
-        if ((rc = gemv_A(d_x, d_r, d_b, 1))) return rc;
         double rr;
-        if ((rc = norm2(d_r, &rr))) return rc;
+        if ((rc = residual_norm(d_x, d_r, nullptr, &rr))) return rc;
         *be_out = (bn > 0.0) ? std::sqrt(rr) / bn : 0.0;
         return RF_OK;
     }
@@ -755,9 +790,8 @@ int rf_sim::solve_lu(double* be_out)
     for (int it = 0; it < 30; ++it) {
         if ((rc = lu_apply(d_r))) return rc;
         HIP_TRY(launch_axpby(n, 1.0, d_x, 1.0, d_r, d_x, stream));
-        if ((rc = gemv_A(d_x, d_r, d_b, 1))) return rc;
         double rr;
-        if ((rc = norm2(d_r, &rr))) return rc;
+        if ((rc = residual_norm(d_x, d_r, nullptr, &rr))) return rc;
         be = (bn > 0.0) ? std::sqrt(rr) / bn : 0.0;
         stats.last_gmres_iters = it + 1;
         if (be <= tol) break;
@@ -1176,9 +1210,6 @@ int rf_sim::solve_refined(int* iters_out, double* be_out)
     const int ldh = mo + 1;
     std::vector<double> H((size_t)(mo + 1) * (mo + 1)), g(mo + 1), cs(mo + 1), sn(mo + 1), y(mo + 1);
     const int m = restart;  // slot layout of d_dots (inner GMRES)
-    double* D1 = d_dots;
-    double* D2 = d_dots + (m + 2);
-    double* D3 = d_dots + 2 * (m + 2);
     int total = 0, outer = 0;
     double be = 0.0;
     // the FP64 residual b - A x; ||r||^2 stays in d_dots[0] for the scaling
@@ -1238,11 +1269,8 @@ int rf_sim::solve_refined(int* iters_out, double* be_out)
             HIP_TRY(launch_copy_vec(d_dx, zj, n, stream));
             if ((rc = apply_operator(kOpAx, zj, d_fw))) return rc;
             k = j + 1;
-            HIP_TRY(launch_multidot(d_fV, lda, k, d_fw, n, d_dparts, d_counter, D1, stream));
-            HIP_TRY(launch_orth_dots(d_fV, lda, k, D1, d_fw, n, 1, d_dparts, d_counter, D2, stream));
-            HIP_TRY(launch_orth_dots(d_fV, lda, k, D2, d_fw, n, 0, d_dparts, d_counter, D3, stream));
-            if (k < mo) HIP_TRY(launch_scale_copy(d_fw, D3, 0, n, d_fV + (size_t)k * lda, stream));
-            if ((rc = fetch_dots(3 * (m + 2)))) return rc;
+            if ((rc = arnoldi(d_fw, false, nullptr, d_fV, k, k < mo ? d_fV + (size_t)k * lda : nullptr))) return rc;
+            if ((rc = await_arnoldi(k))) return rc;
             for (int i = 0; i < k; ++i) H[i + (size_t)j * ldh] = h_dots[i] + h_dots[(m + 2) + i];
             H[k + (size_t)j * ldh] = std::sqrt(h_dots[2 * (m + 2)]);
             for (int i = 0; i < j; ++i) rot1(&H[i + (size_t)j * ldh], &H[i + 1 + (size_t)j * ldh], cs[i], sn[i]);

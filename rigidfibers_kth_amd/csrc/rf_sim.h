@@ -80,9 +80,11 @@ struct rf_sim {
     double* d_fZ = nullptr;  // [outer_m][lda]
     double* d_fw = nullptr;  // [lda]
     double* h_dots = nullptr;  // pinned; its last double holds the copy's sequence word
+    unsigned long long* d_slots = nullptr;  // of the Arnoldi steps
+    int arn_set = 0;           // the next one's set of slots
     unsigned host_seq = 0;     // sequence number of the last copy into h_dots
     unsigned* host_seq_word() const { return reinterpret_cast<unsigned*>(h_dots + 3 * (restart + 2) + 7); }
-    int await_host_copy(bool poll = false);
+    int await_host_copy();
     double* h_y = nullptr;     // pinned
     // neighbourhoods and preconditioner (allocated on first use)
     int knn = 0;           // neighbours kept per fiber
@@ -141,10 +143,14 @@ struct rf_sim {
     int update_velocities();
     int advance();
     int step();
-    // y = A x (mode 0) or b - A x (mode 1); with x_nrm2, A (x / sqrt(*x_nrm2))
-    // and the scaled vector stored to x_out
-    int gemv_A(const double* x, double* y, const double* b, int mode, const double* x_nrm2 = nullptr,
-               double* x_out = nullptr);
+    // y = A x (mode 0) or b - A x (mode 1); y == nullptr: the partial sums stay in d_gparts
+    int gemv_A(const double* x, double* y, const double* b, int mode);
+    // queues an Arnoldi step on w (the partial sums in d_gparts with `product`,
+    // b minus them with b); its scalars are in h_dots after await_arnoldi
+    int await_arnoldi(int k);
+    int arnoldi(double* w, bool product, const double* b, double* V, int k, double* v_next);
+    // r = b - A x and |r|^2 (in d_dots[0] too); v (when not null) = r / |r|
+    int residual_norm(const double* x, double* r, double* v, double* rr);
     int fetch_dots(int count);
     int norm2(const double* v, double* out);
     int solve_gmres(int* iters, double* be, int* status, int maxit);
