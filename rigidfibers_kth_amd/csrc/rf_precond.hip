@@ -9,12 +9,13 @@
 // C_i = {i} + its K nearest fibers is solved exactly:
 //     z_i = [ (A_{C_i C_i})^{-1} r_{C_i} ]_i
 // The 3M rows of the cluster inverse that belong to fiber i are precomputed
-// once per assembly (Gauss-Jordan in LDS, one workgroup per fiber), so one
-// application is a gather + small dense product per fiber.
+// once per assembly (Gauss-Jordan in registers, one workgroup per fiber), so
+// one application is a gather + small dense product per fiber.
 #include "rf_internal.h"
 #include "rf_precond.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace rf {
 namespace {
@@ -112,119 +113,203 @@ __global__ void __launch_bounds__(256) knn_kernel(int N, int K, const double* __
     }
 }
 
-// One workgroup per fiber: Gauss-Jordan with partial pivoting on the
-// transposed cluster matrix augmented with the first 3M unit vectors, which
-// leaves in the augmented columns the rows of A_CC^{-1} that belong to fiber
-// i.  B[i] is stored as [dim][bs] (bs = 3M, dim = bs (K+1)).
-template <typename T>
-__global__ void __launch_bounds__(256) ras_setup_kernel(int N, int K, int ldn, int bs, const int* __restrict__ nbr,
-                                                        const T* __restrict__ A, int64_t lda,
-                                                        double* __restrict__ B, int* __restrict__ info)
+// The largest key of the wavefront, in every lane.
+__device__ __forceinline__ unsigned long long wave_max(unsigned long long v)
 {
-    extern __shared__ double sm[];
-    const int dim = bs * (K + 1);
-    const int ldm = dim + bs + 1;  // row stride: dim columns + bs augmented + pad
-    double* Mt = sm;               // [dim][ldm]
-    __shared__ int fib[16];
-    __shared__ int piv;
-    __shared__ double pivval;
-    const int i = blockIdx.x;
-    if (threadIdx.x == 0) {
-        fib[0] = i;
-        for (int c = 0; c < K; ++c) fib[c + 1] = nbr[(size_t)i * ldn + c];
-    }
-    __syncthreads();
-    // Mt[r][c] = A_CC[c][r]; cluster row/col q -> global (fib[q/bs]*bs + q%bs)
-    for (int e = threadIdx.x; e < dim * dim; e += blockDim.x) {
-        const int rr = e % dim, cc = e / dim;  // A_CC row rr, column cc
-        const int64_t grow = (int64_t)fib[rr / bs] * bs + rr % bs;
-        const int64_t gcol = (int64_t)fib[cc / bs] * bs + cc % bs;
-        Mt[cc * ldm + rr] = (double)A[gcol * lda + grow];
-    }
-    for (int e = threadIdx.x; e < dim * bs; e += blockDim.x) {
-        const int rr = e / bs, q = e % bs;
-        Mt[rr * ldm + dim + q] = (rr == q) ? 1.0 : 0.0;
-    }
-    __syncthreads();
-    const int W = dim + bs;
-    for (int k = 0; k < dim; ++k) {
-        if (threadIdx.x < 64) {
-            double best = -1.0;
-            int bi = dim;
-            for (int r = k + threadIdx.x; r < dim; r += 64) {
-                const double v = fabs(Mt[r * ldm + k]);
-                if (v > best) {
-                    best = v;
-                    bi = r;
-                }
-            }
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                const double ov = __shfl_xor(best, off, 64);
-                const int oi = __shfl_xor(bi, off, 64);
-                if (ov > best || (ov == best && oi < bi)) {
-                    best = ov;
-                    bi = oi;
-                }
-            }
-            if (threadIdx.x == 0) piv = bi;
-        }
-        __syncthreads();
-        const int p = piv;
-        if (p != k && p < dim) {
-            for (int c = threadIdx.x; c < W; c += blockDim.x) {
-                const double t = Mt[k * ldm + c];
-                Mt[k * ldm + c] = Mt[p * ldm + c];
-                Mt[p * ldm + c] = t;
-            }
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) pivval = Mt[k * ldm + k];
-        __syncthreads();
-        const double pv = pivval;
-        if (pv == 0.0) {
-            if (threadIdx.x == 0) atomicExch(info, i + 1);
-            return;
-        }
-        const double rp = 1.0 / pv;
-        // eliminate column k from every other row; row k is scaled last
-        for (int e = threadIdx.x; e < dim * W; e += blockDim.x) {
-            const int r = e / W, c = e % W;
-            if (r == k || c == k) continue;
-            const double f = Mt[r * ldm + k] * rp;
-            Mt[r * ldm + c] -= f * Mt[k * ldm + c];
-        }
-        __syncthreads();
-        for (int r = threadIdx.x; r < dim; r += blockDim.x)
-            if (r != k) Mt[r * ldm + k] = 0.0;
-        for (int c = threadIdx.x; c < W; c += blockDim.x) Mt[k * ldm + c] *= rp;
-        __syncthreads();
-    }
-    // augmented column q = row q of A_CC^{-1}: B[i][c][q] = Mt[c][dim + q]
-    double* Bi = B + (size_t)i * dim * bs;
-    for (int e = threadIdx.x; e < dim * bs; e += blockDim.x) {
-        const int c = e / bs, q = e % bs;
-        Bi[e] = Mt[c * ldm + dim + q];
+    auto join = [](unsigned hi, unsigned lo) { return ((unsigned long long)hi << 32) | lo; };
+    auto dpp = [&](auto ctrl) {
+        constexpr int C = decltype(ctrl)::value;
+        const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)v, C, 0xf, 0xf, true);
+        const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(v >> 32), C, 0xf, 0xf, true);
+        v = max(v, join(hi, lo));
+    };
+    dpp(std::integral_constant<int, 0xB1>{});   // lane ^ 1
+    dpp(std::integral_constant<int, 0x4E>{});   // lane ^ 2
+    dpp(std::integral_constant<int, 0x141>{});  // mirrored in its eight
+    dpp(std::integral_constant<int, 0x128>{});  // lane ^ 8
+    auto lo = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+    auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(v >> 32), (unsigned)(v >> 32), false, false);
+    v = max(join(hi[0], lo[0]), join(hi[1], lo[1]));
+    lo = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+    hi = __builtin_amdgcn_permlane32_swap((unsigned)(v >> 32), (unsigned)(v >> 32), false, false);
+    return max(join(hi[0], lo[0]), join(hi[1], lo[1]));
+}
+
+// body(integral constants 0 .. N-1): register arrays are only indexed by constants
+template <int N, typename F, int I = 0>
+__device__ __forceinline__ void static_for(F&& body)
+{
+    if constexpr (I < N) {
+        body(std::integral_constant<int, I>{});
+        static_for<N, F, I + 1>(static_cast<F&&>(body));
     }
 }
 
-// z_i = B_i r_{C_i}: thread per (fiber, row q)
-__global__ void ras_apply_kernel(int N, int K, int ldn, int bs, const int* __restrict__ nbr, const double* __restrict__ B,
-                                 const double* __restrict__ r, double* __restrict__ z)
+// One workgroup per fiber: Gauss-Jordan with partial pivoting on the
+// transposed cluster matrix augmented with the first bs unit vectors, which
+// leaves in the augmented columns the rows of A_CC^{-1} that belong to fiber
+// i.  B[i] is stored as [dim][bs] (bs = 3M, dim = bs (K+1)).
+// The matrix stays in registers, element (ty + TY a, tx + TX b) in thread
+// (ty, tx) of TY x TX: a step passes only the pivot's column and row through
+// LDS and needs two barriers, the rows are not swapped (a row is its unknown's
+// once it has been the pivot row) and eliminated columns are skipped.
+// The work around a step's update (pivot search, quotient, addresses) is per
+// wavefront, so few threads with many elements each are better than 256 with
+// few, as far as registers go: 1000 clusters of 75 rows take 111 us with
+// 16 x 8 threads, 122 with 16 x 16, 154 with 8 x 8; 421 of 105 rows 161 us with
+// 16 x 16, 167 with 16 x 8.  With the matrix in LDS, every column updated in
+// every step and five barriers a step they took 932 and 1952 us.
+template <typename T, int TY, int TX, int RA, int AB>
+__global__ void __launch_bounds__(TY* TX) ras_setup_kernel(int K, int ldn, int bs, const int* __restrict__ nbr,
+                                                           const T* __restrict__ A, int64_t lda,
+                                                           double* __restrict__ B, int* __restrict__ info)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= N * bs) return;
-    const int i = t / bs, q = t - (t / bs) * bs;
-    const int dim = bs * (K + 1);
-    const double* Bi = B + (size_t)i * dim * bs + q;
-    double s = 0.0;
-    for (int c = 0; c <= K; ++c) {
-        const int f = (c == 0) ? i : nbr[(size_t)i * ldn + c - 1];
-        const double* rf = r + (size_t)f * bs;
-        const double* bc = Bi + (size_t)c * bs * bs;
-        for (int e = 0; e < bs; ++e) s += bc[(size_t)e * bs] * rf[e];
+    constexpr int DM = TY * RA, CA = DM / TX;
+    static_assert(CA * TX == DM && DM <= 128, "whole column blocks");
+    __shared__ double col[2][DM], row[DM + TX * AB], rscale[DM];
+    __shared__ int rowcol[DM];  // the unknown of a row: the step it was pivot row in
+    __shared__ int fib[kMaxRasNeighbours + 1];
+    const int dim = bs * (K + 1), i = blockIdx.x, tid = threadIdx.x;
+    const int tx = tid % TX, ty = tid / TX, lane = tid & 63;
+    if (tid <= K) fib[tid] = tid == 0 ? i : nbr[(size_t)i * ldn + tid - 1];
+    __syncthreads();
+    // x[a][b] = A_CC[c][r], r = ty + TY a, c = tx + TX b; cluster index q is
+    // global (fib[q / bs] bs + q % bs); rows past dim stay 0 and are no pivots
+    double x[RA][CA], g[RA][AB];
+    int grow[CA];
+#pragma unroll
+    for (int b = 0; b < CA; ++b) {
+        const int c = min(tx + TX * b, dim - 1);
+        grow[b] = fib[c / bs] * bs + c % bs;
     }
-    z[t] = s;
+#pragma unroll
+    for (int a = 0; a < RA; ++a) {
+        const int r = min(ty + TY * a, dim - 1);
+        const T* at = A + ((int64_t)fib[r / bs] * bs + r % bs) * lda;
+#pragma unroll
+        for (int b = 0; b < CA; ++b) {
+            const double v = (double)at[grow[b]];
+            x[a][b] = (ty + TY * a < dim && tx + TX * b < dim) ? v : 0.0;
+        }
+#pragma unroll
+        for (int b = 0; b < AB; ++b) g[a][b] = (ty + TY * a == tx + TX * b && tx + TX * b < bs) ? 1.0 : 0.0;
+    }
+    auto publish_col = [&](auto kb, int k) {
+        if (tx != k % TX) return;
+#pragma unroll
+        for (int a = 0; a < RA; ++a) col[k & 1][ty + TY * a] = x[a][decltype(kb)::value];
+    };
+    publish_col(std::integral_constant<int, 0>{}, 0);
+    bool singular = false;
+    int used = 0;  // bit q: row lane + 64 q has been pivot row
+    static_for<CA>([&](auto block) {
+        constexpr int KB = decltype(block)::value;  // columns TX KB .. of the steps
+        for (int k = TX * KB; k < min(dim, TX * KB + TX); ++k) {
+            __syncthreads();
+            // the pivot row: largest magnitude among the rows not used yet, the
+            // first of equal ones (the last 8 bits of the magnitude give way to it)
+            const double* ck = col[k & 1];
+            unsigned long long key = 0;
+#pragma unroll
+            for (int q = 0; q < (DM + 63) / 64; ++q) {
+                const int r = lane + 64 * q;
+                if (r < dim && !((used >> q) & 1)) {
+                    const unsigned long long bits = (unsigned long long)__double_as_longlong(ck[r]) & 0x7FFFFFFFFFFFFFFFull;
+                    key = max(key, (bits & ~255ull) | (unsigned)(255 - r));
+                }
+            }
+            const int p = __builtin_amdgcn_readfirstlane(255 - (int)(wave_max(key) & 255ull));
+            if (lane == (p & 63)) used |= 1 << (p >> 6);
+            const double pv = ck[p];
+            singular |= pv == 0.0;  // the same for every thread; goes on (one way out of the loop) with inf and NaN
+            const double rp = 1.0 / pv;
+            static_for<RA>([&](auto aa) {
+                constexpr int a = decltype(aa)::value;
+                if (ty + TY * a == p) {
+#pragma unroll
+                    for (int b = KB; b < CA; ++b) row[tx + TX * b] = x[a][b];
+#pragma unroll
+                    for (int b = 0; b < AB; ++b) row[DM + tx + TX * b] = g[a][b];
+                }
+            });
+            __syncthreads();
+            if (tid == 0) {
+                rowcol[p] = k;
+                rscale[p] = rp;
+            }
+            // every other row loses column k; the pivot row is scaled at the end
+            double f[RA];
+#pragma unroll
+            for (int a = 0; a < RA; ++a) f[a] = (ty + TY * a == p) ? 0.0 : ck[ty + TY * a] * rp;
+#pragma unroll
+            for (int b = KB; b < CA; ++b) {
+                const double v = row[tx + TX * b];
+#pragma unroll
+                for (int a = 0; a < RA; ++a) x[a][b] -= f[a] * v;
+            }
+#pragma unroll
+            for (int b = 0; b < AB; ++b) {
+                const double v = row[DM + tx + TX * b];
+#pragma unroll
+                for (int a = 0; a < RA; ++a) g[a][b] -= f[a] * v;
+            }
+            if (k + 1 < dim) {
+                if ((k + 1) % TX != 0)
+                    publish_col(block, k + 1);
+                else
+                    publish_col(std::integral_constant<int, (KB + 1 < CA ? KB + 1 : KB)>{}, k + 1);
+            }
+        }
+    });
+    if (singular) {
+        if (tid == 0) atomicExch(info, i + 1);
+        return;
+    }
+    __syncthreads();
+    // augmented column q of unknown c = row q of A_CC^{-1}: B[i][c][q]
+    double* Bi = B + (size_t)i * dim * bs;
+#pragma unroll
+    for (int a = 0; a < RA; ++a) {
+        const int r = ty + TY * a;
+        if (r >= dim) continue;
+        const int c = rowcol[r];
+        const double sc = rscale[r];
+#pragma unroll
+        for (int b = 0; b < AB; ++b)
+            if (tx + TX * b < bs) Bi[(size_t)c * bs + tx + TX * b] = g[a][b] * sc;
+    }
+}
+
+// z_i = B_i r_{C_i}: a workgroup per fiber, its lanes in groups of bs that take
+// every G-th cluster row, so consecutive lanes read consecutive words of B and
+// all loads of a group are in flight together.  A thread per (fiber, row of
+// B_i) is 59 workgroups at N = 1000, M = 5 and reads one row after the other.
+// N = 1000, M = 5, K = 4: 22 -> 5.4 us; N = 4000 26 -> 11 us (36 MB of B).
+constexpr int kRasApplyThreads = 256;
+__global__ void __launch_bounds__(kRasApplyThreads) ras_apply_kernel(int K, int ldn, int bs, const int* __restrict__ nbr,
+                                                                     const double* __restrict__ B,
+                                                                     const double* __restrict__ r,
+                                                                     double* __restrict__ z)
+{
+    __shared__ double part[kRasApplyThreads];
+    const int i = blockIdx.x, dim = bs * (K + 1);
+    const int G = kRasApplyThreads / bs, grp = threadIdx.x / bs, q = threadIdx.x % bs;
+    double s = 0.0;
+    if (grp < G) {
+        const double* Bi = B + (size_t)i * dim * bs + q;
+#pragma unroll 4
+        for (int c = grp; c < dim; c += G) {
+            const int m = c / bs;
+            const int f = m == 0 ? i : nbr[(size_t)i * ldn + m - 1];
+            s += Bi[(size_t)c * bs] * r[(size_t)f * bs + c % bs];
+        }
+    }
+    part[threadIdx.x] = s;
+    __syncthreads();
+    if (grp == 0) {
+        for (int h = 1; h < G; ++h) s += part[h * bs + q];
+        z[(size_t)i * bs + q] = s;
+    }
 }
 
 }  // namespace
@@ -239,31 +324,50 @@ hipError_t launch_knn(int N, int K, const double* pos, const double* orient, int
     return hipGetLastError();
 }
 
-size_t ras_setup_lds(int K, int bs)
-{
-    const int dim = bs * (K + 1);
-    return sizeof(double) * (size_t)dim * (dim + bs + 1);
-}
-
 hipError_t launch_ras_setup(int N, int K, int ldn, int bs, const int* nbr, const void* A, int elem_bytes,
                             int64_t lda, double* B, int* info, hipStream_t s)
 {
-    const size_t lds = ras_setup_lds(K, bs);
-    if (K < 1 || K > kMaxRasNeighbours || K > ldn || lds > 160 * 1024) return hipErrorInvalidValue;
-    if (elem_bytes == 8)
-        hipLaunchKernelGGL(ras_setup_kernel<double>, dim3(N), dim3(256), lds, s, N, K, ldn, bs, nbr,
-                           static_cast<const double*>(A), lda, B, info);
+    const int dim = bs * (K + 1);
+    if (K < 1 || K > kMaxRasNeighbours || K > ldn || bs < 1 || bs > 24 || dim > kMaxRasRows) return hipErrorInvalidValue;
+    // TY x TX threads with RA rows each; AB covers bs <= 16 or bs <= 24
+    auto launch = [&](auto ty, auto tx, auto ra) {
+        constexpr int TY = decltype(ty)::value, TX = decltype(tx)::value, RA = decltype(ra)::value;
+        auto go = [&](auto* At, auto ab) {
+            using T = std::remove_const_t<std::remove_pointer_t<decltype(At)>>;
+            hipLaunchKernelGGL((ras_setup_kernel<T, TY, TX, RA, decltype(ab)::value>), dim3(N), dim3(TY * TX), 0, s, K,
+                               ldn, bs, nbr, At, lda, B, info);
+        };
+        auto go_t = [&](auto* At) {
+            if (bs <= 16)
+                go(At, std::integral_constant<int, (16 + TX - 1) / TX>{});
+            else
+                go(At, std::integral_constant<int, (24 + TX - 1) / TX>{});
+        };
+        if (elem_bytes == 8)
+            go_t(static_cast<const double*>(A));
+        else
+            go_t(static_cast<const float*>(A));
+    };
+    using I8 = std::integral_constant<int, 8>;
+    using I16 = std::integral_constant<int, 16>;
+    using R4 = std::integral_constant<int, 4>;
+    if (dim <= 32)
+        launch(I8{}, I8{}, R4{});
+    else if (dim <= 64)
+        launch(I16{}, I8{}, R4{});
+    else if (dim <= 80)
+        launch(I16{}, I8{}, std::integral_constant<int, 5>{});
+    else if (dim <= 112)
+        launch(I16{}, I16{}, std::integral_constant<int, 7>{});
     else
-        hipLaunchKernelGGL(ras_setup_kernel<float>, dim3(N), dim3(256), lds, s, N, K, ldn, bs, nbr,
-                           static_cast<const float*>(A), lda, B, info);
+        launch(I16{}, I16{}, std::integral_constant<int, 8>{});
     return hipGetLastError();
 }
 
 hipError_t launch_ras_apply(int N, int K, int ldn, int bs, const int* nbr, const double* B, const double* r,
                             double* z, hipStream_t s)
 {
-    const int tot = N * bs;
-    hipLaunchKernelGGL(ras_apply_kernel, dim3((tot + 255) / 256), dim3(256), 0, s, N, K, ldn, bs, nbr, B, r, z);
+    hipLaunchKernelGGL(ras_apply_kernel, dim3(N), dim3(kRasApplyThreads), 0, s, K, ldn, bs, nbr, B, r, z);
     return hipGetLastError();
 }
 
