@@ -552,10 +552,13 @@ int rf_sim::update_iterate(int k)
 // the same iterates as the reference's modified Gram-Schmidt.  With
 // rf_params.precond the same iteration runs on A M^-1 (right preconditioning,
 // the stopping test still uses the true residual b - A x).
+// zero_guess: d_x is zero, so r0 = b without a product.  verify = false, for
+// the directions of the mixed mode's outer iteration (which measures what they
+// are worth with the FP64 operator): stop on the Arnoldi backward error alone.
 // iterations done after step k of restart cycle `cycle`
 static inline int total_before(int cycle, int m, int k) { return cycle * m + k; }
 
-int rf_sim::solve_gmres(int* iters_out, double* be_out, int* status_out, int maxit)
+int rf_sim::solve_gmres(int* iters_out, double* be_out, int* status_out, int maxit, bool zero_guess, bool verify)
 {
     const int m = restart;
     double tol = cur_tol;
@@ -575,7 +578,11 @@ int rf_sim::solve_gmres(int* iters_out, double* be_out, int* status_out, int max
     }
     // r0 = b - A x (the learned guess leaves it in d_r)
     double beta2;
-    if (r0_ready) {
+    if (zero_guess) {  // r0 = b, whose norm norm2 left in d_dots[0]
+        r0_ready = false;
+        beta2 = bn2;
+        HIP_TRY(launch_scale_copy(d_b, d_dots, 0, n, d_V, stream));
+    } else if (r0_ready) {
         r0_ready = false;
         if ((rc = norm2(d_r, &beta2))) return rc;
         HIP_TRY(launch_scale_copy(d_r, d_dots, 0, n, d_V, stream));
@@ -601,6 +608,7 @@ int rf_sim::solve_gmres(int* iters_out, double* be_out, int* status_out, int max
         std::fill(g.begin(), g.end(), 0.0);
         g[0] = beta;
         double bea = 0.0;
+        double before = beta / bn, rate = 1.0;  // the estimate and its last reduction
         bool have_xc = false;
         bool w_ready = false;  // d_gparts already holds the product for v_jH
         for (int jH = 0; jH < m; ++jH) {
@@ -609,10 +617,12 @@ int rf_sim::solve_gmres(int* iters_out, double* be_out, int* status_out, int max
             w_ready = false;
             // The step sends the Hessenberg column to the host.  The next
             // basis vector is then on the device, so its product is queued
-            // before the host waits (it is discarded if this iteration ends
-            // the solve).
+            // before the host waits, unless the reduction of the iteration
+            // before says that this one ends the solve (a product that turns
+            // out not to be needed costs its whole time, 2 ms at N = 4000; one
+            // that is queued late a round trip to the host).
             if ((rc = arnoldi(d_w, true, nullptr, d_V, k, k < m ? d_V + (size_t)k * lda : nullptr))) return rc;
-            if (k < m && total_before(iterOut, m, k) < maxit) {
+            if (k < m && total_before(iterOut, m, k) < maxit && before * rate > 2.0 * tol) {
                 if ((rc = matvec(k))) return rc;
                 w_ready = true;
             }
@@ -628,14 +638,19 @@ int rf_sim::solve_gmres(int* iters_out, double* be_out, int* status_out, int max
             bea = std::fabs(g[k]) / bn;
             const int total = iterOut * m + k;
             last_bea = bea;
+            rate = bea / before;
+            before = bea;
             if (bea <= tol || total >= maxit) {
                 hess_solve(H, ldh, g, k, y);
                 std::copy(y.begin(), y.begin() + k, h_y);
                 if ((rc = update_iterate(k))) return rc;
                 have_xc = true;
-                double rr;
-                if ((rc = residual_norm(d_xc, d_r, nullptr, &rr))) return rc;
-                const double be = std::sqrt(rr) / bn;
+                double be = bea;
+                if (verify) {
+                    double rr;
+                    if ((rc = residual_norm(d_xc, d_r, nullptr, &rr))) return rc;
+                    be = std::sqrt(rr) / bn;
+                }
                 if (be <= tol || total >= maxit) {
                     HIP_TRY(launch_copy_vec(d_xc, d_x, n, stream));
                     *iters_out = total;
@@ -1066,7 +1081,7 @@ int rf_sim::apply_operator(int mode, const double* x, double* y)
 // the relative tolerance `tol` with the configured method: the direct
 // solver, or GMRES (optionally preconditioned) with the reference's LU
 // fallback.  *be is the backward error against the stored matrix.
-int rf_sim::solve_system(int maxit, double tol, int* iters_out, double* be_out)
+int rf_sim::solve_system(int maxit, double tol, int* iters_out, double* be_out, bool direction)
 {
     int rc;
     int iters = 0, status = 0;
@@ -1095,10 +1110,10 @@ int rf_sim::solve_system(int maxit, double tol, int* iters_out, double* be_out)
         const bool lu_first = lu_factored || (auto_lu_run > 0 && auto_lu_run % kAutoRetry != 0);
         if (lu_first) {
             if ((rc = setup_precond(RF_PRECOND_LU))) return rc;
-            if ((rc = solve_gmres(&iters, &be, &status, maxit))) return rc;
+            if ((rc = solve_gmres(&iters, &be, &status, maxit, direction, !direction))) return rc;
         } else {
             if ((rc = setup_precond(RF_PRECOND_NEIGHBOUR))) return rc;
-            if ((rc = solve_gmres(&iters, &be, &status, std::min(budget, restart)))) return rc;
+            if ((rc = solve_gmres(&iters, &be, &status, std::min(budget, restart), direction, !direction))) return rc;
         }
         const double r0 = stats.last_initial_residual;
         if (!lu_first && status != 0 && iters < budget && r0 > 0.0 && be > 0.0 && be < r0) {
@@ -1106,7 +1121,7 @@ int rf_sim::solve_system(int maxit, double tol, int* iters_out, double* be_out)
             const double needed = std::log(tol / be) / std::log(rate);
             if (iters + needed <= budget) {
                 int it2 = 0;
-                if ((rc = solve_gmres(&it2, &be, &status, budget - iters))) return rc;
+                if ((rc = solve_gmres(&it2, &be, &status, budget - iters, false, !direction))) return rc;
                 iters += it2;
             }
         }
@@ -1114,13 +1129,13 @@ int rf_sim::solve_system(int maxit, double tol, int* iters_out, double* be_out)
         if (!lu_first && status != 0 && iters < maxit) {
             int it2 = 0;
             if ((rc = setup_precond(RF_PRECOND_LU))) return rc;
-            if ((rc = solve_gmres(&it2, &be, &status, maxit - iters))) return rc;
+            if ((rc = solve_gmres(&it2, &be, &status, maxit - iters, false, !direction))) return rc;
             iters += it2;
         }
         stats.last_initial_residual = r0;
     } else {
         if (p.precond != RF_PRECOND_NONE && (rc = setup_precond(p.precond))) return rc;
-        if ((rc = solve_gmres(&iters, &be, &status, maxit))) return rc;
+        if ((rc = solve_gmres(&iters, &be, &status, maxit, direction, !direction))) return rc;
         stats.last_neighbour_iters = (p.precond == RF_PRECOND_NEIGHBOUR) ? iters : 0;
     }
     stats.last_precond = prec_kind;
@@ -1259,7 +1274,7 @@ int rf_sim::solve_refined(int* iters_out, double* be_out)
             int it = 0;
             double be_in = 0.0;
             rc = launch_fill(d_x, 0.0, (size_t)n, stream) == hipSuccess ? RF_OK : RF_EHIP;
-            if (rc == RF_OK) rc = solve_system(std::max(1, maxit - total), inner_tol, &it, &be_in);
+            if (rc == RF_OK) rc = solve_system(std::max(1, maxit - total), inner_tol, &it, &be_in, true);
             std::swap(d_b, d_res64);
             std::swap(d_x, d_dx);
             if (rc) return rc;

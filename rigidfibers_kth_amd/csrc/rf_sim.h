@@ -153,8 +153,9 @@ struct rf_sim {
     int residual_norm(const double* x, double* r, double* v, double* rr);
     int fetch_dots(int count);
     int norm2(const double* v, double* out);
-    int solve_gmres(int* iters, double* be, int* status, int maxit);
-    int solve_system(int maxit, double tol, int* iters, double* be);
+    int solve_gmres(int* iters, double* be, int* status, int maxit, bool zero_guess, bool verify);
+    // direction: d_x is zero and the caller measures the result (solve_gmres)
+    int solve_system(int maxit, double tol, int* iters, double* be, bool direction = false);
     int solve_refined(int* iters, double* be);
     int apply_operator(int mode, const double* x, double* y);
     int solve_lu(double* be);
