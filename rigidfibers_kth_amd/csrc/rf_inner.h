@@ -40,6 +40,10 @@ __device__ __forceinline__ int sym6(int a, int b)
 // of the 26-step backward recurrences of the far field (double, or float in
 // mixed precision, whose error is then ~FP32 rounding of the moments).
 // BRANCH: the recurrences by c (kByDistance), or those the caller knows to apply.
+// YFIRST: which product of the three-term sums b and c is rounded first.  Near
+// a source's axis line and for |R|^2 around 10 the closed forms and recurrences
+// amplify their last bit up to 1e-6 of an entry, so the order is written out
+// and not left to the compiler's choice of fused operations.
 enum MomentBranch { kByDistance, kForward, kBackward };
 template <int M>
 struct Moments {
@@ -47,15 +51,15 @@ struct Moments {
     double I[M + 3], J[M + 3], S[M + 3];
 };
 
-template <int M, typename RB, MomentBranch BRANCH = kByDistance>
+template <int M, typename RB, MomentBranch BRANCH = kByDistance, bool YFIRST = false>
 __device__ __forceinline__ void analytic_moments(double X0, double X1, double X2, const double* xj, const double* tj,
                                                  Moments<M>& mo)
 {
     constexpr int NM = M + 3;  // moments 0..M+2
     const double r0x = X0 - xj[0], r0y = X1 - xj[1], r0z = X2 - xj[2];
     const double px = tj[0], py = tj[1], pz = tj[2];
-    const double b = -2.0 * (px * r0x + py * r0y + pz * r0z);
-    const double c = r0x * r0x + r0y * r0y + r0z * r0z;
+    const double b = -2.0 * fma(pz, r0z, YFIRST ? fma(py, r0y, px * r0x) : fma(px, r0x, py * r0y));
+    const double c = fma(r0z, r0z, YFIRST ? fma(r0y, r0y, r0x * r0x) : fma(r0x, r0x, r0y * r0y));
     const double ue = sqrt(1.0 + b + c);
     const double ub = sqrt(1.0 - b + c);
     const double d = c - 0.25 * b * b;

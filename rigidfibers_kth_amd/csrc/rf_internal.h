@@ -37,8 +37,11 @@ struct Tables {
     static constexpr int kFarClasses = 3;
     FarClass fc[kFarClasses];
     double point_c = 0.0;  // least |R|^2 of a single point for the inner nodes of class 0
-    int far_total = 0;
-    double far[704] = {0};
+    int far_total = 0;  // of the operator; the assembly's tables follow:
+    // [(n+1)/2][M+1] weights of the first half of the outer points (w_p P_k) and
+    // of the class 0 nodes (W), and [q][M+4]: s_q, w_q P_l(s_q) for l = 0..M+2
+    int asm_near = 0, asm_far = 0, asm_inner = 0;
+    double far[1344] = {0};
 };
 
 // Inner Gauss nodes of the far classes by M, and their centre distances.
@@ -55,17 +58,16 @@ struct AssembleArgs {
     int analytic = 1;
     int rhs_z_only = 1;     // analytic RHS reads only F_z (matrix_assembly.f90:857-859)
     int splits = 1;         // source splits (partial rhs slices)
-    int targets_per_block = 0;
     const double* pos = nullptr;
     const double* orient = nullptr;
     const double* force = nullptr;
     const double* wp = nullptr;   // device copy of Tables::wp
     const double* pv = nullptr;   // device copy of Tables::pv
+    const double* far = nullptr;  // device copy of Tables::far
     void* A = nullptr;            // double* (FP64) or float* (mixed)
     double* bpart = nullptr;      // [splits][n]
     void* W = nullptr;            // [3(M+1)N cols][ldw rows], double or float; nullptr: not written
     int mixed = 0;                // 1: A and W stored as float
-    double near_c = 10.0;         // mixed: (pair, point) with c < near_c computed in FP64
 };
 
 hipError_t launch_assemble(const Tables& t, const AssembleArgs& a, hipStream_t s);

@@ -24,7 +24,7 @@ namespace rf {
 static thread_local std::string g_error;
 void set_error(const std::string& msg) { g_error = msg; }
 
-int assemble_targets_per_block(int LQ, int M, bool analytic);
+int assemble_targets_per_block(int N, int LQ, int M, bool analytic);
 
 namespace {
 
@@ -130,6 +130,20 @@ void build_far_tables(Tables* t)
     // 11 inner nodes at a single point: 2e-14 from |R|^2 = 10 on for M <= 5, 7e-14 from 17 on for M = 8
     t->point_c = (M <= 5) ? 10.0 : 17.0;
     t->far_total = off;
+    const Tables::FarClass& f = t->fc[0];
+    t->asm_near = off;
+    t->asm_far = t->asm_near + (t->LQ + 1) / 2 * (M + 1);
+    t->asm_inner = t->asm_far + (f.n + 1) / 2 * (M + 1);
+    for (int k = 0; k <= M; ++k) {
+        for (int p = 0; p < (t->LQ + 1) / 2; ++p) t->far[t->asm_near + p * (M + 1) + k] = t->wp[k * t->LQ + p];
+        for (int p = 0; p < (f.n + 1) / 2; ++p) t->far[t->asm_far + p * (M + 1) + k] = t->far[f.W + k * f.n + p];
+    }
+    for (int q = 0; q < f.q; ++q) {
+        double* row = t->far + t->asm_inner + q * (M + 4);
+        row[0] = rules[f.q].x[q];
+        legendre_values(M + 2, row[0], row + 1);
+        for (int l = 0; l <= M + 2; ++l) row[1 + l] *= rules[f.q].w[q];
+    }
 }
 
 }  // namespace
@@ -1034,6 +1048,7 @@ int rf_sim::assemble()
     a.force = d_force;
     a.wp = d_wp;
     a.pv = d_pv;
+    a.far = d_far;
     a.A = d_A;
     a.W = d_W;  // nullptr in the mixed mode
     a.bpart = d_bpart;
@@ -1491,9 +1506,12 @@ extern "C" int rf_create(const rf_params* params, int32_t num_fibers, const doub
         set_error("rf_create: cannot query the device");
         return RF_EHIP;
     }
-    const int T = assemble_targets_per_block(s->LQ, s->M, P.use_analytical_integration != 0);
+    const int T = assemble_targets_per_block(s->N, s->LQ, s->M, P.use_analytical_integration != 0);
     const int tiles = (s->N + T - 1) / T;
-    s->asm_splits = std::max(1, std::min(std::min(64, s->N), (4096 + tiles - 1) / tiles));
+    // analytic: a wavefront each, eight a CU at a time, a few times over; numeric: a workgroup each
+    s->asm_splits = P.use_analytical_integration
+                        ? std::max(1, std::min(std::min(128, s->N), (8192 + tiles - 1) / tiles))
+                        : std::max(1, std::min(std::min(64, s->N), (4096 + tiles - 1) / tiles));
     const int es = s->mixed ? 4 : 8;
     s->planA = plan_gemv(s->n, s->n, s->lda, es, s->num_cus);
     s->planW = plan_gemv(6 * s->N, s->wcols, s->ldw, es, s->num_cus);
