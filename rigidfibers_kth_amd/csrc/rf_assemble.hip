@@ -19,14 +19,6 @@
 //     W = Theta_{r l} (P_0 and P_1 outer weights of
 //     fortran/coeffs_and_vels.f90:612-620,715-724), so the velocities of the
 //     step are one GEMV with [F/2, a^1..a^M] per source fiber.
-//
-// Numeric inner integrals (the analytic ones: see assemble_analytic_kernel): a
-// workgroup owns T consecutive target fibers and one range of source fibers.
-// Phase 1: thread (t,p) evaluates G_0..G_M at the
-// quadrature point p of target t and stores them in LDS.  Phase 2: thread
-// (t,l,c) contracts over p into Theta_{0..M,l,c}.  Phase 3: threads own rows
-// of A / W and write the 3M (resp. 3(M+1)) columns of source j, so each
-// column segment of T*3M consecutive rows is one coalesced store.
 #include "rf_inner.h"
 #include "rf_internal.h"
 
@@ -34,22 +26,6 @@
 
 namespace rf {
 namespace {
-
-struct KArgs {
-    int N, n, LQ, T, src_per_split;
-    int64_t lda, ldw;
-    int write_w;
-    double eps, D1;
-    double Ek[kMaxTerms + 1], gam[kMaxTerms + 1];
-    const double* pos;
-    const double* orient;
-    const double* force;
-    const double* wp;
-    const double* pv;
-    void* A;
-    void* W;
-    double* bpart;
-};
 
 // body(integral constant M)
 template <typename F>
@@ -68,172 +44,8 @@ hipError_t with_terms(int M, F&& body)
     return hipErrorInvalidValue;
 }
 
-constexpr double kNearC = 10.0;  // mixed: closer points (|R|^2) in FP64
-constexpr int kMaxItems = 8;  // A-row items per thread (3M/LQ <= 8)
-
-template <int M, bool MIXED>
-__global__ void __launch_bounds__(256, 2) assemble_numeric_kernel(const KArgs a)
-{
-    using AT = typename std::conditional<MIXED, float, double>::type;
-    constexpr int NL = M + 1;
-    extern __shared__ double smem[];
-    const int T = a.T, LQ = a.LQ, N = a.N;
-    const int gstride = LQ + 1;
-    double* sG = smem;                                    // [T*NL*6][LQ+1]
-    double* sTh = smem + (size_t)T * NL * 6 * gstride;    // [T][NL k][NL l][6]
-    double* sW = sTh + (size_t)T * NL * NL * 6;           // [LQ][NL]: w_p P_k(s_p)
-    const int tid = threadIdx.x;
-    const int nthr = blockDim.x;
-    const int i0 = blockIdx.x * T;
-    const int jb = blockIdx.y * a.src_per_split;
-    const int je = min(N, jb + a.src_per_split);
-
-    // phase-1 identity: target t1, point p1
-    const int t1 = tid / LQ, p1 = tid - (tid / LQ) * LQ;
-    const int i1 = i0 + t1;
-    const bool on1 = (t1 < T) && (i1 < N);
-    double X0 = 0, X1 = 0, X2 = 0;
-    if (on1) {
-        const double s = a.pv[p1];
-        X0 = a.pos[3 * i1 + 0] + s * a.orient[3 * i1 + 0];
-        X1 = a.pos[3 * i1 + 1] + s * a.orient[3 * i1 + 1];
-        X2 = a.pos[3 * i1 + 2] + s * a.orient[3 * i1 + 2];
-    }
-    // the Legendre weights of the Theta contraction, once per workgroup
-    for (int q = tid; q < LQ * NL; q += nthr) {
-        const int p = q / NL, k = q - p * NL;
-        sW[q] = a.wp[k * LQ + p];
-    }
-    // (the first barrier of the source loop orders these stores before the reads)
-    const int nA = T * 3 * M;          // A-row items
-    const int nItems = nA + (a.write_w ? T * 6 : 0);  // + W-row items
-    double bacc[kMaxItems];
-#pragma unroll
-    for (int s = 0; s < kMaxItems; ++s) bacc[s] = 0.0;
-
-    for (int j = jb; j < je; ++j) {
-        const double xj[3] = {a.pos[3 * j], a.pos[3 * j + 1], a.pos[3 * j + 2]};
-        const double tj[3] = {a.orient[3 * j], a.orient[3 * j + 1], a.orient[3 * j + 2]};
-        const bool act = on1 && (i1 != j);
-        // ---- phase 1: G_l at the point into LDS ----
-        if (t1 < T) {
-            double Gn[NL * 6] = {};
-            if (act) {
-                bool fp64 = true;
-                if (MIXED) {
-                    const double dx = X0 - xj[0], dy = X1 - xj[1], dz = X2 - xj[2];
-                    fp64 = (dx * dx + dy * dy + dz * dz) < kNearC;
-                }
-                if (fp64)
-                    numeric_G<M, double>(X0, X1, X2, xj, tj, a.eps, LQ, a.pv, a.wp, Gn);
-                else
-                    numeric_G<M, float>(X0, X1, X2, xj, tj, a.eps, LQ, a.pv, a.wp, Gn);
-            }
-#pragma unroll
-            for (int q = 0; q < NL * 6; ++q) sG[(size_t)(t1 * NL * 6 + q) * gstride + p1] = Gn[q];
-        }
-        __syncthreads();
-        // ---- phase 2: Theta_{k l c} = sum_p w_p P_k(s_p) G_{l c}(p) ----
-        for (int it = tid; it < T * NL * 6; it += nthr) {
-            const int t = it / (NL * 6), rem = it - t * (NL * 6);
-            const int l = rem / 6, c = rem - l * 6;
-            const double* gr = sG + (size_t)it * gstride;
-            double acc[NL];
-#pragma unroll
-            for (int k = 0; k < NL; ++k) acc[k] = 0.0;
-            for (int p = 0; p < LQ; ++p) {
-                const double gp = gr[p];
-                const double* wk = sW + p * NL;
-#pragma unroll
-                for (int k = 0; k < NL; ++k) acc[k] += wk[k] * gp;
-            }
-#pragma unroll
-            for (int k = 0; k < NL; ++k) sTh[((t * NL + k) * NL + l) * 6 + c] = acc[k];
-        }
-        __syncthreads();
-        // ---- phase 3: A rows, W rows, rhs partials ----
-        int slot = 0;
-        for (int it = tid; it < nItems; it += nthr, ++slot) {
-            if (it < nA) {
-                const int t = it / (3 * M), rem = it - t * (3 * M);
-                const int i = i0 + t;
-                if (i >= N) continue;
-                const int k = rem / 3 + 1, ar = rem - (rem / 3) * 3;
-                const double ti[3] = {a.orient[3 * i], a.orient[3 * i + 1], a.orient[3 * i + 2]};
-                const int64_t row = (int64_t)i * 3 * M + rem;
-                AT* A = reinterpret_cast<AT*>(a.A);
-                if (i == j) {
-#pragma unroll 1
-                    for (int l = 1; l <= M; ++l)
-#pragma unroll
-                        for (int bc = 0; bc < 3; ++bc) {
-                            const int64_t col = (int64_t)j * 3 * M + (l - 1) * 3 + bc;
-                            __builtin_nontemporal_store((AT)((k == l && ar == bc) ? 1.0 : 0.0), &A[col * a.lda + row]);
-                        }
-                    continue;
-                }
-                const double* th = sTh + (size_t)(t * NL + k) * NL * 6;
-                const double Ek = a.Ek[k], gk = a.gam[k];
-#pragma unroll 1
-                for (int l = 1; l <= M; ++l) {
-                    const double* tl = th + l * 6;
-#pragma unroll
-                    for (int bc = 0; bc < 3; ++bc) {
-                        const double Qb = tl[sym6(bc, 0)] * ti[0] + tl[sym6(bc, 1)] * ti[1] + tl[sym6(bc, 2)] * ti[2];
-                        const double v = (k == 1) ? a.D1 * ti[ar] * Qb : gk * (tl[sym6(ar, bc)] - Ek * ti[ar] * Qb);
-                        const int64_t col = (int64_t)j * 3 * M + (l - 1) * 3 + bc;
-                        __builtin_nontemporal_store((AT)v, &A[col * a.lda + row]);
-                    }
-                }
-                // rhs: contr = Theta_{k0} f0_j
-                const double F0 = 0.5 * a.force[3 * j + 0];
-                const double F1 = 0.5 * a.force[3 * j + 1];
-                const double F2 = 0.5 * a.force[3 * j + 2];
-                const double* t0 = th;  // l = 0
-                double cr[3];
-#pragma unroll
-                for (int cc = 0; cc < 3; ++cc)
-                    cr[cc] = t0[sym6(cc, 0)] * F0 + t0[sym6(cc, 1)] * F1 + t0[sym6(cc, 2)] * F2;
-                const double tdc = ti[0] * cr[0] + ti[1] * cr[1] + ti[2] * cr[2];
-                const double db = (k == 1) ? a.D1 * tdc * ti[ar] : gk * (cr[ar] - Ek * tdc * ti[ar]);
-#pragma unroll
-                for (int s = 0; s < kMaxItems; ++s)
-                    if (s == slot) bacc[s] -= db;
-            } else {
-                const int u = it - nA;
-                const int t = u / 6, r6 = u - t * 6;
-                const int i = i0 + t;
-                if (i >= N) continue;
-                const int r = r6 / 3, c = r6 - r * 3;
-                const int64_t row = (int64_t)i * 6 + r6;
-                AT* W = reinterpret_cast<AT*>(a.W);
-                const double* th = sTh + (size_t)(t * NL + r) * NL * 6;
-#pragma unroll 1
-                for (int l = 0; l <= M; ++l)
-#pragma unroll
-                    for (int c2 = 0; c2 < 3; ++c2) {
-                        const int64_t col = (int64_t)j * 3 * NL + l * 3 + c2;
-                        __builtin_nontemporal_store((AT)((i == j) ? 0.0 : th[l * 6 + sym6(c, c2)]), &W[col * a.ldw + row]);
-                    }
-            }
-        }
-    }
-    // rhs partial of this source split
-    int slot = 0;
-    for (int it = tid; it < nA; it += nthr, ++slot) {
-        const int t = it / (3 * M), rem = it - t * (3 * M);
-        const int i = i0 + t;
-        if (i >= N) continue;
-        double v = 0.0;
-#pragma unroll
-        for (int s = 0; s < kMaxItems; ++s)
-            if (s == slot) v = bacc[s];
-        a.bpart[(size_t)blockIdx.y * a.n + (size_t)i * 3 * M + rem] = v;
-    }
-}
-
 // ---------------------------------------------------------------------------
-// Analytic inner integrals.  A wavefront (its own workgroup) owns up to kTW
+// A wavefront (its own workgroup) owns up to kTW
 // consecutive targets and a range of sources.  For a source it sorts the
 // targets into near and far pairs (the operator's first far class: centres 4.2
 // apart, 5.2 for M > 5, and not within 0.1 of the source's axis line) and takes
@@ -241,9 +53,11 @@ __global__ void __launch_bounds__(256, 2) assemble_numeric_kernel(const KArgs a)
 // outer points h and n-1-h of a pair.
 //   * near: the closed-form moments at the n = LQ points;
 //   * far: 11 Gauss nodes on the source, n = 14 outer nodes with the weights
-//     that stand for the composite rule.
-// Either way the lane has G_l = al_l I + be_l R0 R0^T + ga_l (t R0^T + R0 t^T)
-// + de_l t t^T.  Two l at a time the 6 components go to LDS as G(h) +- G(n-1-h)
+//     that stand for the composite rule;
+//   * numeric inner integrals: every pair is near, with the LQ-point rule on
+//     the source.
+// Each way the lane has G_l = al_l I + be_l V V^T + ga_l (t V^T + V t^T)
+// + de_l t t^T, V = R0 or (numeric) its part across t.  Two l at a time the 6 components go to LDS as G(h) +- G(n-1-h)
 // (P_k is even or odd, so each k needs one of the two: half the products), a
 // lane per (pair, l, c) contracts them over h with weights in scalar registers,
 // and a lane per (pair, l, k) writes the 9 entries of A, and of W for k = 0, 1.
@@ -275,6 +89,7 @@ struct AKArgs {
     const double* near_w;     // [H][M+1]: w_p P_k(s_p) of the first half of the points
     const double* far_w;      // [H][M+1]
     const double* inner;      // [far_q][M+4]: s_q, w_q P_l(s_q) for l = 0..M+2
+    const double* numeric;    // [LQ][M+2]: s_q, w_q P_l(s_q)
     void* A;
     void* W;
     double* bpart;
@@ -348,6 +163,54 @@ __device__ __forceinline__ void far_coefficients(const double (&R0)[3], const do
     }
 }
 
+// Numeric inner integrals (fortran/quadrature.f90:121-155) at two points:
+// with R(s) = V + (h - s) t, |R|^2 = |V|^2 + (h - s)^2 keeps its relative
+// accuracy where the fibers come close.  43 operations a point and node in
+// place of 64 with the six components accumulated, and one read of the node's
+// weights (scalar registers) for both points: N = 333, M = 5, LQ = 24 510 -> 203 us
+// with the wavefront's other steps.
+template <int M>
+__device__ __forceinline__ void numeric_coefficients(double (&R1)[3], double (&R2)[3], const double* tj, double e2,
+                                                     double e6, int LQ, const_ptr table, double (&c1)[4][M + 1],
+                                                     double (&c2)[4][M + 1])
+{
+    double h[2], d[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        double(&R)[3] = p ? R2 : R1;
+        h[p] = tj[0] * R[0] + tj[1] * R[1] + tj[2] * R[2];
+#pragma unroll
+        for (int x = 0; x < 3; ++x) R[x] -= h[p] * tj[x];
+        d[p] = R[0] * R[0] + R[1] * R[1] + R[2] * R[2];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int l = 0; l <= M; ++l) c1[e][l] = c2[e][l] = 0.0;
+    for (int q = 0; q < LQ; ++q) {
+        const_ptr row = table + q * (M + 2);
+        const double s = row[0];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            double(&co)[4][M + 1] = p ? c2 : c1;
+            const double u = h[p] - s, x = fma(u, u, d[p]);
+            const double y = __builtin_amdgcn_rsq(x);
+            const double e = fma(-x * y, y, 1.0);
+            const double inv = fma(y * e, fma(e, 0.375, 0.5), y);
+            const double inv2 = inv * inv, inv3 = inv2 * inv;
+            const double dg = inv + e2 * inv3, of = inv3 - e6 * inv3 * inv2;
+            const double of1 = of * u, of2 = of1 * u;
+#pragma unroll
+            for (int l = 0; l <= M; ++l) {
+                co[0][l] += row[1 + l] * dg;
+                co[1][l] += row[1 + l] * of;
+                co[2][l] += row[1 + l] * of1;
+                co[3][l] += row[1 + l] * of2;
+            }
+        }
+    }
+}
+
 // LDS written by some lanes of the wavefront is read by others
 __device__ __forceinline__ void wave_fence()
 {
@@ -369,8 +232,8 @@ __device__ __forceinline__ void store3(float* p, double x, double y, double z)
     p[2] = (float)z;
 }
 
-template <int M, typename AT>
-__global__ void __launch_bounds__(64, 2) assemble_analytic_kernel(const AKArgs a)
+template <int M, typename AT, bool NUMERIC>
+__global__ void __launch_bounds__(64, 2) assemble_kernel(const AKArgs a)
 {
     constexpr int NL = M + 1, NCH = (NL + 1) / 2;
     typedef double d2 __attribute__((ext_vector_type(2)));
@@ -427,7 +290,7 @@ __global__ void __launch_bounds__(64, 2) assemble_analytic_kernel(const AKArgs a
             const double dt = dx * g[3] + dy * g[4] + dz * g[5];
             const double aq = 1.0 - tl * tl, bq = dt - dl * tl, cq = D2 - dl * dl;
             const double s = (aq > 1e-12) ? fmin(1.0, fmax(-1.0, -bq / aq)) : 0.0;
-            cls = (D2 >= a.far_dist2 && cq + s * (2.0 * bq + s * aq) >= 1e-2) ? 1 : 0;
+            cls = (!NUMERIC && D2 >= a.far_dist2 && cq + s * (2.0 * bq + s * aq) >= 1e-2) ? 1 : 0;
         }
         int count[2];
 #pragma unroll
@@ -446,7 +309,7 @@ __global__ void __launch_bounds__(64, 2) assemble_analytic_kernel(const AKArgs a
                 for (int e = lane; e < 18 * NL; e += 64)
                     W[((int64_t)j * 3 * NL + e / 6) * a.ldw + (int64_t)j * 6 + e % 6] = (AT)0.0;
         }
-        for (int f = 0; f < 2; ++f) {
+        for (int f = 0; f < (NUMERIC ? 1 : 2); ++f) {
             const int Hf = f ? H[1] : H[0];
             const int slot = f ? slot_of[1] : slot_of[0], h = f ? h_of[1] : h_of[0];
             const int stride = 2 * Hf + ((Hf & 1) ? 4 : 2);  // an odd number of 16-byte words
@@ -459,10 +322,12 @@ __global__ void __launch_bounds__(64, 2) assemble_analytic_kernel(const AKArgs a
                 const double s1 = f ? node1[1] : node1[0], s2 = f ? node2[1] : node2[0];
                 const double X1[3] = {g[0] + s1 * g[3], g[1] + s1 * g[4], g[2] + s1 * g[5]};
                 const double X2[3] = {g[0] + s2 * g[3], g[1] + s2 * g[4], g[2] + s2 * g[5]};
-                const double R1[3] = {X1[0] - xj[0], X1[1] - xj[1], X1[2] - xj[2]};
-                const double R2[3] = {X2[0] - xj[0], X2[1] - xj[1], X2[2] - xj[2]};
+                double R1[3] = {X1[0] - xj[0], X1[1] - xj[1], X1[2] - xj[2]};
+                double R2[3] = {X2[0] - xj[0], X2[1] - xj[1], X2[2] - xj[2]};
                 double c1[4][NL], c2[4][NL];
-                if (f == 0) {
+                if constexpr (NUMERIC) {
+                    numeric_coefficients<M>(R1, R2, tj, e2, e6, LQ, (const_ptr)a.numeric, c1, c2);
+                } else if (f == 0) {
                     near_coefficients<M, AT>(X1, xj, tj, e2, e6, c1);
                     near_coefficients<M, AT>(X2, xj, tj, e2, e6, c2);
                 } else {
@@ -586,79 +451,21 @@ __global__ void __launch_bounds__(64, 2) assemble_analytic_kernel(const AKArgs a
 
 }  // namespace
 
-static size_t numeric_lds_bytes(int T, int LQ, int M)
+int assemble_targets(int N)
 {
-    const size_t NL = M + 1;
-    return sizeof(double) * ((size_t)T * NL * 6 * (LQ + 1) + (size_t)T * NL * NL * 6 + (size_t)LQ * NL);
-}
-
-int assemble_targets_per_block(int N, int LQ, int M, bool analytic)
-{
-    if (analytic)  // fewer where the pairs are too few for two fillings of all wavefronts (N = 100: 54 -> 29 us)
-        return 5 * (int)std::min<int64_t>(kTW / 5, std::max<int64_t>(1, (int64_t)N * N / (5 * 2 * 2048)));
-    // T*LQ threads; prefer a whole number of 64-wide wavefronts <= 256 whose
-    // LDS fits in the 160 KiB of a CU.
-    const size_t cap = 160 * 1024;
-    for (int thr = 256; thr >= 64; thr -= 64)
-        if (thr % LQ == 0 && numeric_lds_bytes(thr / LQ, LQ, M) <= cap) return thr / LQ;
-    int T = std::max(1, 256 / LQ);
-    while (T > 1 && numeric_lds_bytes(T, LQ, M) > cap) --T;
-    return T;
-}
-
-static hipError_t launch_numeric(const Tables& t, const AssembleArgs& a, hipStream_t s)
-{
-    const int M = t.M, LQ = t.LQ;
-    const int T = assemble_targets_per_block(a.N, LQ, M, false);
-    const int threads = T * LQ;
-    if (threads > 1024 || T * 3 * M > kMaxItems * threads) return hipErrorInvalidValue;
-    KArgs k;
-    k.N = a.N;
-    k.n = a.n;
-    k.LQ = LQ;
-    k.T = T;
-    k.src_per_split = (a.N + a.splits - 1) / a.splits;
-    k.lda = a.lda;
-    k.ldw = a.ldw;
-    k.write_w = (a.W != nullptr) ? 1 : 0;
-    k.eps = t.eps;
-    k.D1 = t.D1;
-    for (int i = 0; i <= kMaxTerms; ++i) {
-        k.Ek[i] = t.Ek[i];
-        k.gam[i] = t.gammak[i];
-    }
-    k.pos = a.pos;
-    k.orient = a.orient;
-    k.force = a.force;
-    k.wp = a.wp;
-    k.pv = a.pv;
-    k.A = a.A;
-    k.W = a.W;
-    k.bpart = a.bpart;
-    const size_t lds = numeric_lds_bytes(T, LQ, M);
-    if (lds > 160 * 1024) return hipErrorInvalidValue;
-    const dim3 grid((a.N + T - 1) / T, a.splits);
-    auto launch = [&](auto mm) {
-        constexpr int MM = decltype(mm)::value;
-        if (a.mixed)
-            hipLaunchKernelGGL((assemble_numeric_kernel<MM, true>), grid, dim3(threads), lds, s, k);
-        else
-            hipLaunchKernelGGL((assemble_numeric_kernel<MM, false>), grid, dim3(threads), lds, s, k);
-        return hipGetLastError();
-    };
-    return with_terms(M, launch);
+    // fewer where the pairs are too few for two fillings of all wavefronts (N = 100: 54 -> 29 us)
+    return 5 * (int)std::min<int64_t>(kTW / 5, std::max<int64_t>(1, (int64_t)N * N / (5 * 2 * 2048)));
 }
 
 hipError_t launch_assemble(const Tables& t, const AssembleArgs& a, hipStream_t s)
 {
-    if (!a.analytic) return launch_numeric(t, a, s);
     AKArgs k;
     k.N = a.N;
     k.n = a.n;
     k.LQ = t.LQ;
-    k.targets = assemble_targets_per_block(a.N, t.LQ, t.M, true);
+    k.targets = assemble_targets(a.N);
     k.src_per_split = (a.N + a.splits - 1) / a.splits;
-    k.rhs_z_only = a.rhs_z_only;
+    k.rhs_z_only = a.analytic ? a.rhs_z_only : 0;
     k.lda = a.lda;
     k.ldw = a.ldw;
     k.eps = t.eps;
@@ -678,16 +485,21 @@ hipError_t launch_assemble(const Tables& t, const AssembleArgs& a, hipStream_t s
     k.near_w = a.far + t.asm_near;
     k.far_w = a.far + t.asm_far;
     k.inner = a.far + t.asm_inner;
+    k.numeric = a.far + t.asm_numeric;
     k.A = a.A;
     k.W = a.W;
     k.bpart = a.bpart;
     const dim3 grid((a.N + k.targets - 1) / k.targets, a.splits);
     auto launch = [&](auto mm) {
         constexpr int MM = decltype(mm)::value;
-        if (a.mixed)
-            hipLaunchKernelGGL((assemble_analytic_kernel<MM, float>), grid, dim3(64), 0, s, k);
+        if (a.analytic && a.mixed)
+            hipLaunchKernelGGL((assemble_kernel<MM, float, false>), grid, dim3(64), 0, s, k);
+        else if (a.analytic)
+            hipLaunchKernelGGL((assemble_kernel<MM, double, false>), grid, dim3(64), 0, s, k);
+        else if (a.mixed)
+            hipLaunchKernelGGL((assemble_kernel<MM, float, true>), grid, dim3(64), 0, s, k);
         else
-            hipLaunchKernelGGL((assemble_analytic_kernel<MM, double>), grid, dim3(64), 0, s, k);
+            hipLaunchKernelGGL((assemble_kernel<MM, double, true>), grid, dim3(64), 0, s, k);
         return hipGetLastError();
     };
     return with_terms(t.M, launch);

@@ -1,8 +1,6 @@
 // rf_inner.h -- device math shared by the assembly kernel and the
-// matrix-free operator: the Legendre monomial coefficients, the analytic
-// moments I, J, S of the inner integral (fortran/Int_analytical.f90:5-293),
-// the G_l tensor built from them (fortran/Int_analytical.f90:663-767) and the
-// numeric inner integrals (fortran/quadrature.f90:100-164).
+// matrix-free operator: the Legendre monomial coefficients and the analytic
+// moments I, J, S of the inner integral (fortran/Int_analytical.f90:5-293).
 #pragma once
 
 #include "rf_internal.h"
@@ -125,75 +123,6 @@ __device__ __forceinline__ void analytic_moments(double X0, double X1, double X2
     mo.px = px;
     mo.py = py;
     mo.pz = pz;
-}
-
-// G_l from the moments: the Legendre combinations L11..L24 of
-// Int_analytical.f90:213-288 and the tensor of :735-736, regrouped as
-// G = al I + be R0 R0^T + ga (t R0^T + R0 t^T) + de t t^T.
-template <int M>
-__device__ __forceinline__ void analytic_Gl(const Moments<M>& mo, int l, double e2, double e6, double (&g)[6])
-{
-    double L11 = 0, L12 = 0, L13 = 0, L14 = 0, L22 = 0, L23 = 0, L24 = 0;
-#pragma unroll
-    for (int m = 0; m <= kMaxTerms; ++m) {
-        if (m <= l && kLeg[l][m] != 0.0) {
-            const double cf = kLeg[l][m];
-            L11 += cf * mo.I[m];
-            L12 += cf * mo.J[m];
-            L13 += cf * mo.J[m + 1];
-            L14 += cf * mo.J[m + 2];
-            L22 += cf * mo.S[m];
-            L23 += cf * mo.S[m + 1];
-            L24 += cf * mo.S[m + 2];
-        }
-    }
-    const double al = L11 + e2 * L12;
-    const double be = L12 - e6 * L22;
-    const double ga = e6 * L23 - L13;
-    const double de = L14 - e6 * L24;
-    const double rx = mo.r0x, ry = mo.r0y, rz = mo.r0z, px = mo.px, py = mo.py, pz = mo.pz;
-    g[0] = al + be * rx * rx + 2.0 * ga * px * rx + de * px * px;
-    g[1] = al + be * ry * ry + 2.0 * ga * py * ry + de * py * py;
-    g[2] = al + be * rz * rz + 2.0 * ga * pz * rz + de * pz * pz;
-    g[3] = be * rx * ry + ga * (px * ry + rx * py) + de * px * py;
-    g[4] = be * rx * rz + ga * (px * rz + rx * pz) + de * px * pz;
-    g[5] = be * ry * rz + ga * (py * rz + ry * pz) + de * py * pz;
-}
-
-// Numeric inner integrals (fortran/quadrature.f90:121-155): LQ-point sum of
-// the kernel times w_q P_l(s_q) over fiber j.
-template <int M, typename R>
-__device__ __forceinline__ void numeric_G(double X0, double X1, double X2, const double* xj, const double* tj,
-                                          double eps, int LQ, const double* __restrict__ pv,
-                                          const double* __restrict__ wp, double (&G)[(M + 1) * 6])
-{
-    R acc[(M + 1) * 6];
-#pragma unroll
-    for (int q = 0; q < (M + 1) * 6; ++q) acc[q] = 0;
-    const R e2 = R(2.0 * eps * eps), e6 = R(6.0 * eps * eps);
-    const double bx = X0 - xj[0], by = X1 - xj[1], bz = X2 - xj[2];
-    for (int q = 0; q < LQ; ++q) {
-        const double s = pv[q];
-        const R rx = (R)(bx - tj[0] * s), ry = (R)(by - tj[1] * s), rz = (R)(bz - tj[2] * s);
-        const R r2 = rx * rx + ry * ry + rz * rz;
-        const R inv = R(1) / sqrt(r2);
-        const R inv2 = inv * inv, inv3 = inv * inv2, inv5 = inv3 * inv2;
-        const R dg = inv + e2 * inv3, of = inv3 - e6 * inv5;
-        const R K0 = dg + of * rx * rx, K1 = dg + of * ry * ry, K2 = dg + of * rz * rz;
-        const R K3 = of * rx * ry, K4 = of * rx * rz, K5 = of * ry * rz;
-#pragma unroll
-        for (int l = 0; l <= M; ++l) {
-            const R w = (R)wp[l * LQ + q];
-            acc[l * 6 + 0] += w * K0;
-            acc[l * 6 + 1] += w * K1;
-            acc[l * 6 + 2] += w * K2;
-            acc[l * 6 + 3] += w * K3;
-            acc[l * 6 + 4] += w * K4;
-            acc[l * 6 + 5] += w * K5;
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < (M + 1) * 6; ++q) G[q] = (double)acc[q];
 }
 
 }  // namespace

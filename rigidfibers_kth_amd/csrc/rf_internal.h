@@ -39,9 +39,10 @@ struct Tables {
     double point_c = 0.0;  // least |R|^2 of a single point for the inner nodes of class 0
     int far_total = 0;  // of the operator; the assembly's tables follow:
     // [(n+1)/2][M+1] weights of the first half of the outer points (w_p P_k) and
-    // of the class 0 nodes (W), and [q][M+4]: s_q, w_q P_l(s_q) for l = 0..M+2
-    int asm_near = 0, asm_far = 0, asm_inner = 0;
-    double far[1344] = {0};
+    // of the class 0 nodes (W), [q][M+4]: s_q, w_q P_l(s_q) for l = 0..M+2, and
+    // [LQ][M+2]: the LQ-point rule's s_q, w_q P_l(s_q)
+    int asm_near = 0, asm_far = 0, asm_inner = 0, asm_numeric = 0;
+    double far[2304] = {0};
 };
 
 // Inner Gauss nodes of the far classes by M, and their centre distances.

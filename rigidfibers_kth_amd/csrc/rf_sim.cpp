@@ -24,7 +24,7 @@ namespace rf {
 static thread_local std::string g_error;
 void set_error(const std::string& msg) { g_error = msg; }
 
-int assemble_targets_per_block(int N, int LQ, int M, bool analytic);
+int assemble_targets(int N);
 
 namespace {
 
@@ -143,6 +143,12 @@ void build_far_tables(Tables* t)
         row[0] = rules[f.q].x[q];
         legendre_values(M + 2, row[0], row + 1);
         for (int l = 0; l <= M + 2; ++l) row[1 + l] *= rules[f.q].w[q];
+    }
+    t->asm_numeric = t->asm_inner + f.q * (M + 4);
+    for (int q = 0; q < t->LQ; ++q) {
+        double* row = t->far + t->asm_numeric + q * (M + 2);
+        row[0] = t->pv[q];
+        for (int l = 0; l <= M; ++l) row[1 + l] = t->wp[l * t->LQ + q];
     }
 }
 
@@ -1506,12 +1512,10 @@ extern "C" int rf_create(const rf_params* params, int32_t num_fibers, const doub
         set_error("rf_create: cannot query the device");
         return RF_EHIP;
     }
-    const int T = assemble_targets_per_block(s->N, s->LQ, s->M, P.use_analytical_integration != 0);
+    const int T = assemble_targets(s->N);
     const int tiles = (s->N + T - 1) / T;
-    // analytic: a wavefront each, eight a CU at a time, a few times over; numeric: a workgroup each
-    s->asm_splits = P.use_analytical_integration
-                        ? std::max(1, std::min(std::min(128, s->N), (8192 + tiles - 1) / tiles))
-                        : std::max(1, std::min(std::min(64, s->N), (4096 + tiles - 1) / tiles));
+    // a wavefront each, eight a CU at a time, a few times over
+    s->asm_splits = std::max(1, std::min(std::min(128, s->N), (8192 + tiles - 1) / tiles));
     const int es = s->mixed ? 4 : 8;
     s->planA = plan_gemv(s->n, s->n, s->lda, es, s->num_cus);
     s->planW = plan_gemv(6 * s->N, s->wcols, s->ldw, es, s->num_cus);

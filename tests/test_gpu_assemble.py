@@ -84,3 +84,29 @@ def test_velocity_operator(M, noqi, N):
     tol = 1e-11 if M <= 5 else 1e-8
     assert np.abs(v - vo).max() <= tol * np.abs(vo).max()
     assert np.abs(w - wo).max() <= tol * max(np.abs(wo).max(), np.abs(vo).max())
+
+
+@pytest.mark.parametrize("precision", [rf.PREC_FP64, rf.PREC_MIXED])
+@pytest.mark.parametrize("N,M,noqi,phi", [
+    (2, 1, 1, 1e-3), (5, 2, 3, 1e-2), (6, 3, 32, 1e-2), (19, 4, 5, 2e-2), (21, 5, 8, 1e-4), (41, 6, 4, 2e-2),
+    (33, 8, 21, 1e-2), (64, 7, 11, 5e-2), (150, 5, 8, 5e-2)])
+def test_numeric_against_the_oracle(N, M, noqi, phi, precision):
+    """The same sums of the same products, so rounding alone: 1e-12 of the
+    largest entry, as the parity tests; FP32 storage 6e-8 of an entry."""
+    pos, ori = layout(N, phi, 50 + N)
+    p = rf.default_params(use_analytical_integration=0, num_terms=M, num_quad_intervals=noqi, slenderness=EPS,
+                          precision=precision, external_force=(0.2, -0.1, -1.0))
+    with rf.Simulation(rf.Configuration(p, pos, ori)) as sim:
+        sim.assemble_system()
+        A, b = sim.matrix(), sim.rhs()
+        pos, ori = (np.asarray(v).ravel() for v in sim.state()[:2])
+    Ao = oracle.assemble_matrix(0, EPS, pos, ori, M, noqi)
+    bo = oracle.assemble_rhs(0, EPS, pos, ori, np.tile([0.2, -0.1, -1.0], N), M, noqi)
+    scale = np.abs(Ao - np.eye(Ao.shape[0])).max()
+    err_b = np.abs(b - bo).max() / np.abs(bo).max()
+    print("numeric N=%d M=%d NoQI=%d: A %.2e, b %.2e" % (N, M, noqi, np.abs(A - Ao).max() / scale, err_b))
+    if precision == rf.PREC_MIXED:
+        assert np.all(np.abs(A - Ao) <= 6e-8 * np.abs(Ao) + 1e-12 * scale)
+    else:
+        assert np.abs(A - Ao).max() <= 1e-12 * scale
+    assert err_b <= 1e-12
