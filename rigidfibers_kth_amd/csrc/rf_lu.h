@@ -38,11 +38,12 @@ size_t lu_workspace_bytes(int n, int update_fp16);
 hipError_t lu_factor(void* A, int elem_bytes, int64_t lda, int n, int nb, int* ipiv, int* info, int use_mfma,
                      int block_pivot, int update_fp16, void* ws, int* redone, int* host_flag, hipStream_t s,
                      const LuSide* side = nullptr);
-// x <- U^-1 L^-1 P x with FP64 vectors, one launch per 64-row block and
-// sweep (FP32 or FP64 factors).  aux holds
+// x <- U^-1 L^-1 P x with FP64 vectors: FP64 factors one launch a sweep, FP32
+// factors two launches per 512-row block and sweep.  aux holds
 // lu_solve_aux_bytes(n, elem_bytes): the row permutation and the inverses of
-// the 64x64 diagonal blocks of L and U, filled by lu_prepare_solve once per
-// factorisation; tmp is n doubles.
+// the 64-row (FP32: 512-row) diagonal blocks of L and U, filled by
+// lu_prepare_solve once per factorisation, and scratch of the FP64 sweeps (the
+// solves that share it are on one stream); tmp is n doubles.
 size_t lu_solve_aux_bytes(int n, int elem_bytes);
 hipError_t lu_prepare_solve(const void* LU, int elem_bytes, int64_t lda, int n, const int* ipiv, void* aux,
                             hipStream_t s);

@@ -2435,11 +2435,7 @@ __global__ void mfma_probe_kernel(int mode, double* out64, float* out32)
 // ---- solves with the factors ------------------------------------------------
 // Once per factorisation the pivots become one permutation and the 64 x 64
 // diagonal blocks of L and U are inverted (one workgroup per block).
-//   FP64 factors (one solve each): each 64-row block of the forward and
-// backward sweeps is one launch, in which every workgroup forms
-// y = inv(D) v_block (4 lanes per row) and updates 64 of the remaining rows
-// (each wavefront takes 16 of the block's columns with all 16 loads in
-// flight; the 4 partial sums meet in LDS).
+//   FP64 factors: one launch a sweep (sweep_chain_kernel).
 //   FP32 factors precondition: a solve runs once per GMRES iteration, and at
 // 4 to 7 us a launch the 938 launches of n = 30000 took 5.1 ms for 3.6 GB of
 // factors.  The inverses are therefore merged to 512 x 512 diagonal blocks, and
@@ -2449,11 +2445,14 @@ __global__ void mfma_probe_kernel(int mode, double* out64, float* out32)
 // ramp of the updates.
 constexpr int kSB = 64;
 
+// y = P x; clear (when not null) to kArnoldiEmpty
 __global__ void permute_kernel(const double* __restrict__ x, const int* __restrict__ perm, int n,
-                               double* __restrict__ y)
+                               double* __restrict__ y, unsigned long long* __restrict__ clear)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) y[i] = x[perm[i]];
+    if (i >= n) return;
+    y[i] = x[perm[i]];
+    if (clear) clear[i] = kArnoldiEmpty;
 }
 
 // Element (r, q) of the inverse of diagonal block b of L (u = 0, unit lower) or
@@ -2683,50 +2682,80 @@ __global__ void __launch_bounds__(512) wide_update_kernel(const float* __restric
     }
 }
 
-// lower = 1: forward block (unit lower L), rows updated i >= k0+bs;
-// lower = 0: backward block (U), rows updated i < k0.
-template <typename T, int LOWER>
-__global__ void __launch_bounds__(256) sweep_block_kernel(const T* __restrict__ LU, int64_t lda, int n,
-                                                          const T* __restrict__ inv, double* __restrict__ v,
-                                                          double* __restrict__ out, int k0, int bs)
+// FP64 factors: a whole triangular solve in one launch.  A workgroup owns the 64
+// rows of a block: it subtracts the blocks before its own as their solutions
+// appear, multiplies by its block's inverse and publishes its 64 values.  A
+// word of the solution holds kArnoldiEmpty until its value is stored (agent
+// scope), so it needs no flag and no fence.  Workgroups are in the order of the
+// chain and wait only for earlier ones, which were dispatched before them, so
+// the first unfinished one always runs; the wait is bounded all the same (then
+// the result is NaN).  The next block's columns are loaded before the wait.
+// A launch per block took 4 us a block and sweep, and a gap as long at small n;
+// a block of the chain takes 1.5 us: n = 1500 97 -> 34 us a sweep (without the
+// gaps), n = 15000 1050 -> 380 us.
+// LOWER: L z = v (unit lower), clear emptied behind it; else U y = v.
+constexpr int kChainSpins = 1 << 22;
+template <int LOWER>
+__global__ void __launch_bounds__(256) sweep_chain_kernel(const double* __restrict__ LU, int64_t lda, int n,
+                                                          const double* __restrict__ inv, const double* __restrict__ v,
+                                                          unsigned long long* out, unsigned long long* clear)
 {
     constexpr int QW = kSB / 4;  // inverse columns per lane, block columns per wavefront
-    __shared__ double vb[kSB];
-    __shared__ double yk[kSB];
-    __shared__ double part[4][64];
+    __shared__ double part[4][kSB];
+    __shared__ double rest[kSB];
+    const int nb = gridDim.x, b = LOWER ? blockIdx.x : nb - 1 - blockIdx.x;
+    const int k0 = b * kSB, bs = min(kSB, n - k0);
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    if (t < kSB) vb[t] = (t < bs) ? v[k0 + t] : 0.0;
-    const T* X = inv + ((size_t)(k0 / kSB) * 2 + (LOWER ? 0 : 1)) * kSB * kSB;
     const int r = t >> 2, qb = (t & 3) * QW;
-    T xr[QW];
+    const double* X = inv + ((size_t)b * 2 + (LOWER ? 0 : 1)) * kSB * kSB;
+    double xr[QW];
 #pragma unroll
     for (int u = 0; u < QW; ++u) xr[u] = X[r * kSB + qb + u];
-    const int i = (LOWER ? k0 + bs : 0) + blockIdx.x * 64 + lane;
-    const int rend = LOWER ? n : k0;
-    const int q0 = wave * QW;
-    T a[QW];
-    if (i < rend) {
-        const T* li = LU + (int64_t)(k0 + q0) * lda + i;
+    const double rhs = (t < bs) ? v[k0 + t] : 0.0;
+    if (LOWER && t < bs) clear[k0 + t] = kArnoldiEmpty;
+    const bool row_in = lane < bs;
+    const double* Li = LU + k0 + (row_in ? lane : 0);
+    const int before = LOWER ? b : nb - 1 - b;
+    double a[QW], acc = 0.0;
+    auto load = [&](int q) {
+        const int c0 = (LOWER ? q : nb - 1 - q) * kSB + wave * QW;
 #pragma unroll
-        for (int u = 0; u < QW; ++u) a[u] = (q0 + u < bs) ? li[(int64_t)u * lda] : T(0);
-    }
-    __syncthreads();
-    double sum = 0.0;
+        for (int u = 0; u < QW; ++u) a[u] = (c0 + u < n) ? Li[(int64_t)(c0 + u) * lda] : 0.0;
+    };
+    if (before > 0) load(0);
+    for (int q = 0; q < before; ++q) {
+        const int c = (LOWER ? q : nb - 1 - q) * kSB + wave * QW + lane;
+        const bool want = lane < QW && c < n;
+        unsigned long long bits = kArnoldiEmpty;
+        for (int spin = 0; spin < kChainSpins; ++spin) {
+            if (want && bits == kArnoldiEmpty)
+                bits = __hip_atomic_load(&out[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (!__any(want && bits == kArnoldiEmpty)) break;
+            __builtin_amdgcn_s_sleep(1);
+        }
+        if (!want) bits = 0;
 #pragma unroll
-    for (int u = 0; u < QW; ++u) sum += (double)xr[u] * vb[qb + u];
-    sum += __shfl_xor(sum, 1, 64);
-    sum += __shfl_xor(sum, 2, 64);
-    if ((t & 3) == 0) yk[r] = sum;
-    __syncthreads();
-    if (blockIdx.x == 0 && t < bs) out[k0 + t] = yk[t];
-    double acc = 0.0;
-    if (i < rend) {
-#pragma unroll
-        for (int u = 0; u < QW; ++u) acc += (double)a[u] * yk[q0 + u];
+        for (int u = 0; u < QW; ++u) {
+            const unsigned lo = __builtin_amdgcn_readlane((unsigned)bits, u);
+            const unsigned hi = __builtin_amdgcn_readlane((unsigned)(bits >> 32), u);
+            acc += a[u] * __hiloint2double((int)hi, (int)lo);
+        }
+        if (q + 1 < before) load(q + 1);
     }
     part[wave][lane] = acc;
     __syncthreads();
-    if (wave == 0 && i < rend) v[i] -= (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+    if (t < kSB) rest[t] = (t < bs) ? rhs - ((part[0][t] + part[1][t]) + (part[2][t] + part[3][t])) : 0.0;
+    __syncthreads();
+    double sum = 0.0;
+#pragma unroll
+    for (int u = 0; u < QW; ++u) sum += xr[u] * rest[qb + u];
+    sum += __shfl_xor(sum, 1, 64);
+    sum += __shfl_xor(sum, 2, 64);
+    if ((t & 3) == 0 && r < bs) {
+        unsigned long long bits = (unsigned long long)__double_as_longlong(sum);
+        if (bits == kArnoldiEmpty) bits = 0x7FF8000000000000ull;
+        __hip_atomic_store(&out[k0 + r], bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 }
 
 }  // namespace
@@ -2765,7 +2794,8 @@ size_t lu_solve_aux_bytes(int n, int elem_bytes)
 {
     const size_t w = (elem_bytes == 4) ? kWI : kSB;  // diagonal blocks inverted as a whole
     const size_t blocks = ((size_t)n + w - 1) / w;
-    return perm_bytes(n) + blocks * 2 * w * w * (size_t)elem_bytes;
+    // FP64: and the words of L^-1 P x
+    return perm_bytes(n) + blocks * 2 * w * w * (size_t)elem_bytes + (elem_bytes == 8 ? sizeof(double) * (size_t)n : 0);
 }
 
 hipError_t lu_prepare_solve(const void* LU, int elem_bytes, int64_t lda, int n, const int* ipiv, void* aux,
@@ -2803,32 +2833,25 @@ hipError_t lu_prepare_solve(const void* LU, int elem_bytes, int64_t lda, int n, 
     return hipGetLastError();
 }
 
-static hipError_t solve_f64(const double* LU, int64_t lda, int n, const int* perm, const double* inv, double* x,
-                            double* tmp, hipStream_t s)
+static hipError_t solve_f64(const double* LU, int64_t lda, int n, const int* perm, double* inv, double* x, double* tmp,
+                            hipStream_t s)
 {
     const int nb = (n + kSB - 1) / kSB;
-    hipLaunchKernelGGL(permute_kernel, dim3((n + 255) / 256), dim3(256), 0, s, x, perm, n, tmp);
-    for (int b = 0; b < nb; ++b) {  // L z = P x: tmp -> x
-        const int k0 = b * kSB, bs = std::min(kSB, n - k0);
-        const int rows = n - k0 - bs;
-        hipLaunchKernelGGL((sweep_block_kernel<double, 1>), dim3(std::max(1, (rows + 63) / 64)), dim3(256), 0, s, LU,
-                           lda, n, inv, tmp, x, k0, bs);
-    }
-    for (int b = nb - 1; b >= 0; --b) {  // U y = z: x -> tmp
-        const int k0 = b * kSB, bs = std::min(kSB, n - k0);
-        hipLaunchKernelGGL((sweep_block_kernel<double, 0>), dim3(std::max(1, (k0 + 63) / 64)), dim3(256), 0, s, LU,
-                           lda, n, inv, x, tmp, k0, bs);
-    }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return launch_copy_vec(tmp, x, n, s);
+    auto* z = reinterpret_cast<unsigned long long*>(inv + (size_t)nb * 2 * kSB * kSB);
+    auto* y = reinterpret_cast<unsigned long long*>(x);
+    hipLaunchKernelGGL(permute_kernel, dim3((n + 255) / 256), dim3(256), 0, s, x, perm, n, tmp, z);
+    hipLaunchKernelGGL(sweep_chain_kernel<1>, dim3(nb), dim3(256), 0, s, LU, lda, n, inv, tmp, z, y);
+    hipLaunchKernelGGL(sweep_chain_kernel<0>, dim3(nb), dim3(256), 0, s, LU, lda, n, inv,
+                       reinterpret_cast<const double*>(z), y, static_cast<unsigned long long*>(nullptr));
+    return hipGetLastError();
 }
 
 static hipError_t solve_f32(const float* LU, int64_t lda, int n, const int* perm, float* inv, double* x, double* tmp,
                             hipStream_t s)
 {
     const int nb = (n + kWI - 1) / kWI;
-    hipLaunchKernelGGL(permute_kernel, dim3((n + 255) / 256), dim3(256), 0, s, x, perm, n, tmp);
+    hipLaunchKernelGGL(permute_kernel, dim3((n + 255) / 256), dim3(256), 0, s, x, perm, n, tmp,
+                       static_cast<unsigned long long*>(nullptr));
     for (int b = 0; b < nb; ++b) {  // L z = P x: tmp -> x
         const int bs = std::min(kWI, n - b * kWI), rows = n - b * kWI - bs;
         hipLaunchKernelGGL(wide_diag_kernel<1>, dim3((bs + 31) / 32), dim3(256), 0, s, n, inv, tmp, x, b);
@@ -2852,7 +2875,7 @@ hipError_t lu_solve_blocks(const void* LU, int elem_bytes, int64_t lda, int n, c
     const int* perm = static_cast<const int*>(aux);
     char* inv = const_cast<char*>(static_cast<const char*>(aux)) + perm_bytes(n);
     if (elem_bytes == 8)
-        return solve_f64(static_cast<const double*>(LU), lda, n, perm, reinterpret_cast<const double*>(inv), x, tmp, s);
+        return solve_f64(static_cast<const double*>(LU), lda, n, perm, reinterpret_cast<double*>(inv), x, tmp, s);
     return solve_f32(static_cast<const float*>(LU), lda, n, perm, reinterpret_cast<float*>(inv), x, tmp, s);
 }
 
