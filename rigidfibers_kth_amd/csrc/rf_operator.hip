@@ -280,7 +280,7 @@ __device__ __forceinline__ void quadrature_g(const double (&r0)[K][3], const dou
 // and far pairs in kernels of their own, 168 and 108 registers, take longer
 // together: 68 / 553 / 8015 us).  In a far class a lane takes two outer nodes,
 // so a source vector is loaded once for both: 7037 us, one node a lane 8167.
-// M = 5, LQ = 24, N = 250 / 1000 / 6000: 58 / 445 / 7150 us; a thread per
+// M = 5, LQ = 24, N = 250 / 1000 / 6000: 52 / 440 / 7100 us; a thread per
 // (target, point) with every pair through the moments: 59 / 796 / 27062 us.
 constexpr int kFarSplit = 2048;           // sources per workgroup at a time
 constexpr int kFarWave = kFarSplit / 4;   // and per wavefront
@@ -561,12 +561,17 @@ OperatorPlan plan_operator(int N, int M, int LQ, int analytic, int num_cus, int 
     p.LQ = LQ;
     p.analytic = analytic;
     if (analytic) {
-        // a workgroup per target and split: three workgroups fit a CU, and at
-        // least 16 sources per split (fewer leave lanes without elements)
+        // A workgroup per target and split; two fit a CU.  As many splits as
+        // one filling of the places takes with at least 16 sources each (fewer
+        // leave lanes without elements), and two beyond that where the
+        // wavefronts still have some 800 points each: N = 150 44 us (51 with
+        // five), N = 600 198 us (one 224, three 207), N = 390 with 12 points 78
+        // us (two 84).
         p.far = far;
         p.T = 1;
         p.threads = 256;
-        p.splits = std::max(1, std::min(3 * num_cus / N, N / 16));
+        p.splits = std::max(1, std::min(2 * num_cus / N, N / 16));
+        if (p.splits == 1 && (int64_t)N * LQ >= 6400) p.splits = 2;
         p.src_stride = 4 * (M + 1);
         for (int c = 0; c < Tables::kFarClasses && far; ++c) p.src_stride += 3 * far_inner_nodes(M, c);
     } else {
