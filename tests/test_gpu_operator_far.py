@@ -91,11 +91,13 @@ def _rows(i, pos, ori, M, noqi, x, panels=1, order=None):
     return y.ravel()
 
 
-@pytest.mark.parametrize("dmin,dmax", [(3.1, 4.3), (4.15, 5.6), (5.2, 8.1), (7.9, 30.0)])
-@pytest.mark.parametrize("M,noqi", [(1, 1), (2, 8), (3, 4), (4, 5), (5, 8), (5, 32), (6, 3), (7, 8), (8, 6), (8, 32)])
+# more than five terms: the closed forms' own error below 5.2 is 6e-9
+SHELLS = [(3.1, 4.3), (4.15, 5.6), (5.2, 8.1), (7.9, 30.0)]
+RULES = [(1, 1), (2, 8), (3, 4), (4, 5), (5, 8), (5, 32), (6, 3), (7, 8), (8, 6), (8, 32)]
+
+
+@pytest.mark.parametrize("M,noqi,dmin,dmax", [r + d for r in RULES for d in SHELLS if r[0] <= 5 or d[0] >= 5.0])
 def test_far_pairs_against_the_integrals(M, noqi, dmin, dmax):
-    if M > 5 and dmin < 5.0:
-        pytest.skip("more than five terms: the closed forms' own error there is 6e-9")
     N = 48
     pos, ori = _shell(N, dmin, dmax, 10 * M + noqi)
     x = np.random.default_rng(M).normal(size=3 * M * N)
